@@ -1,10 +1,11 @@
 // MFMA GEMM for prefill and batched decode: C[M, N] = A[M, K] x W[N, K]^T with fused epilogues.
 // Both operands are K-contiguous and accumulation is float32; bf16 uses v_mfma_f32_32x32x16_bf16, float32 uses
-// v_mfma_f32_32x32x2_f32 (true fp32).  Two kernels share the epilogues:
+// v_mfma_f32_32x32x2_f32 (true fp32).  Three kernels share the epilogues:
 //   gemm_kernel      any dtype and shape: global -> registers -> LDS (padded rows, so that the 16-byte fragment
 //                    reads of a 32x32 MFMA hit distinct banks), LDS double-buffered;
-//   gemm_dma_kernel  large bf16 problems: 256x256x64 tiles written straight into LDS by the memory pipeline
-//                    (buffer_load ... lds), rows xor-swizzled instead of padded, no staging registers.
+//   gemm_dma_kernel  large 16-bit problems: 256x256x64 tiles written straight into LDS by the memory pipeline
+//                    (buffer_load ... lds), rows xor-swizzled instead of padded, no staging registers;
+//   gemm_stream_kernel  16-bit problems of few rows: the same operand path, all rows in one tile, three or four stages.
 #include "mtj_common.h"
 #include <type_traits>
 
@@ -785,6 +786,162 @@ __global__ __launch_bounds__(512) void gemm_dma_kernel(const gemm_args a) {
   epilogue<EPI, WAVES_M, WAVES_N, WM, WN, true>(a, out, acc, smem, m0, n0);
 }
 
+// 16-bit operands, up to 256 rows (a short prompt, a few scored continuations) or K ranges of a few rows: bound by the
+// weights, which come from memory once, and by the operand path into LDS.  Row tiles of BM rows - normally ONE, so that no
+// weight is read twice -, BN = 128 columns per workgroup, 8 wavefronts, K step 64, S LDS stages written by the memory
+// pipeline as in gemm_dma_kernel (same row layout and swizzle): S - 1 k-tiles in flight without a register for them.
+//
+// Per k-tile there is one workgroup barrier.  Before it a wavefront waits for its own loads of the next k-tile and its own
+// fragment reads of this one, so behind it every operand of the next k-tile is in LDS and this k-tile's stage is free.
+// The fragments of a k-step are read while the MFMAs of the k-step before run, and the loads of k-tile kt+S are spread
+// over the MFMAs of two k-steps: issued in one burst (6 loads of 1 KiB per wavefront, which a CU accepts in ~800 cycles)
+// they held the MFMAs behind them up and cost 5 %.
+//
+// Measured at the 6B shapes (input projection N = 28672, K = 4096 / out projection N = 4096, K = 20480 in 8 ranges with
+// its reduce; weights of six layers in rotation) against the register-staged tiles this replaced: M = 64 40.3 / 37.1 us
+// (43.2 / 42.2 with 64 x 128 tiles), M = 128 51 / 45 (62 / 58), M = 256 70 / 57 (93 / 82, 128 x 128 tiles); M = 32 with K
+// ranges 34.1 (37.2).  The loads alone take 48 (M = 128) and 60 us (M = 256) for the input projection, the MFMAs and
+// fragment reads alone 23 and 43: what is left is the path into LDS (235 MB of weights plus 2 MB of activations per
+// workgroup, 12.6 TB/s), and neither more stages nor another walk over k changes it.
+template <typename T, int EPI, int BM, int S>
+__global__ __launch_bounds__(512) void gemm_stream_kernel(const gemm_args a) {
+  static_assert(sizeof(T) == 2, "16-bit operands");
+  constexpr int BN = 128, BK = 64, ROWB = BK * 2;
+  constexpr int WAVES_M = BM == 64 ? 2 : 4, WAVES_N = 8 / WAVES_M, WM = BM / 32 / WAVES_M, WN = BN / 32 / WAVES_N;
+  constexpr int OPB = BM * ROWB, STAGEB = OPB + BN * ROWB;
+  constexpr int NW = BN / 64, NL = NW + BM / 64;                     // loads per wavefront and k-tile: of W, in all
+  extern __shared__ __align__(16) unsigned char smem[];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+  const int fr = lane & 15, fq = lane >> 4;
+
+  // workgroups are dealt round-robin over the XCDs: with a multiple of 8 K ranges an XCD sees one or two of them and
+  // keeps that part of the activations in its L2 for all column tiles; without a split the row tiles of a column tile
+  // follow each other at a distance of 8, on one XCD, whose L2 then reads each weight once
+  const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
+  const int y = blockIdx.x % a.splits, t = blockIdx.x / a.splits;
+  const int first_n = t / (8 * tiles_m) * 8, tl = t - first_n * tiles_m;
+  const int gs = tiles_n - first_n < 8 ? tiles_n - first_n : 8;
+  const int tm = tl / gs, tn = first_n + tl - tm * gs;
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int rows_a = (a.M - m0 < BM) ? a.M - m0 : BM, rows_b = (a.N - n0 < BN) ? a.N - n0 : BN;
+  const T* tile_a = reinterpret_cast<const T*>(a.A) + (int64_t)m0 * a.lda;
+  const T* tile_b = reinterpret_cast<const T*>(a.W) + (int64_t)n0 * a.K;
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<T*>(tile_a), 0, (int)((((int64_t)rows_a - 1) * a.lda + a.K) * 2), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<T*>(tile_b), 0, (int)((((int64_t)rows_b - 1) * a.K + a.K) * 2), 0x00020000);
+
+  const int chunk = (lane & 7) ^ ((lane >> 4) & 3) ^ ((wave & 1) << 2);
+  const int row = wave * 8 + (lane >> 3);
+  const int voff_a = (int)((int64_t)row * a.lda * 2) + chunk * 16;
+  const int voff_b = (int)((int64_t)row * a.K * 2) + chunk * 16;
+
+  const int kt0 = (int)((int64_t)y * (a.K / BK) / a.splits);
+  const int KT = (int)((int64_t)(y + 1) * (a.K / BK) / a.splits) - kt0;
+  const int krot = (int)(((unsigned)tn * 5u) % (unsigned)KT);        // see gemm_kernel
+  // load n of k-tile kt into stage st: W rows first, then A rows, 64 rows each
+  auto issue_one = [&](int st, int kt, auto N_) {
+    constexpr int n = decltype(N_)::value;
+    const int kr = kt + krot;
+    const int koff = (kt0 + (kr >= KT ? kr - KT : kr)) * ROWB;
+    const int beyond = kt < KT ? 0 : 0x40000000;                     // see gemm_dma_kernel
+    unsigned char* d = smem + st * STAGEB + wave * 8 * ROWB;
+    if constexpr (n < NW)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr)(d + OPB + n * 64 * ROWB), 16, voff_b + beyond,
+                                               koff + (int)((int64_t)n * 64 * a.K * 2), 0, 2);   // nt: streamed once
+    else
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr)(d + (n - NW) * 64 * ROWB), 16, voff_a + beyond,
+                                               koff + (int)((int64_t)(n - NW) * 64 * a.lda * 2), 0, 0);
+  };
+
+  floatx4 acc[2 * WM][2 * WN];
+#pragma unroll
+  for (int i = 0; i < 2 * WM; ++i)
+#pragma unroll
+    for (int j = 0; j < 2 * WN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll
+  for (int st = 0; st < S - 1; ++st) for_stages<0, NL>([&](auto N_) { issue_one(st, st, N_); });
+
+  int xo[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) xo[ks] = ((4 * ks + fq) ^ ((fr >> 1) & 7)) * 16;
+  const int a_row = (wm * WM * 32 + fr) * ROWB, b_row = OPB + (wn * WN * 32 + fr) * ROWB;
+
+  typename mma<T>::frag fa[2][2 * WM], fb[2][2 * WN];
+  auto read = [&](int st, auto KS_) {
+    constexpr int ks = decltype(KS_)::value;
+    const unsigned char* sb = smem + st * STAGEB;
+#pragma unroll
+    for (int j = 0; j < 2 * WN; ++j) fb[ks][j] = mma<T>::load(reinterpret_cast<const T*>(sb + b_row + j * 16 * ROWB + xo[ks]));
+#pragma unroll
+    for (int i = 0; i < 2 * WM; ++i) fa[ks][i] = mma<T>::load(reinterpret_cast<const T*>(sb + a_row + i * 16 * ROWB + xo[ks]));
+  };
+  // the MFMAs of one k-step with the loads [N0, N1) of k-tile kt between them
+  auto multiply = [&](auto KS_, auto N0_, auto N1_, int st, int kt) {
+    constexpr int ks = decltype(KS_)::value, n0_ = decltype(N0_)::value, n1_ = decltype(N1_)::value;
+    for_stages<0, 2 * WM>([&](auto I_) {
+      constexpr int i = decltype(I_)::value;
+      if constexpr (n0_ + i < n1_) {
+        issue_one(st, kt, std::integral_constant<int, n0_ + i>{});
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int j = 0; j < 2 * WN; ++j) mma<T>::run16(acc[i][j], fb[ks][j], fa[ks][i]);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    for_stages<0, NL>([&](auto N_) {             // more loads than rows of blocks
+      constexpr int n = decltype(N_)::value;
+      if constexpr (n >= n0_ + 2 * WM && n < n1_) issue_one(st, kt, N_);
+    });
+  };
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  using IH = std::integral_constant<int, NL / 2>;
+  using IL = std::integral_constant<int, NL>;
+  // my loads of the next k-tile have landed, and so have my fragment reads of this one; behind the barrier both hold
+  // for the whole workgroup
+  auto next_tile = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(wait_vmcnt((S - 2) * NL) & wait_lgkmcnt(0));
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  next_tile();
+  for_stages<0, NL / 2>([&](auto N_) { issue_one(S - 1, S - 1, N_); });
+  read(0, I0{});
+  int st = 0;
+  for (int kt = 0; kt < KT; ++kt) {
+    const int nx = st + 1 == S ? 0 : st + 1;
+    read(st, I1{});
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(I0{}, IH{}, IL{}, st == 0 ? S - 1 : st - 1, kt + S - 1);   // second half of the loads of k-tile kt+S-1
+    next_tile();
+    read(nx, I0{});                            // beyond the last k-tile: zeros that nothing multiplies
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(I1{}, I0{}, IH{}, st, kt + S);    // first half of those of k-tile kt+S
+    st = nx;
+  }
+  __builtin_amdgcn_s_waitcnt(wait_vmcnt(0));   // the surplus loads land before the stages are reused
+  __syncthreads();
+
+  void* out = a.splits > 1 ? (void*)(reinterpret_cast<float*>(a.out) + y * a.split_stride) : a.out;
+  epilogue<EPI, WAVES_M, WAVES_N, WM, WN, true>(a, out, acc, smem, m0, n0);
+}
+
+template <typename T, int EPI, int BM, int S>
+int launch_stream(const gemm_args& a, hipStream_t s) {
+  constexpr size_t lds = (size_t)S * (BM + 128) * 128;
+  static_assert(lds >= 2 * BM * sizeof(int) + 8 * 32 * 36 * sizeof(float), "epilogue scratch does not fit");
+  static mtj_device_once once;
+  if (int rc = mtj_allow_lds(once, "mtj_gemm", &gemm_stream_kernel<T, EPI, BM, S>, lds)) return rc;
+  gemm_stream_kernel<T, EPI, BM, S><<<(unsigned)((a.M + BM - 1) / BM * ((a.N + 127) / 128) * a.splits), 512, lds, s>>>(a);
+  return mtj_check_launch("mtj_gemm");
+}
+
 template <typename T, int EPI>
 int launch_dma(const gemm_args& a, hipStream_t s) {
   constexpr size_t lds = 2 * 2 * 256 * 64 * 2;
@@ -810,8 +967,20 @@ int launch(const gemm_args& a, hipStream_t s) {
 
 template <typename T, int EPI, int BK>
 int dispatch_tile(const gemm_args& a, hipStream_t s) {
-  if (a.M <= 32) return launch<T, EPI, 1, 4, 1, 1, BK, 2>(a, s);    // 32 x 128: batched decode, weights stream once
-  if (a.M <= 64) return launch<T, EPI, 1, 4, 2, 1, BK, 2>(a, s);    // 64 x 128
+  if constexpr (sizeof(T) == 2) {
+    // 32 x 128 tiles, up to three workgroups per CU: batched decode without a split.  Against the stream kernel at M = 8:
+    // 38.4 / 39.2 us for the input projection, 66.7 / 67.9 for 50400 logits (two rounds of one workgroup per CU); with K
+    // ranges (the out projection) the stream kernel's deeper queue wins, 32.8 against 34.5 us.
+    if (a.M <= 32 && a.splits == 1) return launch<T, EPI, 1, 4, 1, 1, BK, 2>(a, s);
+    if (a.M <= 64) return launch_stream<T, EPI, 64, 4>(a, s);
+    // 129 .. 256 rows: one row tile while that fills more than half of the chip, else two (at d_model 2048, 112 column
+    // tiles, M = 256: 28 us in two row tiles, 38 in one; at d_model 4096 the second one would only read the weights again)
+    if (a.M > 128 && a.M <= 256 && (a.N + 127) / 128 * a.splits > 128) return launch_stream<T, EPI, 256, 3>(a, s);
+    if (a.M <= 256) return launch_stream<T, EPI, 128, 4>(a, s);
+  } else {
+    if (a.M <= 32) return launch<T, EPI, 1, 4, 1, 1, BK, 2>(a, s);  // 32 x 128: the weights stream once
+    if (a.M <= 64) return launch<T, EPI, 1, 4, 2, 1, BK, 2>(a, s);  // 64 x 128
+  }
   if constexpr (sizeof(T) == 2) {
     // e.g. M = 16384, N = 28672 or N = 4096 (a whole 6B layer at 8 x 2048 tokens): 7168 / 1024 tiles
     const int64_t big = (int64_t)((a.M + 255) / 256) * ((a.N + 255) / 256);
@@ -963,7 +1132,7 @@ __global__ __launch_bounds__(256) void xent_merge_kernel(const float* __restrict
 
 // column-tile width that dispatch_tile will use for this problem
 int xent_tile_n(int64_t M, int64_t N, int dtype) {
-  if (M > 64 && dtype != MTJ_F32 && ((M + 255) / 256) * ((N + 255) / 256) >= 200) return 256;
+  if (M > 256 && dtype != MTJ_F32 && ((M + 255) / 256) * ((N + 255) / 256) >= 200) return 256;
   return 128;
 }
 
@@ -973,7 +1142,7 @@ int pick_splits(int64_t M, int64_t N, int64_t K, int dtype) {
   const int bk = dtype == MTJ_F32 ? 32 : 64;
   const int64_t kt = K / bk;
   int splits = 1;
-  if (M <= 64) {          // one row of 32 x 128 or 64 x 128 tiles: up to 16 ranges
+  if (M <= (dtype == MTJ_F32 ? 64 : 256)) {   // one row of tiles, 128 columns each: up to 16 ranges
     const int64_t tiles = (N + 127) / 128;
     while (splits < 16 && tiles * splits * 2 <= 256 && kt % (splits * 2) == 0 && kt / (splits * 2) >= 4) splits *= 2;
   } else {

@@ -428,6 +428,37 @@ def test_direct_to_lds_kernel_with_few_k_tiles_and_ragged_columns(L, K, N, ldo):
     assert bool((out[:, N:] == 7.0).all())
 
 
+@pytest.mark.parametrize("M", [33, 64, 65, 128, 129, 256])
+@pytest.mark.parametrize("N,K", [(900, 64), (16500, 192), (1026, 448), (2048, 1024)])
+def test_few_rows_stream_kernel_tile_edges(L, M, N, K):
+    """gemm_stream_kernel at the edges of its row tiles (64, 128, two of 128, 256 once the columns fill half of the chip:
+    N = 16500 is 129 column tiles), with fewer k-tiles than LDS stages, a ragged last column tile, padded rows of A and K
+    ranges.  Operands are rounded already and the reference is float64, so only the float32 accumulation differs: its
+    error is below K * 2^-24 relative to the sum of magnitudes, here < 5e-6 of the result's norm as for the other tiles."""
+    a = abi()
+    g = torch.Generator().manual_seed(M + N + K)
+    lda = K + 64
+    A = torch.randn(M, lda, generator=g).to(torch.float16).to(DEV)
+    Wh = (torch.randn(K, N, generator=g) * 0.05).to(torch.float16).to(DEV)
+    bias = torch.randn(N, generator=g).to(DEV)
+    W = _packed(Wh)
+    ref = A[:, :K].double() @ Wh.double() + bias.double()
+    code = a.dtype_code(torch.float16)
+    out = torch.full((M + 1, N), 7.0, device=DEV)
+    a.check(L.mtj_gemm(a.ptr(A), lda, a.ptr(W), a.ptr(bias), M, N, K, code, a.EPI_STORE, a.ptr(out), N, 0, None, 1.0, S()))
+    torch.cuda.synchronize()
+    assert rel_err(out[:M], ref) < 5e-6
+    assert bool((out[M] == 7.0).all())                         # no row beyond M is written
+    if N % 4 == 0:
+        work = torch.empty(max(L.mtj_gemm_splitk_work_bytes(M, N, K, code), 16), dtype=torch.uint8, device=DEV)
+        x0 = torch.randn(M, N, generator=g).to(DEV)
+        x = x0.clone()
+        a.check(L.mtj_gemm_splitk(a.ptr(A), lda, a.ptr(W), a.ptr(bias), M, N, K, code, a.EPI_RESID, a.ptr(x), N, 0, a.ptr(work),
+                                  work.numel(), 1.0, S()))
+        torch.cuda.synchronize()
+        assert rel_err(x, x0.double() + ref) < 5e-6
+
+
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
 def test_inproj_gemv_decode_appends_to_ring(dt):
     from mesh_transformer.engine import Engine
