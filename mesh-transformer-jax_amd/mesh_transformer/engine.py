@@ -259,8 +259,11 @@ class Engine:
         M = B * Tp
         x, h, act = ses.x_pf[:M], ses.h_pf[:M], ses.act_pf[:M]
         check(L.mtj_embed(ptr(tokens_rect), M, ptr(w.we), ptr(w.be), w.V, d, w.dtype, ptr(x), s))
-        for i in w.layer_ids:
-            self.layer_prefill(ses, i, x, h, act, Tp, ses.pos0, key_limit)
+        # as in batched decode: the launch that completes a layer's residual rows also normalises them for the next layer
+        ids = w.layer_ids
+        for j, i in enumerate(ids):
+            nxt = (w.ln_s[ids[j + 1]], w.ln_o[ids[j + 1]]) if j + 1 < len(ids) else None
+            self.layer_prefill(ses, i, x, h, act, Tp, ses.pos0, key_limit, normed=j > 0, next_ln=nxt)
         return x
 
     def project(self, ses, x, out):
@@ -286,16 +289,23 @@ class Engine:
         check(L.mtj_gemm_xent(ptr(h), d, ptr(w.w_p_mm), ptr(w.b_p), M, V, d, w.mm_dtype, w.alpha_p, ptr(target),
                               ptr(loss), ptr(correct), ptr(ses.xent_work), ses.xent_work.numel() * 4, s))
 
-    def layer_prefill(self, ses, i, x, h, act, Tp, pos0, key_limit=None):
+    def layer_prefill(self, ses, i, x, h, act, Tp, pos0, key_limit=None, normed=False, next_ln=None):
+        """One layer on [B * Tp] rows; normed and next_ln as in layer_decode, with h in the place of ses.h."""
         L, w, s = _abi.lib(), self.w, _abi.stream_handle()
         M, d, F = x.shape[0], w.d, w.F
         A = w.act_dtype
-        check(L.mtj_layernorm(ptr(x), ptr(w.ln_s[i]), ptr(w.ln_o[i]), M, d, ptr(h), A, s))
+        if not normed:
+            check(L.mtj_layernorm(ptr(x), ptr(w.ln_s[i]), ptr(w.ln_o[i]), M, d, ptr(h), A, s))
         ip = self._inproj(ses, i, Tp, pos0, ses.q_pf, A, act, A, ses.vt)
         check(L.mtj_gemm(ptr(h), d, ptr(w.w_in_mm[i]), ptr(w.b1[i]), M, 3 * d + F, d, w.mm_dtype, EPI_INPROJ,
                          None, 0, 0, C.byref(ip), w.alpha_in[i], s))
         check(L.mtj_attn_prefill(ptr(ses.q_pf), ptr(ses.kc[i]), ptr(ses.vt), ptr(pos0), ses.B, self.H, Tp, ses.Tcap,
                                  self.dh, ses.ldvt, ptr(act), act.stride(0), A, ptr(key_limit), s))
+        if next_ln is not None:
+            check(L.mtj_gemm_splitk_ln(ptr(act), act.stride(0), ptr(w.w_out_mm[i]), ptr(w.b2[i]), M, d, d + F, w.mm_dtype,
+                                       ptr(x), d, ptr(ses.gemm_work), ses.gemm_work.numel(), ptr(next_ln[0]), ptr(next_ln[1]),
+                                       ptr(h), d, A, w.alpha_out[i], s))
+            return
         check(L.mtj_gemm_splitk(ptr(act), act.stride(0), ptr(w.w_out_mm[i]), ptr(w.b2[i]), M, d, d + F, w.mm_dtype, EPI_RESID,
                                 ptr(x), d, F32, ptr(ses.gemm_work), ses.gemm_work.numel(), w.alpha_out[i], s))
 
