@@ -145,12 +145,13 @@ int mtj_gemm(const void* A, int64_t lda, const void* W, const float* bias, int64
              int dtype, int epi, void* out, int64_t ldo, int out_dtype, const mtj_inproj* ip, float alpha,
              void* stream);
 
-/* mtj_gemm for problems with few output tiles (batched decode; the out projection of a short prompt): when the
- * output has too few tiles to occupy the
- * chip, K is cut into ranges that run as separate workgroups, each storing a float32 partial tile into `work`,
- * and a second kernel adds the partials in a fixed order (results do not depend on scheduling) and applies the
- * epilogue.  STORE and RESID only.  `work` holds mtj_gemm_splitk_work_bytes() bytes (0: no split is used and the
- * call is mtj_gemm); out and bias must then be 16-byte aligned and ldo a multiple of 4.
+/* mtj_gemm for problems whose output tiles do not fill the chip evenly (batched decode; the out projection of a
+ * prompt): when the output has too few tiles, K is cut into ranges that run as separate workgroups, each storing a
+ * float32 partial tile into `work`, and a second kernel adds the partials in a fixed order (results do not depend on
+ * scheduling) and applies the epilogue; when it has some more than whole rounds of tiles, the last rows are such a
+ * problem of their own.  STORE and RESID only.  `work` holds mtj_gemm_splitk_work_bytes() bytes (0: no split is used
+ * and the call is mtj_gemm); out and bias must be 16-byte aligned and ldo a multiple of 4 where a split is needed for
+ * occupancy (up to 256 rows, up to 64 tiles of 256 x 256), and keep larger problems from being split otherwise.
  * Call sites: the out/fc_out projection of decode_once (layers.py:316-344) at batch > 1. */
 int64_t mtj_gemm_splitk_work_bytes(int64_t M, int64_t N, int64_t K, int dtype);
 int mtj_gemm_splitk(const void* A, int64_t lda, const void* W, const float* bias, int64_t M, int64_t N, int64_t K,

@@ -965,6 +965,11 @@ int launch(const gemm_args& a, hipStream_t s) {
   return mtj_check_launch("mtj_gemm");
 }
 
+// 256 x 256 tiles of gemm_dma_kernel, one workgroup per CU, from this many of them on: N = 4096, K = 20480 in one K range,
+// 144 tiles 486 us (602 with 128 x 128 tiles), 192 tiles 458 (650); 96 tiles 455 against 384 for two ranges of 128 x 128.
+constexpr int64_t DMA_MIN_TILES = 144;
+int64_t dma_tiles(int64_t M, int64_t N) { return ((M + 255) / 256) * ((N + 255) / 256); }
+
 template <typename T, int EPI, int BK>
 int dispatch_tile(const gemm_args& a, hipStream_t s) {
   if constexpr (sizeof(T) == 2) {
@@ -983,8 +988,7 @@ int dispatch_tile(const gemm_args& a, hipStream_t s) {
   }
   if constexpr (sizeof(T) == 2) {
     // e.g. M = 16384, N = 28672 or N = 4096 (a whole 6B layer at 8 x 2048 tokens): 7168 / 1024 tiles
-    const int64_t big = (int64_t)((a.M + 255) / 256) * ((a.N + 255) / 256);
-    if (big * a.splits >= 200) return launch_dma<T, EPI>(a, s);                         // 256 x 256, 8 wavefronts of 128 x 64
+    if (dma_tiles(a.M, a.N) * a.splits >= DMA_MIN_TILES) return launch_dma<T, EPI>(a, s);   // 256 x 256, 8 wavefronts of 128 x 64
   }
   return launch<T, EPI, 2, 2, 2, 2, BK, 2>(a, s);                   // 128 x 128
 }
@@ -1154,31 +1158,72 @@ __global__ __launch_bounds__(XM_ROWS * XM_LANES) void xent_merge_kernel(const fl
 
 // column-tile width that dispatch_tile will use for this problem
 int xent_tile_n(int64_t M, int64_t N, int dtype) {
-  if (M > 256 && dtype != MTJ_F32 && ((M + 255) / 256) * ((N + 255) / 256) >= 200) return 256;
+  if (M > 256 && dtype != MTJ_F32 && dma_tiles(M, N) >= DMA_MIN_TILES) return 256;
   return 128;
 }
 
-// how many K ranges a skinny problem is cut into so that its few output tiles still fill the chip
-int pick_splits(int64_t M, int64_t N, int64_t K, int dtype) {
-  if (N % 4) return 1;
+// Time of `tiles` 256 x 256 tiles in s K ranges each, in tenths of the time of one k-tile (1.4 us): rounds of 256
+// workgroups, each walking kt / s k-tiles, and the partials, 0.17 us per tile and range written and read back (N = 4096,
+// K = 20480, 256 tiles: 545 / 575 / 646 / 815 us in 1 / 2 / 4 / 8 ranges).
+int64_t dma_cost(int64_t tiles, int64_t kt, int64_t s) {
+  return (tiles * s + 255) / 256 * ((kt + s - 1) / s) * 10 + (s > 1 ? tiles * s * 6 / 5 : 0);
+}
+
+// How a problem is cut so that its output tiles fill the chip evenly: rows [0, front) in one K range with the epilogue of
+// the product itself, the rows behind them in `splits` K ranges with a reduce.
+struct cut_t { int64_t front; int splits; };
+
+cut_t pick_cut(int64_t M, int64_t N, int64_t K, int dtype) {
+  if (N % 4) return {0, 1};
   const int bk = dtype == MTJ_F32 ? 32 : 64;
   const int64_t kt = K / bk;
   int splits = 1;
   if (M <= (dtype == MTJ_F32 ? 64 : 256)) {   // one row of tiles, 128 columns each: up to 16 ranges
     const int64_t tiles = (N + 127) / 128;
     while (splits < 16 && tiles * splits * 2 <= 256 && kt % (splits * 2) == 0 && kt / (splits * 2) >= 4) splits *= 2;
-  } else {
-    if (dtype != MTJ_F32) {   // 256 x 256 tiles of the direct-to-LDS kernel, one workgroup per CU (a short prompt's out projection)
-      const int64_t big = ((M + 255) / 256) * ((N + 255) / 256);
-      while (splits < 16 && big * splits * 2 <= 256 && kt % (splits * 2) == 0 && kt / (splits * 2) >= 16) splits *= 2;
-      if (big * splits >= 200) return splits;
-      splits = 1;
-    }
-    // 128 x 128 tiles, two workgroups per CU: up to 4 ranges
-    const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
-    while (splits < 4 && tiles * splits * 2 <= 512 && kt % (splits * 2) == 0 && kt / (splits * 2) >= 16) splits *= 2;
+    return {0, splits};
   }
-  return splits;
+  if (dtype != MTJ_F32) {
+    // 256 x 256 tiles of the direct-to-LDS kernel, one workgroup per CU.  A short prompt's out projection (N = 4096,
+    // 16 column tiles) has fewer tiles than CUs: the number of ranges that costs least.  With powers of two only, what did
+    // not come to 200 tiles ran on 128 x 128 ones: 768 rows 207 -> 149 us, 1025 338 -> 198, 1536 384 -> 279, 2304
+    // 602 -> 388, 2875 650 -> 461; 257 .. 512, 769 .. 1024 and 1537 .. 2048 rows keep 8, 4 and 2 ranges.
+    const int64_t tiles = dma_tiles(M, N);
+    if (tiles <= 256) {
+      for (int s = 2; s <= 16 && kt / s >= 16; ++s)
+        if (dma_cost(tiles, kt, s) < dma_cost(tiles, kt, splits)) splits = s;
+      if (tiles * splits >= DMA_MIN_TILES) return {0, splits};
+      splits = 1;
+    } else {
+      // Beyond that the last round would leave most CUs idle for a whole tile's time: whole rounds first, then the rest as
+      // a problem of its own, if that costs less (its second launch and the separate LayerNorm of the front rows: 5 us).
+      // With the reduce and the following LayerNorm: 4097 rows 1034 -> 590 us, 4900 1024 -> 719, 5632 1029 -> 841, 6500
+      // 1024 -> 947 (7000 stays at 1021), 8200 1573 -> 1125, 9000 1552 -> 1255.
+      // Only 2, 3, 4, 8 or 16 ranges: 5 would save another 15 us at 48 tiles, and need more workspace than a short prompt.
+      const int64_t cols = (N + 255) / 256, rounds = tiles / 256;
+      const int64_t front = rounds * 256 / cols * 256;
+      if (front > 0 && M - front > 0) {
+        const int64_t rest = dma_tiles(M - front, N), front_cost = (front / 256 * cols + 255) / 256 * kt * 10;
+        int64_t best = dma_cost(tiles, kt, 1) - front_cost - 36;
+        if (M - front <= 256) {              // these rows go to gemm_stream_kernel: its own ranges, a tile of it costs no more
+          const int s = pick_cut(M - front, N, K, dtype).splits;
+          if (dma_cost(2 * rest, kt, s) < best) splits = s;
+        } else {
+          for (int s : {2, 3, 4, 8, 16})
+            if (kt / s >= 16 && rest * s >= DMA_MIN_TILES && dma_cost(rest, kt, s) < best) {
+              best = dma_cost(rest, kt, s);
+              splits = s;
+            }
+        }
+        if (splits > 1) return {front, splits};
+      }
+      return {0, 1};
+    }
+  }
+  // 128 x 128 tiles, two workgroups per CU: up to 4 ranges
+  const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
+  while (splits < 4 && tiles * splits * 2 <= 512 && kt % (splits * 2) == 0 && kt / (splits * 2) >= 16) splits *= 2;
+  return {0, splits};
 }
 
 int check_common(const void* A, int64_t lda, const void* W, int64_t M, int64_t N, int64_t K, int dtype, const char* who) {
@@ -1204,6 +1249,9 @@ int dispatch_dtype(const gemm_args& a, int dtype, int epi, hipStream_t s) {
   if (dtype == MTJ_BF16) return dispatch<bf16_t, 64>(a, epi, s);
   if (dtype == MTJ_F16) return dispatch<f16_t, 64>(a, epi, s);
   return dispatch<float, 32>(a, epi, s);
+}
+const void* rows_from(const void* base, int64_t elems, int dtype) {
+  return reinterpret_cast<const unsigned char*>(base) + elems * mtj_elem_size(dtype);
 }
 }  // namespace
 
@@ -1239,8 +1287,8 @@ extern "C" int mtj_gemm(const void* A, int64_t lda, const void* W, const float* 
 
 extern "C" int64_t mtj_gemm_splitk_work_bytes(int64_t M, int64_t N, int64_t K, int dtype) {
   if (M <= 0 || N <= 0 || K <= 0 || !mtj_is_dtype(dtype)) return 0;
-  const int splits = pick_splits(M, N, K, dtype);
-  return splits > 1 ? (int64_t)splits * M * N * (int64_t)sizeof(float) : 0;
+  const cut_t cut = pick_cut(M, N, K, dtype);
+  return cut.splits > 1 ? (int64_t)cut.splits * (M - cut.front) * N * (int64_t)sizeof(float) : 0;
 }
 
 extern "C" int mtj_gemm_splitk(const void* A, int64_t lda, const void* W, const float* bias, int64_t M, int64_t N,
@@ -1248,13 +1296,25 @@ extern "C" int mtj_gemm_splitk(const void* A, int64_t lda, const void* W, const 
                                int64_t work_bytes, float alpha, void* stream) {
   MTJ_REQUIRE(epi == MTJ_EPI_STORE || epi == MTJ_EPI_RESID, MTJ_EINVAL, "mtj_gemm_splitk: epilogue %d", epi);
   if (int rc = check_common(A, lda, W, M, N, K, dtype, "mtj_gemm_splitk")) return rc;
-  const int splits = pick_splits(M, N, K, dtype);
-  if (splits == 1) return mtj_gemm(A, lda, W, bias, M, N, K, dtype, epi, out, ldo, out_dtype, nullptr, alpha, stream);
-  MTJ_REQUIRE(out && ldo >= N && ldo % 4 == 0 && mtj_aligned16(out) && (!bias || mtj_aligned16(bias)), MTJ_EINVAL,
+  const cut_t cut = pick_cut(M, N, K, dtype);
+  const int splits = cut.splits;
+  // the reduce moves four columns at a time: rows that do not allow that are taken in one range where a problem of this
+  // size need not be split (more than 64 tiles or an odd number of k-tiles), and refused where it always is
+  const bool rows_ok = out && ldo >= N && ldo % 4 == 0 && mtj_aligned16(out) && (!bias || mtj_aligned16(bias));
+  const bool one_range = !rows_ok && M > 256 && dtype != MTJ_F32 && (dma_tiles(M, N) > 64 || K / 64 % 2);
+  if (splits == 1 || one_range)
+    return mtj_gemm(A, lda, W, bias, M, N, K, dtype, epi, out, ldo, out_dtype, nullptr, alpha, stream);
+  MTJ_REQUIRE(rows_ok, MTJ_EINVAL,
               "mtj_gemm_splitk: out needs ldo >= N, a multiple of 4, and 16-byte alignment (bias too)");
   MTJ_REQUIRE(epi == MTJ_EPI_RESID || mtj_is_dtype(out_dtype), MTJ_EDTYPE, "mtj_gemm_splitk: out_dtype %d", out_dtype);
-  MTJ_REQUIRE(work && mtj_aligned16(work) && work_bytes >= (int64_t)splits * M * N * (int64_t)sizeof(float), MTJ_EINVAL,
-              "mtj_gemm_splitk: work must hold mtj_gemm_splitk_work_bytes() bytes");
+  MTJ_REQUIRE(work && mtj_aligned16(work) && work_bytes >= (int64_t)splits * (M - cut.front) * N * (int64_t)sizeof(float),
+              MTJ_EINVAL, "mtj_gemm_splitk: work must hold mtj_gemm_splitk_work_bytes() bytes");
+  if (cut.front) {
+    if (int rc = mtj_gemm(A, lda, W, bias, cut.front, N, K, dtype, epi, out, ldo, out_dtype, nullptr, alpha, stream)) return rc;
+    A = rows_from(A, cut.front * lda, dtype);
+    out = const_cast<void*>(rows_from(out, cut.front * ldo, epi == MTJ_EPI_RESID ? MTJ_F32 : out_dtype));
+    M -= cut.front;
+  }
   gemm_args a{};
   a.A = A; a.lda = lda; a.W = W; a.bias = nullptr; a.M = (int)M; a.N = (int)N; a.K = (int)K;
   a.out = work; a.ldo = N; a.out_dtype = MTJ_F32; a.alpha = alpha;
@@ -1281,15 +1341,25 @@ extern "C" int mtj_gemm_splitk_ln(const void* A, int64_t lda, const void* W, con
                   (!bias || mtj_aligned16(bias)),
               MTJ_EINVAL, "mtj_gemm_splitk_ln: N a multiple of 4 and <= %d, rows of x and h 16-byte aligned", 4 * RLN_Q * 1024);
   if (int rc = check_common(A, lda, W, M, N, K, dtype, "mtj_gemm_splitk_ln")) return rc;
-  const int splits = pick_splits(M, N, K, dtype);
+  const cut_t cut = pick_cut(M, N, K, dtype);
+  const int splits = cut.splits;
   hipStream_t s = (hipStream_t)stream;
   if (splits == 1) {      // no partials to reduce: the product with its own residual epilogue, then the plain LayerNorm
     MTJ_REQUIRE(ldx == N && ldh == N, MTJ_EINVAL, "mtj_gemm_splitk_ln: without a split, x and h must be dense");
     if (int rc = mtj_gemm(A, lda, W, bias, M, N, K, dtype, MTJ_EPI_RESID, x, ldx, MTJ_F32, nullptr, alpha, stream)) return rc;
     return mtj_layernorm(x, ln_scale, ln_offset, M, N, h, h_dtype, stream);
   }
-  MTJ_REQUIRE(work && mtj_aligned16(work) && work_bytes >= (int64_t)splits * M * N * (int64_t)sizeof(float), MTJ_EINVAL,
-              "mtj_gemm_splitk_ln: work must hold mtj_gemm_splitk_work_bytes() bytes");
+  MTJ_REQUIRE(work && mtj_aligned16(work) && work_bytes >= (int64_t)splits * (M - cut.front) * N * (int64_t)sizeof(float),
+              MTJ_EINVAL, "mtj_gemm_splitk_ln: work must hold mtj_gemm_splitk_work_bytes() bytes");
+  if (cut.front) {
+    MTJ_REQUIRE(ldx == N && ldh == N, MTJ_EINVAL, "mtj_gemm_splitk_ln: rows without a split must be dense in x and h");
+    if (int rc = mtj_gemm(A, lda, W, bias, cut.front, N, K, dtype, MTJ_EPI_RESID, x, ldx, MTJ_F32, nullptr, alpha, stream)) return rc;
+    if (int rc = mtj_layernorm(x, ln_scale, ln_offset, cut.front, N, h, h_dtype, stream)) return rc;
+    A = rows_from(A, cut.front * lda, dtype);
+    x += cut.front * ldx;
+    h = const_cast<void*>(rows_from(h, cut.front * ldh, h_dtype));
+    M -= cut.front;
+  }
   gemm_args a{};
   a.A = A; a.lda = lda; a.W = W; a.bias = nullptr; a.M = (int)M; a.N = (int)N; a.K = (int)K;
   a.out = work; a.ldo = N; a.out_dtype = MTJ_F32; a.alpha = alpha;

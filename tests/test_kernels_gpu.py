@@ -222,6 +222,47 @@ def test_gemm_splitk_matches_reference_and_is_deterministic(L, dt, M, N, K):
                                       a.ptr(work), nb - 4, 1.0, S()))
 
 
+@pytest.mark.parametrize("M,N,K,splits,front", [
+    (513, 4096, 5120, 4, 0), (700, 4096, 20480, 5, 0), (1025, 4096, 4160, 3, 0),     # 48 / 48 / 80 tiles, ragged k ranges
+    (2500, 4096, 20480, 3, 0), (3100, 4096, 1024, 1, 0),                             # 160 / 208 tiles
+    (4097, 4096, 5120, 8, 4096), (4900, 4096, 5184, 3, 4096), (4400, 3840, 5120, 8, 4352)])    # a round, then the rest
+def test_out_projection_is_cut_into_even_rounds(L, M, N, K, splits, front):
+    """Row counts whose 256 x 256 tiles do not fill the chip a whole number of times, with any number of K ranges and with
+    the rows of the last round cut off: x, the rows behind it, and h of the launch with the LayerNorm.  Operands are
+    rounded already, so only the float32 accumulation differs from float64 (bounds as for the other products)."""
+    a = abi()
+    g = torch.Generator().manual_seed(M + N + K)
+    A = torch.randn(M, K + 64, generator=g).to(torch.float16).to(DEV)
+    Wh = (torch.randn(K, N, generator=g) * 0.05).to(torch.float16).to(DEV)
+    bias = torch.randn(N, generator=g).to(DEV)
+    sc = (1 + 0.1 * torch.randn(N, generator=g)).to(DEV)
+    of = (0.1 * torch.randn(N, generator=g)).to(DEV)
+    W = _packed(Wh)
+    x0 = torch.randn(M, N, generator=g).to(DEV)
+    ref = x0.double() + A[:, :K].double() @ Wh.double() + bias.double()
+    nb = L.mtj_gemm_splitk_work_bytes(M, N, K, a.F16)
+    assert nb == (splits * (M - front) * N * 4 if splits > 1 else 0)
+    work = torch.empty(max(nb, 16) + 64, dtype=torch.uint8, device=DEV)
+    work[nb:] = 7
+    for ld in (N, N + 3):                                      # rows that the reduce cannot take in quads: one K range
+        if ld != N and (M <= 1024):
+            continue                                           # (refused there)
+        x = torch.full((M + 1, ld), 7.0, device=DEV)
+        x[:M, :N] = x0
+        a.check(L.mtj_gemm_splitk(a.ptr(A), K + 64, a.ptr(W), a.ptr(bias), M, N, K, a.F16, a.EPI_RESID, a.ptr(x), ld, 0,
+                                  a.ptr(work), nb, 1.0, S()))
+        torch.cuda.synchronize()
+        assert rel_err(x[:M, :N], ref) < 5e-6
+        assert bool((x[M] == 7.0).all()) and bool((x[:, N:] == 7.0).all()) and bool((work[nb:] == 7).all())
+    x, h = x0.clone(), torch.zeros(M + 1, N, dtype=torch.float16, device=DEV)
+    a.check(L.mtj_gemm_splitk_ln(a.ptr(A), K + 64, a.ptr(W), a.ptr(bias), M, N, K, a.F16, a.ptr(x), N, a.ptr(work), nb,
+                                 a.ptr(sc), a.ptr(of), a.ptr(h), N, a.F16, 1.0, S()))
+    torch.cuda.synchronize()
+    assert rel_err(x, ref) < 5e-6
+    assert rel_err(h[:M], torch.nn.functional.layer_norm(ref, (N,), sc.double(), of.double(), 1e-5)) < 5e-4
+    assert bool((h[M] == 0).all()) and bool((work[nb:] == 7).all())
+
+
 @pytest.mark.parametrize("dt", DTS)
 @pytest.mark.parametrize("M,N,K", [(32, 4096, 20480), (5, 512, 2560), (3, 64, 64), (8, 1024, 4096)])
 def test_gemm_splitk_with_the_following_layernorm(L, dt, M, N, K):
