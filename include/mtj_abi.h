@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define MTJ_ABI_VERSION 4
+#define MTJ_ABI_VERSION 5
 
 enum { MTJ_F32 = 0, MTJ_BF16 = 1, MTJ_F16 = 2 };
 
@@ -81,6 +81,9 @@ typedef struct {
   void* act;                            /* [M, ld_act]: gelu(fc_in) goes to columns [d, d+F)           */
   int64_t ld_act;
   int32_t act_dtype;                    /* MTJ_F32 or MTJ_BF16                                         */
+  const int32_t* rows;                  /* optional [M]: row m of the GEMM is row rows[m] of the [B, Tp]
+                                           rectangle (prompts of unequal length without their padding; each
+                                           entry below B * Tp).  mtj_gemm only: others refuse it          */
 } mtj_inproj;
 
 /*
@@ -219,6 +222,13 @@ int mtj_gemv_attn(const float* x, const void* W, const float* bias, int64_t N, i
 int mtj_attn_prefill(const void* q, const void* k_cache, const void* v_t, const int32_t* pos0, int64_t B,
                      int64_t H, int64_t Tp, int64_t Tcap, int64_t dh, int64_t ldvt, void* out, int64_t ld_out,
                      int dtype, const int32_t* key_limit, void* stream);
+
+/* mtj_attn_prefill whose `out` holds the rows of real tokens only, one sequence behind the other: row
+ * b * Tp + t - skipped[b], skipped [B] = the padding rows of sequences 0 .. b (sum of -pos0).  Padding rows are not
+ * written. */
+int mtj_attn_prefill_packed(const void* q, const void* k_cache, const void* v_t, const int32_t* pos0, int64_t B,
+                            int64_t H, int64_t Tp, int64_t Tcap, int64_t dh, int64_t ldvt, void* out, int64_t ld_out,
+                            int dtype, const int32_t* key_limit, const int32_t* skipped, void* stream);
 
 /* One-token attention over the K/V window (decode_once, layers.py:316-344): for sequence b the valid
  * slots are [0, min(pos[b]+1, Tcap)).  q float32 [B,H,dh]; caches in `dtype`; out [B, ld_out] in out_dtype

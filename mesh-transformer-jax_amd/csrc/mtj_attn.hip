@@ -119,12 +119,22 @@ template <> struct mma<float> {
 // double-buffered (the loads of tile kt+1 are in flight while tile kt is multiplied).  The softmax runs in
 // the exp2 domain with the hardware exponential; the accumulator is rescaled only when some lane's running
 // maximum actually moved.
+// Output rows of sequence b: query t goes to row base + t, t from `first` on.  With `skipped` (padding rows of sequences
+// 0 .. b) the rows of padding are left out, otherwise they are there and get zeros.
+struct out_rows {
+  int64_t base;
+  int first;
+  __device__ __forceinline__ out_rows(int b, int Tp, int p0, const int32_t* skipped)
+      : base((int64_t)b * Tp - (skipped ? skipped[b] : 0)), first(skipped ? -p0 : 0) {}
+};
+
 template <typename T, int DH, int NW, int BKV>
 __global__ __launch_bounds__(NW * 64) void attn_prefill_kernel(const T* __restrict__ q, const T* __restrict__ kc,
                                                                const T* __restrict__ vt, const int32_t* __restrict__ pos0,
                                                                int H, int Tp, int Tcap, int64_t ldvt, T* __restrict__ out,
                                                                int64_t ld_out, int nseq, int nqblk,
-                                                               const int32_t* __restrict__ key_limit) {
+                                                               const int32_t* __restrict__ key_limit,
+                                                               const int32_t* __restrict__ skipped) {
   constexpr int NT = NW * 64;
   constexpr int BQ = NW * 32;
   constexpr int EPC = mma<T>::EPC;
@@ -371,9 +381,10 @@ __global__ __launch_bounds__(NW * 64) void attn_prefill_kernel(const T* __restri
   }
 
   // ---- write O: register v of block i is head-dim i*32 + 8*(v/4) + 4*fg + v%4 of query t
-  if (t < Tp) {
+  const out_rows rows(b, Tp, p0, skipped);
+  if (t >= rows.first && t < Tp) {
     const float inv = (qpos >= 0 && lrun > 0.f) ? 1.0f / lrun : 0.f;
-    T* op = out + ((int64_t)b * Tp + t) * ld_out + (int64_t)h * DH;
+    T* op = out + (rows.base + t) * ld_out + (int64_t)h * DH;
 #pragma unroll
     for (int i = 0; i < NBLK; ++i)
 #pragma unroll
@@ -436,7 +447,8 @@ __global__ __launch_bounds__(512) void attn_prefill_pair_kernel(const T* __restr
                                                                 const T* __restrict__ vt, const int32_t* __restrict__ pos0,
                                                                 int H, int Tp, int Tcap, int64_t ldvt, T* __restrict__ out,
                                                                 int64_t ld_out, int nseq, int nqblk,
-                                                                const int32_t* __restrict__ key_limit) {
+                                                                const int32_t* __restrict__ key_limit,
+                                                                const int32_t* __restrict__ skipped) {
   static_assert(sizeof(T) == 2, "16-bit types");
   constexpr int DH = 256, BKV = 32, BQ = 128, KS = DH / 16, NBLK = DH / 32;
   extern __shared__ __align__(16) unsigned char smem[];
@@ -688,9 +700,10 @@ __global__ __launch_bounds__(512) void attn_prefill_pair_kernel(const T* __restr
   __builtin_amdgcn_s_waitcnt(wait_vmcnt(0));                // the surplus loads land before the LDS is given away
 
   // ---- write O: register v of block n is head-dim n*32 + 8*(v/4) + 4*fg + v%4 of query t
-  if (t < Tp) {
+  const out_rows rows(b, Tp, p0, skipped);
+  if (t >= rows.first && t < Tp) {
     const float inv = (qpos >= 0 && lrun > 0.f) ? 1.0f / lrun : 0.f;
-    T* op = out + ((int64_t)b * Tp + t) * ld_out + (int64_t)h * DH;
+    T* op = out + (rows.base + t) * ld_out + (int64_t)h * DH;
 #pragma unroll
     for (int n = 0; n < NBLK; ++n)
 #pragma unroll
@@ -769,7 +782,8 @@ __global__ __launch_bounds__(256) void attn_prefill_q64_kernel(const T* __restri
                                                                const T* __restrict__ vt, const int32_t* __restrict__ pos0,
                                                                int H, int Tp, int Tcap, int64_t ldvt, T* __restrict__ out,
                                                                int64_t ld_out, int nseq, int nqblk,
-                                                               const int32_t* __restrict__ key_limit) {
+                                                               const int32_t* __restrict__ key_limit,
+                                                               const int32_t* __restrict__ skipped) {
   static_assert(sizeof(T) == 2, "16-bit types");
   constexpr int DH = 256, BKV = 32, BQ = 256, KS = DH / 16, NBLK = DH / 32;
   extern __shared__ __align__(16) unsigned char smem[];
@@ -1065,11 +1079,12 @@ __global__ __launch_bounds__(256) void attn_prefill_q64_kernel(const T* __restri
     });
   });
   // (a wavefront's LDS operations stay in order: no barrier between its own writes and reads)
+  const out_rows rows(b, Tp, p0, skipped);
 #pragma unroll 4
   for (int it = 0; it < 32; ++it) {
     const int row = 2 * it + fg, t = qt0 + wave * 64 + row;
     const uint32x4 v = *reinterpret_cast<const uint32x4*>(ob + row * 512 + ((fr ^ (row & 31)) << 4));
-    if (t < Tp) *reinterpret_cast<uint32x4*>(out + ((int64_t)b * Tp + t) * ld_out + (int64_t)h * DH + fr * 8) = v;
+    if (t >= rows.first && t < Tp) *reinterpret_cast<uint32x4*>(out + (rows.base + t) * ld_out + (int64_t)h * DH + fr * 8) = v;
   }
   __builtin_amdgcn_s_barrier();                             // the next part's tiles go where these rows were
   }
@@ -1238,9 +1253,11 @@ int decode_splits(int64_t B, int64_t H, int64_t Tcap) {
 
 }  // namespace
 
-extern "C" int mtj_attn_prefill(const void* q, const void* k_cache, const void* v_t, const int32_t* pos0, int64_t B,
-                                int64_t H, int64_t Tp, int64_t Tcap, int64_t dh, int64_t ldvt, void* out,
-                                int64_t ld_out, int dtype, const int32_t* key_limit, void* stream) {
+namespace {
+
+int attn_prefill_impl(const void* q, const void* k_cache, const void* v_t, const int32_t* pos0, int64_t B, int64_t H,
+                      int64_t Tp, int64_t Tcap, int64_t dh, int64_t ldvt, void* out, int64_t ld_out, int dtype,
+                      const int32_t* key_limit, const int32_t* skipped, void* stream) {
   MTJ_REQUIRE(q && k_cache && v_t && pos0 && out, MTJ_EINVAL, "mtj_attn_prefill: null pointer");
   MTJ_REQUIRE(B > 0 && H > 0 && Tp > 0 && Tp <= Tcap && ld_out >= H * dh && B < 65536 && H < 65536, MTJ_EINVAL,
               "mtj_attn_prefill: bad shape B=%lld H=%lld Tp=%lld Tcap=%lld", (long long)B, (long long)H,
@@ -1262,7 +1279,7 @@ extern "C" int mtj_attn_prefill(const void* q, const void* k_cache, const void* 
     MTJ_REQUIRE(nqblk * H * B < (1ll << 31), MTJ_ELIMIT, "mtj_attn_prefill: too many workgroups");                    \
     attn_prefill_kernel<T, DH, NW, BKV><<<(unsigned)(nqblk * H * B), NW * 64, lds, s>>>(                              \
         (const T*)q, (const T*)k_cache, (const T*)v_t, pos0, (int)H, (int)Tp, (int)Tcap, ldvt, (T*)out, ld_out,      \
-        (int)B, (int)nqblk, key_limit);                                                                                       \
+        (int)B, (int)nqblk, key_limit, skipped);                                                                              \
   } while (0)
 #define MTJ_PREFILL_PAIR(T)                                                                                          \
   do {                                                                                                               \
@@ -1274,7 +1291,7 @@ extern "C" int mtj_attn_prefill(const void* q, const void* k_cache, const void* 
     MTJ_REQUIRE(Tcap * 512 < (1ll << 31) && 512 * ldvt < (1ll << 31), MTJ_ELIMIT, "mtj_attn_prefill: window too long"); \
     attn_prefill_pair_kernel<T><<<(unsigned)(nqblk * H * B), 512, PP_LDS_BYTES, s>>>(                                 \
         (const T*)q, (const T*)k_cache, (const T*)v_t, pos0, (int)H, (int)Tp, (int)Tcap, ldvt, (T*)out, ld_out,      \
-        (int)B, (int)nqblk, key_limit);                                                                              \
+        (int)B, (int)nqblk, key_limit, skipped);                                                                     \
   } while (0)
 #define MTJ_PREFILL_Q64(T)                                                                                           \
   do {                                                                                                               \
@@ -1286,7 +1303,7 @@ extern "C" int mtj_attn_prefill(const void* q, const void* k_cache, const void* 
     MTJ_REQUIRE(Tcap * 512 < (1ll << 31) && 512 * ldvt < (1ll << 31), MTJ_ELIMIT, "mtj_attn_prefill: window too long"); \
     attn_prefill_q64_kernel<T><<<(unsigned)((nqblk + 1) / 2 * H * B), 256, Q64_LDS_BYTES, s>>>(                                 \
         (const T*)q, (const T*)k_cache, (const T*)v_t, pos0, (int)H, (int)Tp, (int)Tcap, ldvt, (T*)out, ld_out,      \
-        (int)B, (int)nqblk, key_limit);                                                                              \
+        (int)B, (int)nqblk, key_limit, skipped);                                                                     \
   } while (0)
   // 256-query blocks, two per workgroup, when that still makes two workgroups per CU (measured on 16 heads x 2048 tokens:
   // 472 us against 529 for 8 sequences, 796 against 1069 for 16, but 225 against 208 for 4); shorter problems keep the
@@ -1305,6 +1322,22 @@ extern "C" int mtj_attn_prefill(const void* q, const void* k_cache, const void* 
 #undef MTJ_PREFILL_PAIR
 #undef MTJ_PREFILL_Q64
   return mtj_check_launch("mtj_attn_prefill");
+}
+
+}  // namespace
+
+extern "C" int mtj_attn_prefill(const void* q, const void* k_cache, const void* v_t, const int32_t* pos0, int64_t B,
+                                int64_t H, int64_t Tp, int64_t Tcap, int64_t dh, int64_t ldvt, void* out,
+                                int64_t ld_out, int dtype, const int32_t* key_limit, void* stream) {
+  return attn_prefill_impl(q, k_cache, v_t, pos0, B, H, Tp, Tcap, dh, ldvt, out, ld_out, dtype, key_limit, nullptr, stream);
+}
+
+extern "C" int mtj_attn_prefill_packed(const void* q, const void* k_cache, const void* v_t, const int32_t* pos0, int64_t B,
+                                       int64_t H, int64_t Tp, int64_t Tcap, int64_t dh, int64_t ldvt, void* out,
+                                       int64_t ld_out, int dtype, const int32_t* key_limit, const int32_t* skipped,
+                                       void* stream) {
+  MTJ_REQUIRE(skipped, MTJ_EINVAL, "mtj_attn_prefill_packed: null pointer");
+  return attn_prefill_impl(q, k_cache, v_t, pos0, B, H, Tp, Tcap, dh, ldvt, out, ld_out, dtype, key_limit, skipped, stream);
 }
 
 extern "C" int mtj_attn_decode_splits(int64_t B, int64_t H, int64_t Tcap) {

@@ -230,7 +230,7 @@ __global__ __launch_bounds__(256) void rope_append_kernel(const float* __restric
 
 extern "C" int mtj_rope_append(const float* q, const float* v, const float* k, int64_t M, const mtj_inproj* ip, void* stream) {
   MTJ_REQUIRE(ip && M > 0 && (q || v || k), MTJ_EINVAL, "mtj_rope_append: nothing to do");
-  MTJ_REQUIRE(ip->n_heads > 0 && ip->d_head > 0 && ip->d_head % 2 == 0 && ip->rotary_dims % 2 == 0 &&
+  MTJ_REQUIRE(!ip->rows && ip->n_heads > 0 && ip->d_head > 0 && ip->d_head % 2 == 0 && ip->rotary_dims % 2 == 0 &&
                   ip->rotary_dims >= 0 && ip->rotary_dims <= ip->d_head && ip->Tp > 0 && M % ip->Tp == 0 && ip->Tcap > 0 &&
                   ip->max_pos > 0 && ip->pos0 && ip->sin_tab && ip->cos_tab,
               MTJ_EINVAL, "mtj_rope_append: inconsistent geometry");

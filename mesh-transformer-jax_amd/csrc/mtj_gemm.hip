@@ -120,7 +120,7 @@ __device__ __forceinline__ void for_stages(F&& f) {
 struct epi_ops { floatx4 o[4]; };
 
 // Epilogue of a workgroup tile whose wavefront (wm, wn) holds WM x WN accumulator tiles of 32x32.  `smem` (the
-// operand staging area, no longer needed) must hold 2*BM ints and one 32x36 float patch per wavefront.
+// operand staging area, no longer needed) must hold 3*BM ints and one 32x36 float patch per wavefront.
 // Two accumulator layouts:
 //   MI16 false  acc is floatx16[WM][WN] from 32x32 MFMAs: register v of lane l holds C[8*(v/4) + 4*(l/32) + v%4][l%32];
 //   MI16 true   acc is floatx4[2*WM][2*WN] from 16x16x32 MFMAs issued with the WEIGHT fragment as the first operand:
@@ -257,16 +257,20 @@ __device__ __forceinline__ void epilogue(const gemm_args& a, void* out, ACC& acc
     __syncthreads();                                       // every wavefront is done with the operand tiles
     int* row_b = reinterpret_cast<int*>(smem);
     int* row_pos = row_b + BM;
-    float* patch = reinterpret_cast<float*>(smem) + 2 * BM + wave * (32 * PS);
+    int* row_t = row_pos + BM;
+    float* patch = reinterpret_cast<float*>(smem) + 3 * BM + wave * (32 * PS);
     for (int r = tid; r < BM; r += NT) {
       const int m = m0 + r;
-      int b = 0, pos = -1;
+      int b = 0, pos = -1, t = 0;
       if (m < a.M) {
-        b = m / a.ip.Tp;
-        pos = a.ip.pos0[b] + (m - b * a.ip.Tp);
+        const int rect = a.ip.rows ? a.ip.rows[m] : m;     // row of the [B, Tp] rectangle
+        b = rect / a.ip.Tp;
+        t = rect - b * a.ip.Tp;
+        pos = a.ip.pos0[b] + t;
       }
       row_b[r] = b;
       row_pos[r] = pos;
+      row_t[r] = t;
     }
     __syncthreads();
     const int d = a.ip.n_heads * a.ip.d_head, dh = a.ip.d_head, rd = a.ip.rotary_dims, Tp = a.ip.Tp;
@@ -354,7 +358,7 @@ __device__ __forceinline__ void epilogue(const gemm_args& a, void* out, ACC& acc
             }
             const int64_t bh = (int64_t)b * a.ip.n_heads + c.h;
             if (c.seg == 0) {
-              store16(a.ip.q, (bh * Tp + (m - b * Tp)) * dh + c.e0, val, a.ip.q_dtype);
+              store16(a.ip.q, (bh * Tp + row_t[r]) * dh + c.e0, val, a.ip.q_dtype);
             } else {
               const int slot = pos % a.ip.Tcap;
               store16(c.seg == 1 ? a.ip.v_cache : a.ip.k_cache, (bh * a.ip.Tcap + slot) * dh + c.e0, val, a.ip.kv_dtype);
@@ -935,7 +939,7 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(const gemm_args a) {
 template <typename T, int EPI, int BM, int S>
 int launch_stream(const gemm_args& a, hipStream_t s) {
   constexpr size_t lds = (size_t)S * (BM + 128) * 128;
-  static_assert(lds >= 2 * BM * sizeof(int) + 8 * 32 * 36 * sizeof(float), "epilogue scratch does not fit");
+  static_assert(lds >= 3 * BM * sizeof(int) + 8 * 32 * 36 * sizeof(float), "epilogue scratch does not fit");
   static mtj_device_once once;
   if (int rc = mtj_allow_lds(once, "mtj_gemm", &gemm_stream_kernel<T, EPI, BM, S>, lds)) return rc;
   gemm_stream_kernel<T, EPI, BM, S><<<(unsigned)((a.M + BM - 1) / BM * ((a.N + 127) / 128) * a.splits), 512, lds, s>>>(a);
@@ -957,7 +961,7 @@ int launch(const gemm_args& a, hipStream_t s) {
   constexpr int BM = WAVES_M * WM * 32, BN = WAVES_N * WN * 32;
   constexpr size_t lds = 2 * (size_t)(BM + BN) * (BK + mma<T>::EPC) * sizeof(T);
   static_assert(lds <= 160 * 1024, "tile does not fit LDS");
-  static_assert(lds >= 2 * BM * sizeof(int) + WAVES_M * WAVES_N * 32 * 36 * sizeof(float), "epilogue scratch does not fit");
+  static_assert(lds >= 3 * BM * sizeof(int) + WAVES_M * WAVES_N * 32 * 36 * sizeof(float), "epilogue scratch does not fit");
   static mtj_device_once once;
   if (int rc = mtj_allow_lds(once, "mtj_gemm", &gemm_kernel<T, EPI, WAVES_M, WAVES_N, WM, WN, BK, NS>, lds)) return rc;
   const int tiles = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
@@ -1266,7 +1270,7 @@ extern "C" int mtj_gemm(const void* A, int64_t lda, const void* W, const float* 
     MTJ_REQUIRE(ip && bias, MTJ_EINVAL, "mtj_gemm: INPROJ needs ip and the fc_in bias");
     a.ip = *ip;
     const int64_t d = (int64_t)ip->n_heads * ip->d_head;
-    MTJ_REQUIRE(ip->Tp > 0 && M % ip->Tp == 0 && N > 3 * d && N % 32 == 0 && d % 32 == 0 && ip->d_head % 32 == 0 &&
+    MTJ_REQUIRE(ip->Tp > 0 && (ip->rows || M % ip->Tp == 0) && N > 3 * d && N % 32 == 0 && d % 32 == 0 && ip->d_head % 32 == 0 &&
                     ip->rotary_dims % 16 == 0 && ip->ld_act % 16 == 0 &&
                     ip->rotary_dims <= ip->d_head && ip->Tcap > 0 && ip->max_pos > 0 && ip->pos0 && ip->sin_tab &&
                     ip->cos_tab && ip->q && ip->k_cache && ip->v_cache && ip->act && ip->ld_act >= N - 2 * d &&

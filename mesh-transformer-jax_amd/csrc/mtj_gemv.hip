@@ -719,7 +719,7 @@ extern "C" int mtj_gemv(const float* x, const float* ln_scale, const float* ln_o
     const int64_t d = (int64_t)ip->n_heads * ip->d_head;
     MTJ_REQUIRE((int64_t)ip->n_heads * ip->Tcap * ip->d_head < (1ll << 31) && N < (1ll << 31) && ip->ld_act < (1ll << 31), MTJ_ELIMIT,
                 "mtj_gemv: n_heads * Tcap * d_head, N and ld_act must be below 2^31");
-    MTJ_REQUIRE(ip->Tp == 1 && N > 3 * d && N % 2 == 0 && ip->rotary_dims % 2 == 0 && ip->rotary_dims <= ip->d_head &&
+    MTJ_REQUIRE(ip->Tp == 1 && !ip->rows && N > 3 * d && N % 2 == 0 && ip->rotary_dims % 2 == 0 && ip->rotary_dims <= ip->d_head &&
                     ip->Tcap > 0 && ip->max_pos > 0 && ip->pos0 && ip->sin_tab && ip->cos_tab && ip->q && ip->k_cache &&
                     ip->v_cache && ip->act && ip->ld_act >= N - 2 * d &&
                     mtj_is_dtype(ip->act_dtype) && mtj_is_dtype(ip->q_dtype) && mtj_is_dtype(ip->kv_dtype),

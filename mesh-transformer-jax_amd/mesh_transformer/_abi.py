@@ -9,7 +9,7 @@ import os
 
 F32, BF16, F16 = 0, 1, 2
 EPI_STORE, EPI_RESID, EPI_INPROJ = 0, 1, 2
-ABI_VERSION = 4
+ABI_VERSION = 5
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libmtj_hip.so")
 
@@ -25,6 +25,7 @@ class InProj(C.Structure):
         ("q", _p), ("q_dtype", C.c_int32), ("kv_dtype", C.c_int32),
         ("k_cache", _p), ("v_cache", _p), ("v_t", _p), ("ldvt", _i64),
         ("act", _p), ("ld_act", _i64), ("act_dtype", C.c_int32),
+        ("rows", _p),
     ]
 
 
@@ -60,6 +61,7 @@ SIGNATURES = {
     "mtj_gemv_attn_work_bytes": (_i64, [_i64, _i64]),
     "mtj_gemv_attn": (_i32, [_p, _p, _p, _i64, _i64, _i32, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i32, _p, _p]),
     "mtj_attn_prefill": (_i32, [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _p, _i64, _i32, _p, _p]),
+    "mtj_attn_prefill_packed": (_i32, [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _p, _i64, _i32, _p, _p, _p]),
     "mtj_attn_decode_splits": (_i32, [_i64, _i64, _i64]),
     "mtj_attn_decode_work_bytes": (_i64, [_i64, _i64, _i64, _i64]),
     "mtj_attn_decode_partials": (_i32, [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i32, _p, C.POINTER(AttnMerge), _p]),

@@ -240,7 +240,7 @@ class Engine:
         self.sessions = {}
 
     # ------------------------------------------------------------------ kernels
-    def _inproj(self, ses, layer, Tp, pos0, q, q_dtype, act, act_dtype, vt):
+    def _inproj(self, ses, layer, Tp, pos0, q, q_dtype, act, act_dtype, vt, rows=None):
         ip = InProj()
         ip.n_heads, ip.d_head, ip.rotary_dims = self.H, self.dh, self.r
         ip.Tp, ip.Tcap, ip.max_pos = Tp, ses.Tcap, ses.max_pos
@@ -249,21 +249,23 @@ class Engine:
         ip.k_cache, ip.v_cache = ptr(ses.kc[layer]), ptr(ses.vc[layer])
         ip.v_t, ip.ldvt = (ptr(vt), ses.ldvt) if vt is not None else (None, 0)
         ip.act, ip.ld_act, ip.act_dtype = ptr(act), act.stride(0), act_dtype
+        ip.rows = ptr(rows)
         return ip
 
-    def prefill(self, ses, tokens_rect, Tp, key_limit=None):
+    def prefill(self, ses, tokens, Tp, key_limit=None, packed=None):
         """generate_initial (transformer_shard.py:74-95) on a [B, Tp] right-aligned rectangle; the
-        dead logits projection of :95 is not computed."""
+        dead logits projection of :95 is not computed.  packed: (rows [M], skipped [B]) as mtj_inproj and
+        mtj_attn_prefill_packed take them, when `tokens` [M] and the rows returned are those of real tokens only."""
         L, w, s = _abi.lib(), self.w, _abi.stream_handle()
-        B, d, F = ses.B, w.d, w.F
-        M = B * Tp
+        d = w.d
+        M = tokens.numel()
         x, h, act = ses.x_pf[:M], ses.h_pf[:M], ses.act_pf[:M]
-        check(L.mtj_embed(ptr(tokens_rect), M, ptr(w.we), ptr(w.be), w.V, d, w.dtype, ptr(x), s))
+        check(L.mtj_embed(ptr(tokens), M, ptr(w.we), ptr(w.be), w.V, d, w.dtype, ptr(x), s))
         # as in batched decode: the launch that completes a layer's residual rows also normalises them for the next layer
         ids = w.layer_ids
         for j, i in enumerate(ids):
             nxt = (w.ln_s[ids[j + 1]], w.ln_o[ids[j + 1]]) if j + 1 < len(ids) else None
-            self.layer_prefill(ses, i, x, h, act, Tp, ses.pos0, key_limit, normed=j > 0, next_ln=nxt)
+            self.layer_prefill(ses, i, x, h, act, Tp, ses.pos0, key_limit, normed=j > 0, next_ln=nxt, packed=packed)
         return x
 
     def project(self, ses, x, out):
@@ -289,18 +291,21 @@ class Engine:
         check(L.mtj_gemm_xent(ptr(h), d, ptr(w.w_p_mm), ptr(w.b_p), M, V, d, w.mm_dtype, w.alpha_p, ptr(target),
                               ptr(loss), ptr(correct), ptr(ses.xent_work), ses.xent_work.numel() * 4, s))
 
-    def layer_prefill(self, ses, i, x, h, act, Tp, pos0, key_limit=None, normed=False, next_ln=None):
-        """One layer on [B * Tp] rows; normed and next_ln as in layer_decode, with h in the place of ses.h."""
+    def layer_prefill(self, ses, i, x, h, act, Tp, pos0, key_limit=None, normed=False, next_ln=None, packed=None):
+        """One layer on [B * Tp] rows, or on the rows of `packed` (see prefill); normed and next_ln as in layer_decode,
+        with h in the place of ses.h."""
         L, w, s = _abi.lib(), self.w, _abi.stream_handle()
         M, d, F = x.shape[0], w.d, w.F
         A = w.act_dtype
         if not normed:
             check(L.mtj_layernorm(ptr(x), ptr(w.ln_s[i]), ptr(w.ln_o[i]), M, d, ptr(h), A, s))
-        ip = self._inproj(ses, i, Tp, pos0, ses.q_pf, A, act, A, ses.vt)
+        rows, skipped = packed or (None, None)
+        ip = self._inproj(ses, i, Tp, pos0, ses.q_pf, A, act, A, ses.vt, rows)
         check(L.mtj_gemm(ptr(h), d, ptr(w.w_in_mm[i]), ptr(w.b1[i]), M, 3 * d + F, d, w.mm_dtype, EPI_INPROJ,
                          None, 0, 0, C.byref(ip), w.alpha_in[i], s))
-        check(L.mtj_attn_prefill(ptr(ses.q_pf), ptr(ses.kc[i]), ptr(ses.vt), ptr(pos0), ses.B, self.H, Tp, ses.Tcap,
-                                 self.dh, ses.ldvt, ptr(act), act.stride(0), A, ptr(key_limit), s))
+        att = (ptr(ses.q_pf), ptr(ses.kc[i]), ptr(ses.vt), ptr(pos0), ses.B, self.H, Tp, ses.Tcap, self.dh, ses.ldvt, ptr(act),
+               act.stride(0), A, ptr(key_limit))
+        check(L.mtj_attn_prefill(*att, s) if packed is None else L.mtj_attn_prefill_packed(*att, ptr(skipped), s))
         if next_ln is not None:
             check(L.mtj_gemm_splitk_ln(ptr(act), act.stride(0), ptr(w.w_out_mm[i]), ptr(w.b2[i]), M, d, d + F, w.mm_dtype,
                                        ptr(x), d, ptr(ses.gemm_work), ses.gemm_work.numel(), ptr(next_ln[0]), ptr(next_ln[1]),

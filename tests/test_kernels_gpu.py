@@ -594,6 +594,67 @@ def test_attn_prefill(L, dt, dh, H, Tp):
             assert rel_err(out[b * Tp:(b + 1) * Tp, :H * dh], ref) < ATT_TOL[dt], (dt, dh, Tp, b)
 
 
+@pytest.mark.parametrize("dt,dh,H,pads,Tp", [
+    ("f32", 64, 3, [0, 5, 40], 41), ("f32", 256, 2, [7, 0], 33), ("f16", 64, 2, [299, 0, 301], 301), ("bf16", 64, 2, [0, 1], 64),
+    ("f16", 256, 2, [0, 129, 199, 13], 200), ("bf16", 256, 1, [1, 0], 2),
+    ("f16", 256, 16, [(37 * b) % 270 for b in range(32)], 270)])      # the last one: two 256-query blocks, 1024 in all
+def test_attn_prefill_without_the_rows_of_padding(L, dt, dh, H, pads, Tp):
+    """mtj_attn_prefill_packed writes what mtj_attn_prefill writes, bit for bit, to the rows of real tokens only - every
+    kernel, sequences of padding only or of all but a token or two, nothing beyond the last row."""
+    a = abi()
+    g = torch.Generator().manual_seed(Tp + dh)
+    B, Tcap, ldvt, ld_out = len(pads), Tp + 3, (Tp + 63) // 64 * 64, H * dh + 16
+    mk = lambda *sh: torch.randn(*sh, generator=g).to(TD[dt]).to(DEV)
+    q, kc, vt = mk(B, H, Tp, dh), mk(B, H, Tcap, dh), mk(B, H, dh, ldvt)
+    pos0 = torch.tensor([-pd for pd in pads], dtype=torch.int32, device=DEV)
+    skipped = torch.tensor(pads, device=DEV).cumsum(0).to(torch.int32)
+    M = B * Tp - sum(pads)
+    rect, out = torch.zeros(B * Tp, ld_out, dtype=TD[dt], device=DEV), torch.full((M + 1, ld_out), 7.0, dtype=TD[dt], device=DEV)
+    args = (a.ptr(q), a.ptr(kc), a.ptr(vt), a.ptr(pos0), B, H, Tp, Tcap, dh, ldvt)
+    a.check(L.mtj_attn_prefill(*args, a.ptr(rect), ld_out, a.dtype_code(TD[dt]), None, S()))
+    a.check(L.mtj_attn_prefill_packed(*args, a.ptr(out), ld_out, a.dtype_code(TD[dt]), None, a.ptr(skipped), S()))
+    torch.cuda.synchronize()
+    real = torch.cat([torch.arange(Tp) >= pd for pd in pads]).to(DEV)
+    assert torch.equal(out[:M, :H * dh], rect[real][:, :H * dh])
+    assert bool((out[M] == 7.0).all()) and bool((out[:, H * dh:] == 7.0).all())
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("B,Tp,pads", [(3, 40, [0, 39, 7]), (4, 90, [90, 0, 41, 3]), (2, 600, [0, 37])])
+def test_inproj_gemm_without_the_rows_of_padding(L, dt, B, Tp, pads):
+    """The fused input projection on the rows of real tokens only fills q, the K/V window, V^T and gelu(fc_in) as the
+    rectangle does (a sequence without any row among them; another row count can take another tile shape, so float32
+    sums may differ in order) and writes nothing for padding."""
+    from mesh_transformer.engine import Engine
+    cfg = dict(layers=1, d_model=512, n_heads=8, n_vocab=64, pe="rotary", pe_rotary_dims=32, cores_per_replica=1)
+    a = abi()
+    p = {k: {n: v.to(DEV) for n, v in m.items()} for k, m in _layer_params(cfg, 3, dt).items()}
+    eng = Engine(cfg, p, DEV, layer_ids=[0], embed=False, proj=False)
+    ses = eng.session(B, Tp + 10, Tp, Tp + 20)
+    w, d, A = eng.w, 512, eng.w.act_dtype
+    h = torch.randn(B * Tp, d, generator=torch.Generator().manual_seed(Tp)).to(w.act_torch_dtype).to(DEV)
+    pos0 = torch.tensor([-pd for pd in pads], dtype=torch.int32, device=DEV)
+    real = torch.cat([torch.arange(Tp) >= pd for pd in pads]).to(DEV)
+    rows = real.nonzero().flatten().to(torch.int32)
+    got = []
+    for packed in (False, True):
+        for t in (ses.kc[0], ses.vc[0], ses.vt, ses.q_pf, ses.act_pf):
+            t.fill_(1000.0)
+        hh = h[real].contiguous() if packed else h
+        ip = eng._inproj(ses, 0, Tp, pos0, ses.q_pf, A, ses.act_pf, A, ses.vt, rows if packed else None)
+        a.check(L.mtj_gemm(a.ptr(hh), d, a.ptr(w.w_in_mm[0]), a.ptr(w.b1[0]), hh.shape[0], 3 * d + 4 * d, d, w.mm_dtype,
+                           a.EPI_INPROJ, None, 0, 0, C.byref(ip), w.alpha_in[0], S()))
+        torch.cuda.synchronize()
+        act = ses.act_pf[:, d:].clone()
+        got.append([ses.kc[0].clone(), ses.vc[0].clone(), ses.vt.clone(), ses.q_pf.clone(),
+                    act[:rows.numel()] if packed else act[real]])
+        if packed:
+            assert bool((act[rows.numel():] == 1000.0).all())
+    for x, y in zip(*got):
+        assert torch.equal(x == 1000.0, y == 1000.0)               # what is written and what is not
+        assert rel_err(x, y) < (1e-6 if dt == "f32" else 1e-3)
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 def test_attn_prefill_full_context_d256(L, dt):
     """2048 queries per sequence at d_head 256 with ragged left padding: 16 query blocks per head, dispatched longest
