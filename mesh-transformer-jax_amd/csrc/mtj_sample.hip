@@ -89,6 +89,7 @@ __device__ __forceinline__ float sub_product(float f, float a, float b) {
 namespace sel {
 constexpr int NB = 4096;         // buckets per pass
 constexpr int LIST_CAP = 1024;   // keys of the crossing bucket kept in LDS
+constexpr int LIST_PAIRS = 256;  // up to this many of them are compared pair by pair
 constexpr double Q_ZERO = -43.0; // exp(t) * 2^62 < 1 below this
 
 struct acc {                     // 96-bit unsigned
@@ -190,6 +191,12 @@ __device__ __forceinline__ acc bucket(const smem& S, int b) {
   return r;
 }
 
+__device__ __forceinline__ uint64_t readlane_u64(uint64_t v, int j) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, j);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), j);
+  return ((uint64_t)hi << 32) | lo;
+}
+
 struct scan_t {
   acc s[4];      // running sums over this thread's four buckets, in descending bucket order
   acc before;    // sum of the buckets ahead of them
@@ -219,12 +226,20 @@ __device__ __forceinline__ scan_t scan_hist(smem& S) {
   if (lane == 0) ex = acc{0, 0};
   if (lane == 63) { S.wave_lo[wave] = inc.lo; S.wave_hi[wave] = inc.hi; }
   __syncthreads();
-  acc base{0, 0}, grand{0, 0};
-  for (int w = 0; w < SNT / 64; ++w) {
-    const acc t{S.wave_lo[w], S.wave_hi[w]};
-    if (w < wave) base = add(base, t);
-    grand = add(grand, t);
+  // the sums of the 16 wavefronts, scanned by the lanes of every wavefront
+  acc tot{0, 0};
+  if (lane < SNT / 64) tot = acc{S.wave_lo[lane], S.wave_hi[lane]};
+#pragma unroll
+  for (int o = 1; o < SNT / 64; o <<= 1) {
+    acc t;
+    t.lo = __shfl_up((unsigned long long)tot.lo, o);
+    t.hi = __shfl_up(tot.hi, o);
+    if (lane >= o) tot = add(tot, t);
   }
+  const acc grand{readlane_u64(tot.lo, SNT / 64 - 1), (uint32_t)__builtin_amdgcn_readlane((int)tot.hi, SNT / 64 - 1)};
+  const int wv = __builtin_amdgcn_readfirstlane(wave), before = wv ? wv - 1 : 0;
+  acc base{readlane_u64(tot.lo, before), (uint32_t)__builtin_amdgcn_readlane((int)tot.hi, before)};
+  if (wv == 0) base = acc{0, 0};
   r.before = add(base, ex);
   r.grand = grand;
   return r;
@@ -254,11 +269,6 @@ __device__ __forceinline__ void clear_hist(smem& S) {
   for (int i = threadIdx.x; i < NB; i += SNT) { S.ha[i] = 0; S.hb[i] = 0; }
   if (threadIdx.x == 0) { S.digit = -1; S.hit = 0; }
 }
-__device__ __forceinline__ uint64_t readlane_u64(uint64_t v, int j) {
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, j);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), j);
-  return ((uint64_t)hi << 32) | lo;
-}
 
 // First key of the descending order at which the running sum of wq(l, id, key) exceeds thr(total) (a double in the
 // same 2^-62 units; negative: the first key with a weight; NaN or no crossing: returns false).  l0 is the row
@@ -274,11 +284,10 @@ __device__ __forceinline__ bool select(smem& S, const float (&l)[NT_MAX], int V,
 #pragma unroll
   for (int n = 0; n < NT_MAX; ++n) {
     const int id = opaque(tid) + n * SNT;
-    if (id < V) {
-      const float x = opaque(l[n]);
-      const uint64_t q = wq(x, (uint32_t)id, sort_key(x, (uint32_t)id));
-      if (q) hist_add<COUNT>(S, coarse(x, l0, scale), q);
-    }
+    const float x = opaque(l[n]);
+    const uint64_t w = wq(x, (uint32_t)id, sort_key(x, (uint32_t)id));
+    const uint64_t q = id < V ? w : 0;             // (selected, not branched around: one basic block less per token)
+    if (q) hist_add<COUNT>(S, coarse(x, l0, scale), q);
     __builtin_amdgcn_sched_barrier(0);   // one token at a time: fifty exponentials in flight would spill
   }
   __syncthreads();
@@ -316,6 +325,32 @@ __device__ __forceinline__ bool select(smem& S, const float (&l)[NT_MAX], int V,
         if (kj > key) ahead = t;
       }
       if (tid < n_list && !gt(ahead, T) && gt(add(ahead, acc{q, 0}), T)) { S.key = key; S.hit = 1; }
+    }
+    __syncthreads();
+    if (!S.hit) return false;                     // cannot happen: the sums are exact
+    key_out = S.key;
+    __syncthreads();
+    return true;
+  }
+  if (n_list <= LIST_PAIRS) {
+    // ---- one key per thread: the sum ahead of a key as above, the other keys and weights read from LDS (the same address
+    // for a whole wavefront).  Rows as flat as a normal distribution of deviation 2 put ~100 of 50400 tokens into a bucket, and
+    // four digits over it cost 8 000 cycles more.
+    uint64_t* qs = S.ha;                          // the histogram has been scanned
+    uint64_t key = 0, q = 0;
+    if (tid < n_list) {
+      key = S.list[tid];
+      q = wq(key_value(key), (uint32_t)(key & 0xffffu), key);
+      qs[tid] = q;
+    }
+    __syncthreads();
+    if (tid < n_list) {
+      acc ahead = above;
+      for (int j = 0; j < n_list; ++j) {
+        const acc t = add(ahead, acc{qs[j], 0});
+        if (S.list[j] > key) ahead = t;
+      }
+      if (!gt(ahead, T) && gt(add(ahead, acc{q, 0}), T)) { S.key = key; S.hit = 1; }
     }
     __syncthreads();
     if (!S.hit) return false;                     // cannot happen: the sums are exact
@@ -404,6 +439,11 @@ __device__ __forceinline__ uint64_t block_ext_u64(smem& S, uint64_t v, bool want
 constexpr size_t SEL_LDS_BYTES = sizeof(sel::smem);
 
 // One workgroup of 1024 threads per row; thread t keeps tokens t, t + 1024, ... in registers for every pass.
+// Bound by the ~50 vector instructions per token and selection pass (exponential, bucket), issued by the four wavefronts of
+// each SIMD of one CU: two or three passes of 38 000 cycles, 55 000 with the temperature, of 150 000 (61 us, 8 rows of
+// 50400 logits with deviation 2).  The LDS atomics (one 32-bit atomic in their place: 1 us) and two or five tokens at a
+// time (2 us slower) are not what it waits for.  With a division per token in the draw, a loop over the wavefronts' sums
+// in every thread and digits for buckets of 65 .. 256 tokens it took 77 us.
 template <int NT_MAX>        // tokens per thread: V <= 1024 * NT_MAX
 __global__ __launch_bounds__(SNT) void nucleus_kernel(const float* __restrict__ logits, int V,
                                                       const double* __restrict__ top_p, const double* __restrict__ temp,
@@ -493,7 +533,15 @@ __global__ __launch_bounds__(SNT) void nucleus_kernel(const float* __restrict__ 
   // In the usual case a token the filter touched has no weight at all (its filtered / temp is 1e10 / temp lower,
   // far below the 2^-62 that still counts) and needs no arithmetic; token 0 is exempt from the top-k penalty, which
   // multiplies by the token id.
-  const bool plain = tmp > 0.0 && tmp <= 1e6 && kk >= 1 && fabsf(l0) <= 1e6f;
+  const bool plain = tmp >= 1e-6 && tmp <= 1e6 && kk >= 1 && fabsf(l0) <= 1e6f;
+  // x / temp with one correctly rounded reciprocal for the row and one correction per token: the correctly rounded
+  // quotient (Markstein 1990; nothing overflows or is subnormal here), so the row maximum still gives 0 exactly.  A logit
+  // of -inf gives NaN, which has no weight either.
+  const double inv_tmp = 1.0 / tmp;
+  auto over_temp = [&](double x) {
+    const double r = x * inv_tmp;
+    return __builtin_fma(__builtin_fma(-r, tmp, x), inv_tmp, r);
+  };
   uint64_t key_t = 0;
   const bool hit = sel::select<NT_MAX, false>(
       S, l, V, l0, sel::coarse_scale(fminf(spread, tmp > 0.0 ? (float)fmin(43.0 * fmax(tmp, 1.0), 1e30) : 1e30f)),
@@ -501,7 +549,7 @@ __global__ __launch_bounds__(SNT) void nucleus_kernel(const float* __restrict__ 
         double t;
         if (plain) {
           if ((cut_p && key < key_p) || (cut_k && key < key_k && id != 0)) return (uint64_t)0;
-          t = (double)x / tmp - tmax;
+          t = over_temp((double)x) - tmax;
         } else {
           t = (double)filtered_of(x, id, key) / tmp - tmax;
         }

@@ -1024,6 +1024,23 @@ def test_nucleus_unusual_parameters(L):
     _check_rows(L, logits[:, :1].copy(), top_p, temp, None, u)          # a vocabulary of one
 
 
+@pytest.mark.parametrize("n", [1, 64, 65, 255, 256, 257, 1024, 1025])
+def test_nucleus_bucket_sizes(L, n):
+    """n tokens in the one bucket that both crossings fall into - by equal values, by values a few ulp apart - on either
+    side of the sizes at which the selection inside a bucket changes its method, at temperatures on either side of those
+    it divides by with a reciprocal."""
+    rng = np.random.default_rng(n)
+    V, R = 3000, 8
+    logits = (rng.standard_normal((R, V)) * 0.5 - 12.0).astype(np.float32)
+    for r in range(R):
+        at = rng.permutation(V)[:n]
+        logits[r, at] = 1.25 if r % 2 else np.float32(1.25) + rng.integers(0, 40, n).astype(np.float32) * np.float32(2 ** -23)
+    temp = np.array([1.0, 0.3, 1e-6, 9e-7, 1e6, 1.1e6, 0.7, 2.0])
+    for u in (rng.random(R), np.zeros(R), np.full(R, 0.999)):
+        _check_rows(L, logits, rng.uniform(0.05, 0.95, R), temp, None, u)
+    _check_rows(L, logits, np.full(R, 0.9), temp, np.array([max(1, n // 2)] * R, np.int32), rng.random(R))
+
+
 def test_nucleus_against_the_committed_fixture(L):
     """tests/golden/nucleus_cases.npz: keep-masks and tokens bit for bit."""
     import os
