@@ -790,6 +790,17 @@ def test_attn_decode_window(L, dt, dh, H, Tcap, positions):
 
 
 @pytest.mark.parametrize("dt", ["f32", "f16"])
+@pytest.mark.parametrize("dh,H,Tcap,positions,ranges", [
+    (256, 16, 700, [0, 1, 2, 63, 64, 650, 699, 900], 4), (64, 16, 300, [5, 40, 299, 130, 77, 3], 4),     # 128, 96 pairs
+    (256, 16, 40, [39, 0, 7, 8, 9, 20, 15, 16], 3), (256, 16, 60, [1, 50, 59, 3, 8], 3)])               # few slots; 80 pairs
+def test_attn_decode_four_ranges_per_sequence(L, dt, dh, H, Tcap, positions, ranges):
+    """A batch for which two key ranges per (sequence, head) would fill the chip is cut into four: ranges without any
+    key, windows too short for four."""
+    assert L.mtj_attn_decode_splits(len(positions), H, Tcap) == ranges
+    test_attn_decode_window(L, dt, dh, H, Tcap, positions)
+
+
+@pytest.mark.parametrize("dt", ["f32", "f16"])
 @pytest.mark.parametrize("dh,H,F", [(64, 8, 2048), (256, 16, 16384)])
 @pytest.mark.parametrize("Tcap,p", [(2047, 650), (2047, 2046), (130, 3), (9, 40)])
 def test_attn_decode_partials_merged_by_the_out_projection_gemv(L, dt, dh, H, F, Tcap, p):
