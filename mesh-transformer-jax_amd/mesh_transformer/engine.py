@@ -38,9 +38,9 @@ def _f32(t):
 
 
 def splitk_work_bound(M_max, N, K, dtype):
-    """Bytes of split-K workspace that cover every row count 1 .. M_max of an [M, K] x [K, N] product.  The number of
-    K ranges falls as M grows, so the need is not monotonic in M; it is constant in the number of ranges between
-    multiples of 128 rows (and below 64 rows), so those row counts are the candidates."""
+    """Bytes of split-K workspace that cover every row count 1 .. M_max of an [M, K] x [K, N] product.  The cut
+    into K ranges changes with M, so the need is not monotonic in M; between multiples of 128 rows (and below 64 rows) the
+    cut is the same and the need grows with M, so those row counts are the candidates."""
     L = _abi.lib()
     cand = set(range(1, min(M_max, 64) + 1)) | set(range(128, M_max + 1, 128)) | {M_max}
     return max(L.mtj_gemm_splitk_work_bytes(m, N, K, dtype) for m in cand)
