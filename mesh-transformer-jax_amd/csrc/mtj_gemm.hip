@@ -1230,6 +1230,18 @@ cut_t pick_cut(int64_t M, int64_t N, int64_t K, int dtype) {
   return {0, splits};
 }
 
+// Problems whose tiles of one K range leave more than half of the chip idle: mtj_gemm_splitk asks for an `out` that the
+// reduce can take in quads for these, whatever pick_cut makes of them.  Every other problem can also run in one range.
+// (Tiles of 128 columns up to 64 rows, of 128 x 128 beyond, two workgroups per CU; 16-bit operands also count the
+// 256 x 256 tiles that two ranges bring to 200 .. 256; a range has at least 4 or 16 k-tiles.)
+bool needs_ranges(int64_t M, int64_t N, int64_t K, int dtype) {
+  const int64_t kt = K / (dtype == MTJ_F32 ? 32 : 64), cols = (N + 127) / 128;
+  if (N % 4 || kt % 2) return false;
+  if (M <= 64) return cols <= 128 && kt >= 8;
+  const int64_t big = dma_tiles(M, N);
+  return kt >= 32 && ((M + 127) / 128 * cols <= 256 || (dtype != MTJ_F32 && big >= 100 && big <= 128));
+}
+
 int check_common(const void* A, int64_t lda, const void* W, int64_t M, int64_t N, int64_t K, int dtype, const char* who) {
   MTJ_REQUIRE(A && W, MTJ_EINVAL, "%s: null pointer", who);
   MTJ_REQUIRE(mtj_is_dtype(dtype), MTJ_EDTYPE, "%s: dtype %d", who, dtype);
@@ -1302,14 +1314,12 @@ extern "C" int mtj_gemm_splitk(const void* A, int64_t lda, const void* W, const 
   if (int rc = check_common(A, lda, W, M, N, K, dtype, "mtj_gemm_splitk")) return rc;
   const cut_t cut = pick_cut(M, N, K, dtype);
   const int splits = cut.splits;
-  // the reduce moves four columns at a time: rows that do not allow that are taken in one range where a problem of this
-  // size need not be split (more than 64 tiles or an odd number of k-tiles), and refused where it always is
+  // the reduce moves four columns at a time
   const bool rows_ok = out && ldo >= N && ldo % 4 == 0 && mtj_aligned16(out) && (!bias || mtj_aligned16(bias));
-  const bool one_range = !rows_ok && M > 256 && dtype != MTJ_F32 && (dma_tiles(M, N) > 64 || K / 64 % 2);
-  if (splits == 1 || one_range)
-    return mtj_gemm(A, lda, W, bias, M, N, K, dtype, epi, out, ldo, out_dtype, nullptr, alpha, stream);
-  MTJ_REQUIRE(rows_ok, MTJ_EINVAL,
+  MTJ_REQUIRE(rows_ok || !needs_ranges(M, N, K, dtype), MTJ_EINVAL,
               "mtj_gemm_splitk: out needs ldo >= N, a multiple of 4, and 16-byte alignment (bias too)");
+  if (splits == 1 || !rows_ok)
+    return mtj_gemm(A, lda, W, bias, M, N, K, dtype, epi, out, ldo, out_dtype, nullptr, alpha, stream);
   MTJ_REQUIRE(epi == MTJ_EPI_RESID || mtj_is_dtype(out_dtype), MTJ_EDTYPE, "mtj_gemm_splitk: out_dtype %d", out_dtype);
   MTJ_REQUIRE(work && mtj_aligned16(work) && work_bytes >= (int64_t)splits * (M - cut.front) * N * (int64_t)sizeof(float),
               MTJ_EINVAL, "mtj_gemm_splitk: work must hold mtj_gemm_splitk_work_bytes() bytes");

@@ -112,6 +112,55 @@ def test_session_workspace_covers_every_prompt_length():
     assert lib.mtj_gemm_splitk_work_bytes(8 * 99, 4096, 20480, _abi.F16) > lib.mtj_gemm_splitk_work_bytes(8 * 599, 4096, 20480, _abi.F16)
 
 
+def _needs_ranges(lib, M, N, K, dtype):
+    """The products that mtj_gemm_splitk has always cut into K ranges, and for which it asks for rows that its reduce can
+    take: ranges are doubled while they are no more than the CUs (128-column tiles, 256 x 256 tiles) or two per CU
+    (128 x 128 tiles) and keep 4 or 16 k-tiles each."""
+    from mesh_transformer import _abi
+    up = lambda a, b: -(-a // b)
+    kt = K // (32 if dtype == _abi.F32 else 64)
+    if N % 4:
+        return False
+
+    def doubled(tiles, limit, most, least):
+        s = 1
+        while s < most and tiles * s * 2 <= limit and kt % (s * 2) == 0 and kt // (s * 2) >= least:
+            s *= 2
+        return s
+    if M <= 64:
+        return doubled(up(N, 128), 256, 16, 4) > 1
+    if dtype != _abi.F32:
+        big = up(M, 256) * up(N, 256)
+        s = doubled(big, 256, 16, 16)
+        if big * s >= 200:
+            return s > 1
+    return doubled(up(M, 128) * up(N, 128), 512, 4, 16) > 1
+
+
+def _splitk_sizes():
+    for M in (1, 33, 64, 65, 100, 128, 129, 200, 256, 257, 384, 700, 1025, 1808, 2048, 3195, 4097, 9000):
+        for N in (64, 408, 512, 1024, 2048, 4096, 4098, 8192, 16384, 25600, 32768):
+            for K in (64, 256, 512, 704, 1024, 1984, 2048, 2560, 4096, 20480):
+                yield M, N, K
+
+
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+def test_splitk_takes_rows_of_any_alignment_where_it_need_not_cut(dtype):
+    """An `out` whose rows are no whole number of quads, an unaligned out and an unaligned bias are refused only where the
+    product is always cut into K ranges; elsewhere the call passes the checks (and then finds no device here)."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("the pointers of this test must never reach a GPU")
+    from mesh_transformer import _abi
+    lib, P = _abi.lib(), 1 << 20
+    for M, N, K in _splitk_sizes():
+        nb = lib.mtj_gemm_splitk_work_bytes(M, N, K, dtype)
+        for out, bias, ldo in ((P, P, N + 2), (P + 4, P, N), (P, P + 4, N)):
+            rc = lib.mtj_gemm_splitk(P, K, P, bias, M, N, K, dtype, _abi.EPI_RESID, out, ldo, 0, P, nb, 1.0, None)
+            refused = rc == -1
+            assert rc in (-1, -4) and refused == _needs_ranges(lib, M, N, K, dtype), (M, N, K, out, bias, ldo, rc)
+
+
 def test_torch_ops_are_registered_for_the_gpu_only():
     """Every kernel entry point is a dispatcher-visible operator torch.ops.mtj.*; there is no CPU implementation, so
     host tensors are refused by the dispatcher instead of taking another path."""

@@ -263,6 +263,37 @@ def test_out_projection_is_cut_into_even_rounds(L, M, N, K, splits, front):
     assert bool((h[M] == 0).all()) and bool((work[nb:] == 7).all())
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 512, 512), (100, 1024, 1024), (223, 640, 1024), (256, 2048, 1984), (700, 4096, 1984)])
+@pytest.mark.parametrize("ld,shift", [(2, 0), (3, 0), (0, 1)])
+def test_splitk_on_rows_that_the_reduce_cannot_take(L, M, N, K, ld, shift):
+    """Few-row products with a short K that could be cut into ranges but need not be: `x` with a row pitch that is no
+    whole number of quads, or at an address that is not 16-byte aligned, through mtj_gemm_splitk and through
+    torch.ops.mtj.gemm_resid_.  Operands are rounded already: only the float32 accumulation differs from float64."""
+    from mesh_transformer import ops  # noqa: F401
+    a = abi()
+    g = torch.Generator().manual_seed(M + N + K)
+    A = torch.randn(M, K, generator=g).to(torch.float16).to(DEV)
+    Wh = (torch.randn(K, N, generator=g) * 0.05).to(torch.float16).to(DEV)
+    bias = torch.randn(N, generator=g).to(DEV)
+    W = _packed(Wh)
+    x0 = torch.randn(M, N, generator=g).to(DEV)
+    ref = x0.double() + A.double() @ Wh.double() + bias.double()
+    nb = L.mtj_gemm_splitk_work_bytes(M, N, K, a.F16)
+    work = torch.empty(max(nb, 16), dtype=torch.uint8, device=DEV)
+    for op in (False, True):
+        store = torch.full(((M + 1) * (N + ld) + shift,), 7.0, device=DEV)
+        x = store[shift:].view(M + 1, N + ld)
+        x[:M, :N] = x0
+        if op:
+            torch.ops.mtj.gemm_resid_(x[:M, :N], A, W, bias, 1.0)
+        else:
+            a.check(L.mtj_gemm_splitk(a.ptr(A), K, a.ptr(W), a.ptr(bias), M, N, K, a.F16, a.EPI_RESID, a.ptr(x), N + ld, 0,
+                                      a.ptr(work), nb, 1.0, S()))
+        torch.cuda.synchronize()
+        assert rel_err(x[:M, :N], ref) < 5e-6
+        assert bool((x[M] == 7.0).all()) and bool((x[:, N:] == 7.0).all())
+
+
 @pytest.mark.parametrize("dt", DTS)
 @pytest.mark.parametrize("M,N,K", [(32, 4096, 20480), (5, 512, 2560), (3, 64, 64), (8, 1024, 4096)])
 def test_gemm_splitk_with_the_following_layernorm(L, dt, M, N, K):
