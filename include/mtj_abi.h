@@ -167,7 +167,8 @@ int mtj_gemm_splitk(const void* A, int64_t lda, const void* W, const float* bias
 /* mtj_gemm_splitk with the RESID epilogue, followed in the same launch by the LayerNorm of the rows it completes:
  * x [M, ldx] float32 += A x W^T + bias, then h [M, ldh] (h_dtype) = ReplicatedLayerNorm(x) with ln_scale / ln_offset
  * [N] (layers.py:17-36) - the LayerNorm of the next layer, or of the projection, that follows the residual add in
- * generate_once (transformer_shard.py:97-115).  `work` as for mtj_gemm_splitk; N <= 16384. */
+ * generate_once (transformer_shard.py:97-115).  `work` as for mtj_gemm_splitk; N <= 16384.
+ * ldx and ldh may exceed N (a multiple of 4, rows 16-byte aligned) where mtj_gemm_splitk asks for aligned rows. */
 int mtj_gemm_splitk_ln(const void* A, int64_t lda, const void* W, const float* bias, int64_t M, int64_t N, int64_t K,
                        int dtype, float* x, int64_t ldx, void* work, int64_t work_bytes, const float* ln_scale,
                        const float* ln_offset, void* h, int64_t ldh, int h_dtype, float alpha, void* stream);

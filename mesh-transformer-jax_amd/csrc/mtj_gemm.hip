@@ -1196,6 +1196,9 @@ cut_t pick_cut(int64_t M, int64_t N, int64_t K, int dtype) {
     if (tiles <= 256) {
       for (int s = 2; s <= 16 && kt / s >= 16; ++s)
         if (dma_cost(tiles, kt, s) < dma_cost(tiles, kt, splits)) splits = s;
+      // a short K, whose partials weigh as much as the walk they save: two ranges as long as they fill the chip (K = 2432,
+      // N = 4096, 1808 rows 62 us, one range of 128 x 128 tiles 71; N = 512, K = 2560, 14000 rows 75 and 86)
+      if (splits == 1 && tiles >= 100 && tiles <= 128 && kt % 2 == 0 && kt >= 32) splits = 2;
       if (tiles * splits >= DMA_MIN_TILES) return {0, splits};
       splits = 1;
     } else {
@@ -1357,16 +1360,17 @@ extern "C" int mtj_gemm_splitk_ln(const void* A, int64_t lda, const void* W, con
   if (int rc = check_common(A, lda, W, M, N, K, dtype, "mtj_gemm_splitk_ln")) return rc;
   const cut_t cut = pick_cut(M, N, K, dtype);
   const int splits = cut.splits;
+  // mtj_layernorm takes dense rows; pick_cut leaves none to it where needs_ranges holds (N <= 16384)
+  MTJ_REQUIRE((ldx == N && ldh == N) || needs_ranges(M, N, K, dtype), MTJ_EINVAL,
+              "mtj_gemm_splitk_ln: x and h must be dense where one K range fills the chip");
   hipStream_t s = (hipStream_t)stream;
   if (splits == 1) {      // no partials to reduce: the product with its own residual epilogue, then the plain LayerNorm
-    MTJ_REQUIRE(ldx == N && ldh == N, MTJ_EINVAL, "mtj_gemm_splitk_ln: without a split, x and h must be dense");
     if (int rc = mtj_gemm(A, lda, W, bias, M, N, K, dtype, MTJ_EPI_RESID, x, ldx, MTJ_F32, nullptr, alpha, stream)) return rc;
     return mtj_layernorm(x, ln_scale, ln_offset, M, N, h, h_dtype, stream);
   }
   MTJ_REQUIRE(work && mtj_aligned16(work) && work_bytes >= (int64_t)splits * (M - cut.front) * N * (int64_t)sizeof(float),
               MTJ_EINVAL, "mtj_gemm_splitk_ln: work must hold mtj_gemm_splitk_work_bytes() bytes");
   if (cut.front) {
-    MTJ_REQUIRE(ldx == N && ldh == N, MTJ_EINVAL, "mtj_gemm_splitk_ln: rows without a split must be dense in x and h");
     if (int rc = mtj_gemm(A, lda, W, bias, cut.front, N, K, dtype, MTJ_EPI_RESID, x, ldx, MTJ_F32, nullptr, alpha, stream)) return rc;
     if (int rc = mtj_layernorm(x, ln_scale, ln_offset, cut.front, N, h, h_dtype, stream)) return rc;
     A = rows_from(A, cut.front * lda, dtype);

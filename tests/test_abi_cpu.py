@@ -161,6 +161,27 @@ def test_splitk_takes_rows_of_any_alignment_where_it_need_not_cut(dtype):
             assert rc in (-1, -4) and refused == _needs_ranges(lib, M, N, K, dtype), (M, N, K, out, bias, ldo, rc)
 
 
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+def test_splitk_ln_takes_padded_rows_where_it_always_cuts(dtype):
+    """x and h with padded rows: taken exactly where the product is always cut into K ranges, and then every row goes
+    through the reduce (the workspace holds whole copies of the output), since the separate LayerNorm wants dense rows."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("the pointers of this test must never reach a GPU")
+    from mesh_transformer import _abi
+    lib, P = _abi.lib(), 1 << 20
+    for M, N, K in _splitk_sizes():
+        if N % 4 or N > 16384:
+            continue
+        nb = lib.mtj_gemm_splitk_work_bytes(M, N, K, dtype)
+        need = _needs_ranges(lib, M, N, K, dtype)
+        if need:
+            assert nb >= 2 * M * N * 4 and nb % (M * N * 4) == 0, (M, N, K, nb)
+        for ldx, ldh in ((N + 8, N), (N, N + 8), (N, N)):
+            rc = lib.mtj_gemm_splitk_ln(P, K, P, P, M, N, K, dtype, P, ldx, P, nb, P, P, P, ldh, dtype, 1.0, None)
+            assert (rc == -1) == (not need and (ldx, ldh) != (N, N)), (M, N, K, ldx, ldh, rc)
+
+
 def test_torch_ops_are_registered_for_the_gpu_only():
     """Every kernel entry point is a dispatcher-visible operator torch.ops.mtj.*; there is no CPU implementation, so
     host tensors are refused by the dispatcher instead of taking another path."""

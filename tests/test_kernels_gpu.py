@@ -294,6 +294,31 @@ def test_splitk_on_rows_that_the_reduce_cannot_take(L, M, N, K, ld, shift):
         assert bool((x[M] == 7.0).all()) and bool((x[:, N:] == 7.0).all())
 
 
+@pytest.mark.parametrize("M,N,K", [(1808, 4096, 2432), (3195, 2048, 2560), (100, 512, 2560), (768, 1024, 5120)])
+def test_splitk_layernorm_on_padded_rows(L, M, N, K):
+    """x and h with padded rows, at a short K (128 and 104 tiles of 256 x 256 in two ranges) and at few rows: the padding
+    stays as it was.  Bounds as in test_out_projection_is_cut_into_even_rounds."""
+    a = abi()
+    g = torch.Generator().manual_seed(M + N + K)
+    A = torch.randn(M, K, generator=g).to(torch.float16).to(DEV)
+    Wh = (torch.randn(K, N, generator=g) * 0.05).to(torch.float16).to(DEV)
+    bias, sc, of = torch.randn(N, generator=g).to(DEV), (1 + 0.1 * torch.randn(N, generator=g)).to(DEV), (0.1 * torch.randn(N, generator=g)).to(DEV)
+    W = _packed(Wh)
+    x = torch.full((M + 1, N + 4), 7.0, device=DEV)
+    x[:M, :N] = torch.randn(M, N, generator=g).to(DEV)
+    h = torch.full((M + 1, N + 8), 7.0, dtype=torch.float16, device=DEV)
+    ref = x[:M, :N].double() + A.double() @ Wh.double() + bias.double()
+    nb = L.mtj_gemm_splitk_work_bytes(M, N, K, a.F16)
+    work = torch.empty(nb, dtype=torch.uint8, device=DEV)
+    a.check(L.mtj_gemm_splitk_ln(a.ptr(A), K, a.ptr(W), a.ptr(bias), M, N, K, a.F16, a.ptr(x), N + 4, a.ptr(work), nb,
+                                 a.ptr(sc), a.ptr(of), a.ptr(h), N + 8, a.F16, 1.0, S()))
+    torch.cuda.synchronize()
+    assert rel_err(x[:M, :N], ref) < 5e-6
+    assert rel_err(h[:M, :N], torch.nn.functional.layer_norm(ref, (N,), sc.double(), of.double(), 1e-5)) < 5e-4
+    for t, n in ((x, N), (h, N)):
+        assert bool((t[M] == 7.0).all()) and bool((t[:, n:] == 7.0).all())
+
+
 @pytest.mark.parametrize("dt", DTS)
 @pytest.mark.parametrize("M,N,K", [(32, 4096, 20480), (5, 512, 2560), (3, 64, 64), (8, 1024, 4096)])
 def test_gemm_splitk_with_the_following_layernorm(L, dt, M, N, K):
