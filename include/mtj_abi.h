@@ -153,7 +153,7 @@ int mtj_gemm(const void* A, int64_t lda, const void* W, const float* bias, int64
  * float32 partial tile into `work`, and a second kernel adds the partials in a fixed order (results do not depend on
  * scheduling) and applies the epilogue; when it has some more than whole rounds of tiles, the last rows are such a
  * problem of their own.  STORE and RESID only.  `work` holds mtj_gemm_splitk_work_bytes() bytes (0: no split is used
- * and the call is mtj_gemm).  The reduce needs out and bias 16-byte aligned and ldo a multiple of 4.  That is required
+ * and the call is mtj_gemm).  The reduce needs them, out and bias 16-byte aligned and ldo a multiple of 4.  That is required
  * where one K range would leave more than half of the chip idle (K of an even number of k-tiles - 64 columns, 32 in
  * float32 -, at least 8 of them, up to 128 tiles of 128 columns up to 64 rows; at least 32, up to 256 tiles of
  * 128 x 128 or 16-bit operands with 100 .. 128 tiles of 256 x 256 beyond); elsewhere a call that does not meet it

@@ -1233,8 +1233,16 @@ cut_t pick_cut(int64_t M, int64_t N, int64_t K, int dtype) {
   return {0, splits};
 }
 
+int64_t cut_bytes(const cut_t& cut, int64_t M, int64_t N) {
+  return cut.splits > 1 ? (int64_t)cut.splits * (M - cut.front) * N * (int64_t)sizeof(float) : 0;
+}
+bool work_holds(const cut_t& cut, int64_t M, int64_t N, const void* work, int64_t work_bytes) {
+  return work && mtj_aligned16(work) && work_bytes >= cut_bytes(cut, M, N);
+}
+
 // Problems whose tiles of one K range leave more than half of the chip idle: mtj_gemm_splitk asks for an `out` that the
-// reduce can take in quads for these, whatever pick_cut makes of them.  Every other problem can also run in one range.
+// reduce can take in quads, and for the workspace, for these, whatever pick_cut makes of them.  Every other problem can
+// also run in one range, and does where these do not allow a cut.
 // (Tiles of 128 columns up to 64 rows, of 128 x 128 beyond, two workgroups per CU; 16-bit operands also count the
 // 256 x 256 tiles that two ranges bring to 200 .. 256; a range has at least 4 or 16 k-tiles.)
 bool needs_ranges(int64_t M, int64_t N, int64_t K, int dtype) {
@@ -1306,8 +1314,7 @@ extern "C" int mtj_gemm(const void* A, int64_t lda, const void* W, const float* 
 
 extern "C" int64_t mtj_gemm_splitk_work_bytes(int64_t M, int64_t N, int64_t K, int dtype) {
   if (M <= 0 || N <= 0 || K <= 0 || !mtj_is_dtype(dtype)) return 0;
-  const cut_t cut = pick_cut(M, N, K, dtype);
-  return cut.splits > 1 ? (int64_t)cut.splits * (M - cut.front) * N * (int64_t)sizeof(float) : 0;
+  return cut_bytes(pick_cut(M, N, K, dtype), M, N);
 }
 
 extern "C" int mtj_gemm_splitk(const void* A, int64_t lda, const void* W, const float* bias, int64_t M, int64_t N,
@@ -1319,13 +1326,13 @@ extern "C" int mtj_gemm_splitk(const void* A, int64_t lda, const void* W, const 
   const int splits = cut.splits;
   // the reduce moves four columns at a time
   const bool rows_ok = out && ldo >= N && ldo % 4 == 0 && mtj_aligned16(out) && (!bias || mtj_aligned16(bias));
-  MTJ_REQUIRE(rows_ok || !needs_ranges(M, N, K, dtype), MTJ_EINVAL,
+  const bool need = needs_ranges(M, N, K, dtype);
+  MTJ_REQUIRE(rows_ok || !need, MTJ_EINVAL,
               "mtj_gemm_splitk: out needs ldo >= N, a multiple of 4, and 16-byte alignment (bias too)");
-  if (splits == 1 || !rows_ok)
+  if (splits == 1 || !rows_ok || (!need && !work_holds(cut, M, N, work, work_bytes)))
     return mtj_gemm(A, lda, W, bias, M, N, K, dtype, epi, out, ldo, out_dtype, nullptr, alpha, stream);
   MTJ_REQUIRE(epi == MTJ_EPI_RESID || mtj_is_dtype(out_dtype), MTJ_EDTYPE, "mtj_gemm_splitk: out_dtype %d", out_dtype);
-  MTJ_REQUIRE(work && mtj_aligned16(work) && work_bytes >= (int64_t)splits * (M - cut.front) * N * (int64_t)sizeof(float),
-              MTJ_EINVAL, "mtj_gemm_splitk: work must hold mtj_gemm_splitk_work_bytes() bytes");
+  MTJ_REQUIRE(work_holds(cut, M, N, work, work_bytes), MTJ_EINVAL, "mtj_gemm_splitk: work must hold mtj_gemm_splitk_work_bytes() bytes");
   if (cut.front) {
     if (int rc = mtj_gemm(A, lda, W, bias, cut.front, N, K, dtype, epi, out, ldo, out_dtype, nullptr, alpha, stream)) return rc;
     A = rows_from(A, cut.front * lda, dtype);
@@ -1361,15 +1368,15 @@ extern "C" int mtj_gemm_splitk_ln(const void* A, int64_t lda, const void* W, con
   const cut_t cut = pick_cut(M, N, K, dtype);
   const int splits = cut.splits;
   // mtj_layernorm takes dense rows; pick_cut leaves none to it where needs_ranges holds (N <= 16384)
-  MTJ_REQUIRE((ldx == N && ldh == N) || needs_ranges(M, N, K, dtype), MTJ_EINVAL,
+  const bool need = needs_ranges(M, N, K, dtype);
+  MTJ_REQUIRE((ldx == N && ldh == N) || need, MTJ_EINVAL,
               "mtj_gemm_splitk_ln: x and h must be dense where one K range fills the chip");
   hipStream_t s = (hipStream_t)stream;
-  if (splits == 1) {      // no partials to reduce: the product with its own residual epilogue, then the plain LayerNorm
+  if (splits == 1 || (!need && !work_holds(cut, M, N, work, work_bytes))) {      // no partials to reduce: the product with its own residual epilogue, then the plain LayerNorm
     if (int rc = mtj_gemm(A, lda, W, bias, M, N, K, dtype, MTJ_EPI_RESID, x, ldx, MTJ_F32, nullptr, alpha, stream)) return rc;
     return mtj_layernorm(x, ln_scale, ln_offset, M, N, h, h_dtype, stream);
   }
-  MTJ_REQUIRE(work && mtj_aligned16(work) && work_bytes >= (int64_t)splits * (M - cut.front) * N * (int64_t)sizeof(float),
-              MTJ_EINVAL, "mtj_gemm_splitk_ln: work must hold mtj_gemm_splitk_work_bytes() bytes");
+  MTJ_REQUIRE(work_holds(cut, M, N, work, work_bytes), MTJ_EINVAL, "mtj_gemm_splitk_ln: work must hold mtj_gemm_splitk_work_bytes() bytes");
   if (cut.front) {
     if (int rc = mtj_gemm(A, lda, W, bias, cut.front, N, K, dtype, MTJ_EPI_RESID, x, ldx, MTJ_F32, nullptr, alpha, stream)) return rc;
     if (int rc = mtj_layernorm(x, ln_scale, ln_offset, cut.front, N, h, h_dtype, stream)) return rc;

@@ -182,6 +182,28 @@ def test_splitk_ln_takes_padded_rows_where_it_always_cuts(dtype):
             assert (rc == -1) == (not need and (ldx, ldh) != (N, N)), (M, N, K, ldx, ldh, rc)
 
 
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+def test_splitk_without_a_workspace_where_it_need_not_cut(dtype):
+    """No workspace, or one that is too small: refused where the product is always cut into K ranges, one range elsewhere -
+    also where a cut would be faster."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("the pointers of this test must never reach a GPU")
+    from mesh_transformer import _abi
+    lib, P = _abi.lib(), 1 << 20
+    for M, N, K in _splitk_sizes():
+        nb = lib.mtj_gemm_splitk_work_bytes(M, N, K, dtype)
+        refused = _needs_ranges(lib, M, N, K, dtype) and nb > 0
+        for work, have in ((None, nb), (P, nb - 4), (P + 4, nb)):
+            if nb == 0 and have < 0:
+                continue
+            rc = lib.mtj_gemm_splitk(P, K, P, P, M, N, K, dtype, _abi.EPI_RESID, P, N, 0, work, have, 1.0, None)
+            assert rc in (-1, -4) and (rc == -1) == refused, (M, N, K, work, have, rc)
+            if N % 4 == 0 and N <= 4096:                      # (the separate LayerNorm takes no longer rows)
+                rc = lib.mtj_gemm_splitk_ln(P, K, P, P, M, N, K, dtype, P, N, work, have, P, P, P, N, dtype, 1.0, None)
+                assert rc in (-1, -4) and (rc == -1) == refused, (M, N, K, work, have, rc)
+
+
 def test_torch_ops_are_registered_for_the_gpu_only():
     """Every kernel entry point is a dispatcher-visible operator torch.ops.mtj.*; there is no CPU implementation, so
     host tensors are refused by the dispatcher instead of taking another path."""

@@ -294,6 +294,28 @@ def test_splitk_on_rows_that_the_reduce_cannot_take(L, M, N, K, ld, shift):
         assert bool((x[M] == 7.0).all()) and bool((x[:, N:] == 7.0).all())
 
 
+@pytest.mark.parametrize("M,N,K", [(100, 1024, 1024), (1025, 4096, 4160), (4400, 3840, 5120)])
+def test_splitk_without_a_workspace(L, M, N, K):
+    """Products that are faster in K ranges but need none run in one when the caller brings no workspace: few rows, 80 tiles
+    of 256 x 256, a full round of tiles with a rest."""
+    a = abi()
+    g = torch.Generator().manual_seed(M + N + K)
+    A = torch.randn(M, K, generator=g).to(torch.float16).to(DEV)
+    Wh = (torch.randn(K, N, generator=g) * 0.05).to(torch.float16).to(DEV)
+    bias, sc, of = torch.randn(N, generator=g).to(DEV), (1 + 0.1 * torch.randn(N, generator=g)).to(DEV), (0.1 * torch.randn(N, generator=g)).to(DEV)
+    W = _packed(Wh)
+    x0 = torch.randn(M, N, generator=g).to(DEV)
+    ref = x0.double() + A.double() @ Wh.double() + bias.double()
+    assert L.mtj_gemm_splitk_work_bytes(M, N, K, a.F16) > 0
+    x, y, h = x0.clone(), x0.clone(), torch.zeros(M, N, dtype=torch.float16, device=DEV)
+    a.check(L.mtj_gemm_splitk(a.ptr(A), K, a.ptr(W), a.ptr(bias), M, N, K, a.F16, a.EPI_RESID, a.ptr(x), N, 0, None, 0, 1.0, S()))
+    a.check(L.mtj_gemm_splitk_ln(a.ptr(A), K, a.ptr(W), a.ptr(bias), M, N, K, a.F16, a.ptr(y), N, None, 0, a.ptr(sc), a.ptr(of),
+                                 a.ptr(h), N, a.F16, 1.0, S()))
+    torch.cuda.synchronize()
+    assert rel_err(x, ref) < 5e-6 and torch.equal(x, y)
+    assert rel_err(h, torch.nn.functional.layer_norm(ref, (N,), sc.double(), of.double(), 1e-5)) < 5e-4
+
+
 @pytest.mark.parametrize("M,N,K", [(1808, 4096, 2432), (3195, 2048, 2560), (100, 512, 2560), (768, 1024, 5120)])
 def test_splitk_layernorm_on_padded_rows(L, M, N, K):
     """x and h with padded rows, at a short K (128 and 104 tiles of 256 x 256 in two ranges) and at few rows: the padding
