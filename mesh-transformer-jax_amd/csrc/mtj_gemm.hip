@@ -169,13 +169,13 @@ __device__ __forceinline__ void epilogue(const gemm_args& a, void* out, ACC& acc
           }
         mx = fmaxf(mx, __shfl_xor(mx, 16));
         mx = fmaxf(mx, __shfl_xor(mx, 32));
+        // exp(-inf) = 0 for columns beyond N; without a maximum the sum is 0, or NaN if a logit is
+        const float ref = mx == -INFINITY ? 0.f : mx;
         float sm = 0.f;
-        if (mx != -INFINITY) {
 #pragma unroll
-          for (int j = 0; j < 2 * WN; ++j)
+        for (int j = 0; j < 2 * WN; ++j)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) sm += __expf(val[j][v] - mx);      // exp(-inf) = 0 for columns beyond N
-        }
+          for (int v = 0; v < 4; ++v) sm += __expf(val[j][v] - ref);
         sm += __shfl_xor(sm, 16);
         sm += __shfl_xor(sm, 32);
         if (m < a.M) {
@@ -244,8 +244,8 @@ __device__ __forceinline__ void epilogue(const gemm_args& a, void* out, ACC& acc
       float sm = 0.f;
 #pragma unroll
       for (int w = 0; w < WAVES_N; ++w) {
-        const float pm = red[(w * BM + r) * 2];
-        sm += pm == -INFINITY ? 0.f : __expf(pm - mx) * red[(w * BM + r) * 2 + 1];
+        const float pm = red[(w * BM + r) * 2], ps = red[(w * BM + r) * 2 + 1];
+        sm += pm == -INFINITY ? ps : __expf(pm - mx) * ps;     // (0 or NaN where there is no maximum)
       }
       a.pmax[(int64_t)tn * a.M + m] = mx;
       a.psum[(int64_t)tn * a.M + m] = sm;
@@ -1123,36 +1123,36 @@ __global__ __launch_bounds__(1024) void splitk_reduce_ln_kernel(const float* __r
 // loss = log(sum exp(l - max)) - (l[target] - max), correct = (l[target] == max); a target outside [0, N) selects
 // nothing (pred = 0), as in xent_kernel.
 // Eight rows per workgroup, 32 threads per row that share its column tiles (394 of 128 columns, 197 of 256 at the 6B
-// vocabulary); every thread merges its tiles as it reads them, then the 32 partial results meet in LDS.  With one thread
-// per row the chain of dependent loads over all tiles took 180 us for 244 rows and kept one workgroup busy; now 5 us.
+// vocabulary): the maximum over all tiles first, then the sum relative to it, each met in LDS.  With one thread per row the
+// chain of dependent loads over all tiles took 180 us for 244 rows and kept one workgroup busy; now 6.5 us.
+// A row without a maximum (all logits -inf or NaN) sums exp(-inf - -inf) and gives NaN.
 constexpr int XM_ROWS = 8, XM_LANES = 32;
-__device__ __forceinline__ void xent_merge(float& mx, float& sm, float pm, float ps) {
-  const float m = fmaxf(mx, pm);
-  if (m == -INFINITY) return;
-  sm = sm * __expf(mx - m) + ps * __expf(pm - m);          // exp(-inf) = 0: an empty side contributes nothing
-  mx = m;
-}
 __global__ __launch_bounds__(XM_ROWS * XM_LANES) void xent_merge_kernel(const float* __restrict__ pmax, const float* __restrict__ psum,
                                                          const float* __restrict__ tlogit, const int32_t* __restrict__ target,
                                                          int M, int N, int tiles_n, float* __restrict__ loss,
                                                          uint8_t* __restrict__ correct) {
-  __shared__ float part[XM_LANES][XM_ROWS][2];
+  __shared__ float part[XM_LANES][XM_ROWS];
   const int r = threadIdx.x % XM_ROWS, l = threadIdx.x / XM_ROWS;
   const int m = blockIdx.x * XM_ROWS + r;
+  // all 32 partial results of a row, combined in the same order by every thread
+  auto meet = [&](float v, auto combine) {
+    __syncthreads();
+    part[l][r] = v;
+    __syncthreads();
+    v = part[0][r];
+#pragma unroll
+    for (int i = 1; i < XM_LANES; ++i) v = combine(v, part[i][r]);
+    return v;
+  };
   float mx = -INFINITY, sm = 0.f;
   if (m < M)
-    for (int t = l; t < tiles_n; t += XM_LANES) xent_merge(mx, sm, pmax[(int64_t)t * M + m], psum[(int64_t)t * M + m]);
-  part[l][r][0] = mx;
-  part[l][r][1] = sm;
-#pragma unroll
-  for (int o = XM_LANES / 2; o > 0; o >>= 1) {
-    __syncthreads();
-    if (l < o) {
-      xent_merge(mx, sm, part[l + o][r][0], part[l + o][r][1]);
-      part[l][r][0] = mx;
-      part[l][r][1] = sm;
-    }
-  }
+#pragma unroll 8
+    for (int t = l; t < tiles_n; t += XM_LANES) mx = fmaxf(mx, pmax[(int64_t)t * M + m]);
+  mx = meet(mx, [](float a, float b) { return fmaxf(a, b); });
+  if (m < M)
+#pragma unroll 8
+    for (int t = l; t < tiles_n; t += XM_LANES) sm += __expf(pmax[(int64_t)t * M + m] - mx) * psum[(int64_t)t * M + m];
+  sm = meet(sm, [](float a, float b) { return a + b; });
   if (l > 0 || m >= M) return;
   const int tg = target[m];
   const float pred = ((uint32_t)tg < (uint32_t)N) ? tlogit[m] - mx : 0.f;

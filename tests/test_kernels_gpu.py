@@ -1211,6 +1211,54 @@ def test_logits_and_cross_entropy_in_one_gemm(L, dt, M, V, K):
                                 a.ptr(ok1), a.ptr(work), nb - 4, S()))
 
 
+@pytest.mark.parametrize("dt,M,V", [("f32", 5, 700), ("f32", 48, 700), ("f32", 200, 700), ("f16", 5, 700), ("f16", 48, 700),
+                                    ("bf16", 100, 700), ("f16", 200, 700), ("f16", 200, 16500), ("bf16", 600, 16500)])
+def test_cross_entropy_of_logits_that_are_not_finite(L, dt, M, V):
+    """NaN, -inf and +inf among the logits, by column tile and by row, in every tile of the fused projection: the loss is
+    what log(sum exp(l - max)) - (l[target] - max) gives, NaN where that is NaN, whatever the target is."""
+    a = abi()
+    g = torch.Generator().manual_seed(M + V)
+    K = 64
+    A0 = torch.randn(M, K, generator=g).to(TD[dt]).to(DEV)
+    Wh0 = (torch.randn(K, V, generator=g) * 0.2).to(TD[dt]).to(DEV)
+    b0 = torch.randn(V, generator=g).to(DEV)
+    tgt = torch.randint(0, V, (M,), generator=g).to(torch.int32).to(DEV)
+    tgt[::3] = V + 5
+    tgt[1] = 300                                          # inside the block below
+    code, inf = a.dtype_code(TD[dt]), float("inf")
+    for what in ("nan columns", "-inf columns", "-inf everywhere", "nan rows", "+inf column", "nan and -inf columns"):
+        A, Wh, bias = A0.clone(), Wh0.clone(), b0.clone()
+        if what == "nan columns":
+            Wh[:, 256:512] = float("nan")
+        elif what == "-inf columns":
+            bias[256:512] = -inf
+        elif what == "-inf everywhere":
+            bias[:] = -inf
+        elif what == "nan rows":
+            A[::2] = float("nan")
+        elif what == "+inf column":
+            bias[300] = inf
+        else:
+            bias[:] = -inf
+            bias[256:512] = float("nan")
+        W = _packed(Wh)
+        loss, ok = torch.zeros(M, device=DEV), torch.zeros(M, dtype=torch.uint8, device=DEV)
+        nb = L.mtj_gemm_xent_work_bytes(M, V, code)
+        work = torch.zeros(nb // 4, device=DEV)
+        a.check(L.mtj_gemm_xent(a.ptr(A), K, a.ptr(W), a.ptr(bias), M, V, K, code, 1.0, a.ptr(tgt), a.ptr(loss), a.ptr(ok),
+                                a.ptr(work), nb, S()))
+        torch.cuda.synchronize()
+        l64 = A.double() @ Wh.double() + bias.double()
+        mx = l64.max(-1, keepdim=True).values
+        pred = torch.where(tgt.long() < V, l64.gather(1, tgt.long().clamp(max=V - 1)[:, None])[:, 0] - mx[:, 0], 0.0)
+        ref = torch.log(torch.exp(l64 - mx).sum(-1)) - pred
+        assert torch.equal(loss.isnan(), ref.isnan()), what
+        fin = ref.isfinite()
+        assert torch.equal(loss[~fin & ~ref.isnan()].double(), ref[~fin & ~ref.isnan()]), what      # a target of -inf: +inf
+        if bool(fin.any()):
+            assert (loss[fin].double() - ref[fin]).abs().max().item() < 2e-5 * max(1.0, ref[fin].abs().max().item()), what
+
+
 @pytest.mark.parametrize("dt,N,K,ln", [("bf16", 50400, 4096, True), ("f32", 1000, 512, False), ("f16", 50400, 1024, True),
                                        ("bf16", 70, 64, False), ("bf16", 4100, 4096, True)])
 def test_logits_launch_that_is_its_own_greedy_sampler(L, dt, N, K, ln):
