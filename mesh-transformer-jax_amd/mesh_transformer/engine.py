@@ -252,15 +252,15 @@ class Engine:
         ip.rows = ptr(rows)
         return ip
 
-    def prefill(self, ses, tokens, Tp, key_limit=None, packed=None):
+    def prefill(self, ses, tokens_rect, Tp, key_limit=None, packed=None):
         """generate_initial (transformer_shard.py:74-95) on a [B, Tp] right-aligned rectangle; the
         dead logits projection of :95 is not computed.  packed: (rows [M], skipped [B]) as mtj_inproj and
-        mtj_attn_prefill_packed take them, when `tokens` [M] and the rows returned are those of real tokens only."""
+        mtj_attn_prefill_packed take them, when `tokens_rect` [M] and the rows returned are those of real tokens only."""
         L, w, s = _abi.lib(), self.w, _abi.stream_handle()
         d = w.d
-        M = tokens.numel()
+        M = ses.B * Tp if packed is None else packed[0].numel()       # (the token buffer may be longer)
         x, h, act = ses.x_pf[:M], ses.h_pf[:M], ses.act_pf[:M]
-        check(L.mtj_embed(ptr(tokens), M, ptr(w.we), ptr(w.be), w.V, d, w.dtype, ptr(x), s))
+        check(L.mtj_embed(ptr(tokens_rect), M, ptr(w.we), ptr(w.be), w.V, d, w.dtype, ptr(x), s))
         # as in batched decode: the launch that completes a layer's residual rows also normalises them for the next layer
         ids = w.layer_ids
         for j, i in enumerate(ids):

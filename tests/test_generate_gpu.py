@@ -180,6 +180,22 @@ def test_forward_logits_every_position():
         net.forward(toks, [70, 71])
 
 
+def test_prefill_reads_its_rectangle_from_a_longer_buffer():
+    """Engine.prefill takes the first B * Tp tokens of the buffer it is given: a program that keeps one buffer for its
+    longest prompt passes it for every shorter one.  Same rows as from a buffer of the right size."""
+    from mesh_transformer.sampling import greedy_sample
+    net = net_for(CFG1, O.seeded_params(CFG1, 0), greedy_sample)
+    eng = net.engine()
+    B, Tp = 2, 37
+    ses = eng.session(B, Tp, Tp, Tp + 1)
+    ses.pos0.zero_()
+    buf = torch.from_numpy(np.random.default_rng(5).integers(0, 50257, B * Tp + 61).astype(np.int32)).to(DEV)
+    want = eng.prefill(ses, buf[:B * Tp].view(B, Tp).contiguous(), Tp).clone()
+    got = eng.prefill(ses, tokens_rect=buf, Tp=Tp)
+    torch.cuda.synchronize()
+    assert got.shape == (B * Tp, CFG1["d_model"]) and torch.equal(got, want)
+
+
 def test_config1_against_the_committed_fixture():
     """BASELINE config 1 against tests/golden/config1_greedy.npz: tokens identical, top-8 logits of every step
     within 1e-4 relative, logit checksums."""
