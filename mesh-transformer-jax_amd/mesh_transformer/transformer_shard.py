@@ -161,8 +161,8 @@ class CausalTransformer:
         Beyond the reference: `uniforms` float64 [B, G] in [0, 1) drive the inverse-CDF draw (default:
         drawn from an unseeded Philox stream, like the reference's unseeded key at :327);
         `sampler` overrides config["sampler"]; `timing`, a dict with key "warmup" (decode steps left out of
-        the timed region), is filled with device-synchronised wall times: prefill_s, warmup_s, decode_s,
-        decode_steps."""
+        the timed region), is filled with device-synchronised wall times: prefill_s, warmup_s, decode_s, and with
+        prefill_tokens (the tokens of prefill without padding) and decode_steps."""
         eng = self.engine()
         self.gen_length, self.return_logits = gen_length, return_logits
         ctx = np.ascontiguousarray(np.asarray(ctx)).astype(np.int64)
@@ -250,7 +250,7 @@ class CausalTransformer:
                 t2 = clock()
                 self._decode(eng, ses, W, G, kind, logits_out, masks)
                 t3 = clock()
-                timing.update(prefill_s=t1 - t0, prefill_tokens=B * Tp, warmup_s=t2 - t1, decode_s=t3 - t2,
+                timing.update(prefill_s=t1 - t0, prefill_tokens=int((P - 1).sum()), warmup_s=t2 - t1, decode_s=t3 - t2,
                               decode_steps=G - W)
             logits_np = None
             if return_logits:

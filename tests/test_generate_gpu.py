@@ -150,6 +150,17 @@ def test_batched_ragged_nucleus_bit_exact_given_logits():
     assert np.array_equal(out2[0], toks)
 
 
+@pytest.mark.parametrize("length,tokens", [([40, 40], 78), ([40, 7, 1], 45), ([1, 1], 0)])
+def test_timing_counts_the_prompt_tokens_that_are_computed(length, tokens):
+    """timing["prefill_tokens"] leaves the padding of unequal prompts out, which no layer sees."""
+    from mesh_transformer.sampling import greedy_sample
+    net = net_for(CFG1, O.seeded_params(CFG1, 0), greedy_sample)
+    ctx = np.concatenate([O.left_pad(O.seeded_prompt(b, 1, n), 60) for b, n in enumerate(length)])
+    timing = {"warmup": 1}
+    net.generate(ctx, np.array(length), 4, {}, timing=timing)
+    assert timing["prefill_tokens"] == tokens and timing["decode_steps"] == 3 and timing["prefill_s"] >= 0
+
+
 def test_forward_logits_every_position():
     """CausalTransformer.forward (embed -> layers -> projection at every position) against the oracle's full
     forward: fp32 within 1e-4 relative; left padding leaves the real rows unchanged and zeroes the padded ones;
