@@ -1242,13 +1242,12 @@ __global__ __launch_bounds__(DH / 4) void attn_combine_kernel(const float* __res
 }
 
 // key ranges per (sequence, head): about one workgroup per CU when the batch alone does not fill the chip; a range
-// never starts out shorter than 16 keys at the full window
+// never starts out shorter than 16 keys at the full window.  Four ranges where this gives two help sequences of very unequal
+// length (8 x 16 heads of 256 x 80 .. 640 keys 17.9 -> 16.3 us, 250 .. 2000 40.8 -> 35.5), leave long equal ones as they are
+// (2000 keys 51.7 -> 49.6) and cost every short window of up to one workgroup step per range: 64 keys 7.8 -> 8.8 us, d_head
+// 64 up to 300 keys 8.1 -> 9.0.
 int decode_splits(int64_t B, int64_t H, int64_t Tcap) {
   int64_t S = 256 / (B * H);
-  // two ranges per sequence become four: with sequences of unequal length the workgroups of the short ones leave early
-  // (8 x 16 heads x 80 .. 640 keys, with the merge: 18.0 -> 15.3 us; all 600 keys 19.4 -> 19.4, all 1900 45.5 -> 45.2).
-  // Twice as many elsewhere costs more: 3 sequences of 32 .. 97 keys 7.3 -> 8.3, 12 of 700 (one range, no merge) 27.3 -> 30.8
-  if (B > 1 && S == 2) S = 4;
   if (S > (Tcap + 15) / 16) S = (Tcap + 15) / 16;
   if (S > MTJ_DEC_MAXS) S = MTJ_DEC_MAXS;
   if (S < 1) S = 1;

@@ -869,11 +869,10 @@ def test_attn_decode_window(L, dt, dh, H, Tcap, positions):
 
 @pytest.mark.parametrize("dt", ["f32", "f16"])
 @pytest.mark.parametrize("dh,H,Tcap,positions,ranges", [
-    (256, 16, 700, [0, 1, 2, 63, 64, 650, 699, 900], 4), (64, 16, 300, [5, 40, 299, 130, 77, 3], 4),     # 128, 96 pairs
-    (256, 16, 40, [39, 0, 7, 8, 9, 20, 15, 16], 3), (256, 16, 60, [1, 50, 59, 3, 8], 3)])               # few slots; 80 pairs
-def test_attn_decode_four_ranges_per_sequence(L, dt, dh, H, Tcap, positions, ranges):
-    """A batch for which two key ranges per (sequence, head) would fill the chip is cut into four: ranges without any
-    key, windows too short for four."""
+    (256, 16, 700, [0, 1, 2, 63, 64, 650, 699, 900], 2), (64, 16, 300, [5, 40, 299, 130, 77, 3], 2),     # 128, 96 pairs
+    (256, 16, 40, [39, 0, 7, 8, 9, 20, 15, 16], 2), (256, 16, 60, [1, 50, 59, 3, 8], 3)])               # 128, 80 pairs
+def test_attn_decode_key_ranges_of_a_batch(L, dt, dh, H, Tcap, positions, ranges):
+    """A batch of 5 to 8 sequences is cut into two or three key ranges per (sequence, head), some without any key."""
     assert L.mtj_attn_decode_splits(len(positions), H, Tcap) == ranges
     test_attn_decode_window(L, dt, dh, H, Tcap, positions)
 
