@@ -316,6 +316,32 @@ def test_splitk_without_a_workspace(L, M, N, K):
     assert rel_err(h, torch.nn.functional.layer_norm(ref, (N,), sc.double(), of.double(), 1e-5)) < 5e-4
 
 
+@pytest.mark.parametrize("N", [4, 252, 256, 260, 1020, 3844, 4092, 4096, 4100, 8200, 16384])
+def test_reduce_with_layernorm_at_every_row_length(L, N):
+    """The reduce that normalises takes a thread per four columns up to 4096 columns and 1024 threads beyond: row lengths
+    at the edges of a wavefront and of the workgroup, float32 operands (x to the float32 accumulation, h to the LayerNorm)."""
+    a = abi()
+    M, K = 5, 512
+    g = torch.Generator().manual_seed(N)
+    A = torch.randn(M, K, generator=g).to(DEV)
+    Wh = (torch.randn(K, N, generator=g) * 0.05).to(DEV)
+    bias, sc, of = torch.randn(N, generator=g).to(DEV), (1 + 0.1 * torch.randn(N, generator=g)).to(DEV), (0.1 * torch.randn(N, generator=g)).to(DEV)
+    W = _packed(Wh)
+    x = torch.full((M + 1, N), 7.0, device=DEV)
+    x[:M] = torch.randn(M, N, generator=g).to(DEV)
+    h = torch.full((M + 1, N), 7.0, device=DEV)
+    ref = x[:M].double() + A.double() @ Wh.double() + bias.double()
+    nb = L.mtj_gemm_splitk_work_bytes(M, N, K, a.F32)
+    assert nb >= 2 * M * N * 4                                 # a product in K ranges, so the reduce runs
+    work = torch.empty(nb, dtype=torch.uint8, device=DEV)
+    a.check(L.mtj_gemm_splitk_ln(a.ptr(A), K, a.ptr(W), a.ptr(bias), M, N, K, a.F32, a.ptr(x), N, a.ptr(work), nb,
+                                 a.ptr(sc), a.ptr(of), a.ptr(h), N, a.F32, 1.0, S()))
+    torch.cuda.synchronize()
+    assert rel_err(x[:M], ref) < 2e-6 and bool((x[M] == 7.0).all())
+    want = torch.nn.functional.layer_norm(ref, (N,), sc.double(), of.double(), 1e-5)
+    assert rel_err(h[:M], want) < 1e-5 and bool((h[M] == 7.0).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(1808, 4096, 2432), (3195, 2048, 2560), (100, 512, 2560), (768, 1024, 5120)])
 def test_splitk_layernorm_on_padded_rows(L, M, N, K):
     """x and h with padded rows, at a short K (128 and 104 tiles of 256 x 256 in two ranges) and at few rows: the padding
