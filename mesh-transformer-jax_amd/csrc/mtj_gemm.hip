@@ -971,7 +971,13 @@ int launch(const gemm_args& a, hipStream_t s) {
 
 // 256 x 256 tiles of gemm_dma_kernel, one workgroup per CU, from this many of them on: N = 4096, K = 20480 in one K range,
 // 144 tiles 486 us (602 with 128 x 128 tiles), 192 tiles 458 (650); 96 tiles 455 against 384 for two ranges of 128 x 128.
+// So are 144 .. 196 tiles with the other epilogues, us against 128 x 128 tiles, at every K from 256 on: STORE 144 tiles 19 (33) at
+// K = 256, 31 (53) at 1024, 49 (80) at 2048; XENT the same; the fused input projection 61 (70) for 513 rows of d_model 2048, 43
+// (49) for 1536 of 1024, 36.4 (37.5) for 1742 of 768.  Its epilogue is long, so with fewer than 12 k-tiles in front of it several
+// small workgroups per CU hide it better: d_model 512, 2766 / 3022 / 3278 rows (154 / 168 / 182 tiles) 32 - 33 us (28 - 30),
+// 3534 rows (196) 33 (34); that epilogue keeps a line of 200 tiles there.
 constexpr int64_t DMA_MIN_TILES = 144;
+constexpr int64_t DMA_MIN_TILES_SHORT_INPROJ = 200;
 int64_t dma_tiles(int64_t M, int64_t N) { return ((M + 255) / 256) * ((N + 255) / 256); }
 
 template <typename T, int EPI, int BK>
@@ -992,7 +998,8 @@ int dispatch_tile(const gemm_args& a, hipStream_t s) {
   }
   if constexpr (sizeof(T) == 2) {
     // e.g. M = 16384, N = 28672 or N = 4096 (a whole 6B layer at 8 x 2048 tokens): 7168 / 1024 tiles
-    if (dma_tiles(a.M, a.N) * a.splits >= DMA_MIN_TILES) return launch_dma<T, EPI>(a, s);   // 256 x 256, 8 wavefronts of 128 x 64
+    const int64_t line = EPI == MTJ_EPI_INPROJ && a.K < 768 ? DMA_MIN_TILES_SHORT_INPROJ : DMA_MIN_TILES;
+    if (dma_tiles(a.M, a.N) * a.splits >= line) return launch_dma<T, EPI>(a, s);        // 256 x 256, 8 wavefronts of 128 x 64
   }
   return launch<T, EPI, 2, 2, 2, 2, BK, 2>(a, s);                   // 128 x 128
 }

@@ -515,10 +515,17 @@ def test_inproj_gemm_prefill_with_left_padding(dt, shape):
 
 
 def test_inproj_gemm_on_the_256x256_direct_to_lds_kernel():
-    """M = 1024 rows x N = 14336 columns is 4 x 56 = 224 tiles of 256 x 256: mtj_gemm dispatches gemm_dma_kernel (at
-    least 200 such tiles), whose 8-wavefront epilogue (RoPE, K/V ring, V^T, GELU) the small shapes never reach."""
+    """M = 1024 rows x N = 14336 columns is 4 x 56 = 224 tiles of 256 x 256: mtj_gemm dispatches gemm_dma_kernel (from 144
+    such tiles on), whose 8-wavefront epilogue (RoPE, K/V ring, V^T, GELU) the small shapes never reach."""
     cfg = dict(layers=1, d_model=2048, n_heads=8, n_vocab=64, pe="rotary", pe_rotary_dims=64, cores_per_replica=1)
     _run_inproj_prefill(cfg, _layer_params(cfg, 9, "bf16"), "bf16", B=2, Tp=512, Tcap=600, pads=[0, 37], seed=10)
+
+
+@pytest.mark.parametrize("d,heads,Tp", [(512, 8, 1383), (512, 2, 1767), (768, 3, 871)])
+def test_inproj_gemm_where_its_tiles_change(d, heads, Tp):
+    """154 and 196 tiles of 256 x 256 with 8 k-tiles keep the 128 x 128 tiles, 147 with 12 take the large ones."""
+    cfg = dict(layers=1, d_model=d, n_heads=heads, n_vocab=64, pe="rotary", pe_rotary_dims=64, cores_per_replica=1)
+    _run_inproj_prefill(cfg, _layer_params(cfg, 9, "bf16"), "bf16", B=2, Tp=Tp, Tcap=Tp + 3, pads=[0, 37], seed=10)
 
 
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
