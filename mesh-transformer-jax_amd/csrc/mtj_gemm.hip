@@ -1176,9 +1176,13 @@ int xent_tile_n(int64_t M, int64_t N, int dtype) {
   return 128;
 }
 
-// Time of `tiles` 256 x 256 tiles in s K ranges each, in tenths of the time of one k-tile (1.4 us): rounds of 256
-// workgroups, each walking kt / s k-tiles, and the partials, 0.17 us per tile and range written and read back (N = 4096,
-// K = 20480, 256 tiles: 545 / 575 / 646 / 815 us in 1 / 2 / 4 / 8 ranges).
+// Time of `tiles` 256 x 256 tiles in s K ranges each, in tenths of the time of one k-tile: rounds of 256 workgroups, each
+// walking kt / s k-tiles, and 1.2 tenths for every partial tile that is written and read back.  Measured: a k-tile takes
+// 1.3 .. 1.7 us once 100 .. 256 workgroups run, and 256 tiles of N = 4096, K = 20480 in 1 / 2 / 4 / 8 ranges take 545 / 575 /
+// 646 / 815 us, 0.06 / 0.10 / 0.13 us per partial tile.  The weight lies above that (0.16 .. 0.2 us) because a range more also
+// costs workspace: with 0.9 tenths 192 tiles get 4 ranges and 180 MiB instead of one range, 452 us against 461, and over 178
+// products of N = 512 .. 4096 the choices are 0.6 % faster on average, single ones up to 10 % slower (7552 rows of N = 512,
+// K = 4096 55 -> 60 us) or faster (1000 rows of N = 2048, K = 10240, 8 ranges instead of 7: 64.7 -> 61.0).
 int64_t dma_cost(int64_t tiles, int64_t kt, int64_t s) {
   return (tiles * s + 255) / 256 * ((kt + s - 1) / s) * 10 + (s > 1 ? tiles * s * 6 / 5 : 0);
 }
@@ -1216,7 +1220,8 @@ cut_t pick_cut(int64_t M, int64_t N, int64_t K, int dtype) {
       // a problem of its own, if that costs less (its second launch and the separate LayerNorm of the front rows: 5 us).
       // With the reduce and the following LayerNorm: 4097 rows 1034 -> 590 us, 4900 1024 -> 719, 5632 1029 -> 841, 6500
       // 1024 -> 947 (7000 stays at 1021), 8200 1573 -> 1125, 9000 1552 -> 1255.
-      // Only 2, 3, 4, 8 or 16 ranges: 5 would save another 15 us at 48 tiles, and need more workspace than a short prompt.
+      // Only 2, 3, 4, 8 or 16 ranges: 5 would save another 15 us at 48 tiles for more workspace.  (The most that any row count
+      // needs at N = 4096, K = 20480 is 120 MiB, three ranges of 160 tiles above; powers of two alone needed 64.)
       const int64_t cols = (N + 255) / 256, rounds = tiles / 256;
       const int64_t front = rounds * 256 / cols * 256;
       if (front > 0 && M - front > 0) {
