@@ -987,6 +987,13 @@ int dispatch_tile(const gemm_args& a, hipStream_t s) {
     // 38.4 / 39.2 us for the input projection, 66.7 / 67.9 for 50400 logits (two rounds of one workgroup per CU); with K
     // ranges (the out projection) the stream kernel's deeper queue wins, 32.8 against 34.5 us.
     if (a.M <= 32 && a.splits == 1) return launch<T, EPI, 1, 4, 1, 1, BK, 2>(a, s);
+    // 33 .. 64 rows of more than one round of column tiles with a short K: 64 x 128 tiles of the same kernel, two or three
+    // workgroups per CU against one.  50400 columns, 33 / 48 / 64 rows: K = 512 16.8 / 18.6 / 19.4 us (stream kernel 18.2 / 18.8 /
+    // 19.3), K = 1024 26.7 / 28.8 / 31.1 (28.6 / 29.1 / 29.8), K = 2048 46.5 / 48.0 / 52.0 (48.6 / 51.9 / 52.6); at K = 4096, 81.1 /
+    // 86.4 / 89.8 (83.8 / 85.6 / 88.9), and with one round, 16384 columns at K = 1024, 16.5 / 17.8 / 17.7 (13.7 / 15.0 / 13.4)
+    // the stream kernel's queue is the better one.  So it is for XENT (K = 512, with the merge 24 us against 32).
+    if constexpr (EPI != MTJ_EPI_XENT)
+      if (a.M <= 64 && a.splits == 1 && a.K < 4096 && (a.N + 127) / 128 > 256) return launch<T, EPI, 1, 4, 2, 1, BK, 2>(a, s);
     if (a.M <= 64) return launch_stream<T, EPI, 64, 4>(a, s);
     // 129 .. 256 rows: one row tile while that fills more than half of the chip, else two (at d_model 2048, 112 column
     // tiles, M = 256: 28 us in two row tiles, 38 in one; at d_model 4096 the second one would only read the weights again)

@@ -611,6 +611,13 @@ def test_few_rows_stream_kernel_tile_edges(L, M, N, K):
         assert rel_err(x, x0.double() + ref) < 5e-6
 
 
+@pytest.mark.parametrize("M", [33, 64])
+@pytest.mark.parametrize("N,K", [(32768, 192), (32772, 192), (32772, 4096)])
+def test_few_rows_of_more_than_one_round_of_columns(L, M, N, K):
+    """33 .. 64 rows on either side of 256 column tiles and of the K from which the stream kernel takes the wide ones too."""
+    test_few_rows_stream_kernel_tile_edges(L, M, N, K)
+
+
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
 def test_inproj_gemv_decode_appends_to_ring(dt):
     from mesh_transformer.engine import Engine
