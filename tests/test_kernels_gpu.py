@@ -1169,6 +1169,20 @@ def test_nucleus_bucket_sizes(L, n):
     _check_rows(L, logits, np.full(R, 0.9), temp, np.array([max(1, n // 2)] * R, np.int32), rng.random(R))
 
 
+@pytest.mark.parametrize("V", [1, 1023, 1025, 10239, 10240, 10241, 20481, 51200, 51201, 61441])
+def test_nucleus_vocabulary_edges_and_small_temperatures(L, V):
+    """Vocabularies on either side of the groups of tokens that a pass leaves out, and temperatures down to those that are
+    divided by token by token, with and without top_k."""
+    rng = np.random.default_rng(V)
+    temp = np.array([1e-7, 1e-100, 1e-200, 9e-201, 0.8, 1e-6])
+    R = len(temp)
+    logits = (rng.standard_normal((R, V)) * 2).astype(np.float32)
+    logits[:, -1] = logits.max(-1)                            # the last token shares the maximum
+    for u in (rng.random(R), np.full(R, 0.999)):
+        _check_rows(L, logits, rng.uniform(0.05, 0.99, R), temp, None, u)
+        _check_rows(L, logits, np.full(R, 0.9), temp, np.array([1, 2, 3, 4, 5, 40], np.int32), u)
+
+
 def test_nucleus_against_the_committed_fixture(L):
     """tests/golden/nucleus_cases.npz: keep-masks and tokens bit for bit."""
     import os
