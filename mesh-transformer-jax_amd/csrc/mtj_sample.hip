@@ -535,10 +535,10 @@ __global__ __launch_bounds__(SNT) void nucleus_kernel(const float* __restrict__ 
   // In the usual case a token the filter touched has no weight at all (its filtered / temp is 1e10 / temp lower,
   // far below the 2^-62 that still counts) and needs no arithmetic; token 0 is exempt from the top-k penalty, which
   // multiplies by the token id.
-  const bool plain = tmp >= 1e-6 && tmp <= 1e6 && kk >= 1 && fabsf(l0) <= 1e6f;
+  const bool plain = tmp >= 1e-200 && tmp <= 1e6 && kk >= 1 && fabsf(l0) <= 1e6f;
   // x / temp with one correctly rounded reciprocal for the row and one correction per token: the correctly rounded
-  // quotient (Markstein 1990; nothing overflows or is subnormal here), so the row maximum still gives 0 exactly.  A logit
-  // of -inf gives NaN, which has no weight either.
+  // quotient (Markstein 1990; a float32 logit over at least 1e-200 does not overflow, and nothing is subnormal), so the
+  // row maximum still gives 0 exactly.  A logit of -inf gives NaN, which has no weight either.
   const double inv_tmp = 1.0 / tmp;
   auto over_temp = [&](double x) {
     const double r = x * inv_tmp;
