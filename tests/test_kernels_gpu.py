@@ -1223,11 +1223,16 @@ def test_xent_rows(L, M, V, ld):
 
 @pytest.mark.parametrize("dt,M,V,K", [("f32", 37, 50400, 256), ("bf16", 37, 50400, 512), ("f16", 64, 1000, 256),
                                       ("f32", 200, 1000, 256), ("bf16", 300, 5000, 128), ("f16", 1, 132, 64),
-                                      ("bf16", 2048, 50400, 1024), ("f16", 2000, 50400, 512)])
+                                      ("bf16", 2048, 50400, 1024), ("f16", 2000, 50400, 512), ("f16", 65, 1000, 128),
+                                      ("bf16", 129, 5000, 192), ("f16", 244, 50400, 256), ("bf16", 256, 16500, 64),
+                                      ("f16", 257, 50400, 128), ("f16", 512, 16500, 128), ("bf16", 513, 16500, 128)])
 def test_logits_and_cross_entropy_in_one_gemm(L, dt, M, V, K):
-    """mtj_gemm_xent against mtj_gemm (STORE) + mtj_xent on the same operands and against float64; the last two shapes
-    are 8 x 197 tiles of 256 x 256 (the direct-to-LDS kernel, ragged in both directions), the others the 32-, 64- and
-    128-row tiles.  Targets include the row's best column, a column in the ragged last tile and one outside the vocabulary."""
+    """mtj_gemm_xent against mtj_gemm (STORE) + mtj_xent on the same operands and against float64.  In 16 bits: 1 row is the
+    32 x 128 tile, 37 and 64 rows the few-row kernel's 64-row tile, 65 its 128-row tile and 129 two of them, 244 and 256
+    rows (more than 128 column tiles) its 256-row tile; 300 x 5000 and 512 x 16500 are 128 x 128 tiles; 257 x 50400, 513 x
+    16500 (195 tiles) and the two long ones the direct-to-LDS kernel, whose column tiles are 256 wide; float32 has the
+    64 x 128 and 128 x 128 tiles.  Targets include the row's best column, a column in the ragged last tile and one
+    outside the vocabulary."""
     a = abi()
     g = torch.Generator().manual_seed(M + V + K)
     A = torch.randn(M, K, generator=g).to(TD[dt]).to(DEV)
