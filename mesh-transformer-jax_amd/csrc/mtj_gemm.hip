@@ -805,8 +805,10 @@ __global__ __launch_bounds__(512) void gemm_dma_kernel(const gemm_args a) {
 // its reduce; weights of six layers in rotation) against the register-staged tiles this replaced: M = 64 40.3 / 37.1 us
 // (43.2 / 42.2 with 64 x 128 tiles), M = 128 51 / 45 (62 / 58), M = 256 70 / 57 (93 / 82, 128 x 128 tiles); M = 32 with K
 // ranges 34.1 (37.2).  The loads alone take 48 (M = 128) and 60 us (M = 256) for the input projection, the MFMAs and
-// fragment reads alone 23 and 43: what is left is the path into LDS (235 MB of weights plus 2 MB of activations per
-// workgroup, 12.6 TB/s), and neither more stages nor another walk over k changes it.
+// fragment reads alone 23 and 43.  Counters at 61 / 128 / 244 rows (40 / 49 / 64 us with a plain store): every weight comes from
+// memory once (5.9 / 5.0 / 3.9 TB/s), 347 / 470 / 683 MB go through L2 into LDS (8.6 / 9.6 / 10.6 TB/s), the matrix units of the
+// CUs in use are busy 16 / 28 / 45 % of the time, no bank conflicts: few rows are bound by the weight stream, many by the
+// path into LDS, and neither more stages nor another walk over k changes it.
 template <typename T, int EPI, int BM, int S>
 __global__ __launch_bounds__(512) void gemm_stream_kernel(const gemm_args a) {
   static_assert(sizeof(T) == 2, "16-bit operands");
