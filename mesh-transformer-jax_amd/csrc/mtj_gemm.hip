@@ -1021,6 +1021,34 @@ int dispatch(const gemm_args& a, int epi, hipStream_t s) {
   return dispatch_tile<T, MTJ_EPI_INPROJ, BK>(a, s);
 }
 
+// p[0] + p[stride] + .. + p[(splits - 1) * stride] in this order, four columns.  The loads of up to eight partials are all
+// issued before the first is added: a loop that asks for one partial per turn pays the latency of memory `splits` times,
+// which for a few rows is most of the launch (product, eight ranges and reduce with LayerNorm, N = 4096, K = 20480: 3 rows
+// 36.7 -> 34.7 us, 244 rows 63.5 -> 61.7; 40 rows of N = 1024, K = 5120 15.0 -> 11.7).
+template <int C> __device__ __forceinline__ void add_partials(floatx4& acc, const float* __restrict__ p, int64_t stride) {
+  floatx4 t[C];
+#pragma unroll
+  for (int i = 0; i < C; ++i) t[i] = *reinterpret_cast<const floatx4*>(p + i * stride);
+#pragma unroll
+  for (int i = 0; i < C; ++i) { acc.x += t[i].x; acc.y += t[i].y; acc.z += t[i].z; acc.w += t[i].w; }
+}
+__device__ __forceinline__ floatx4 sum_partials(const float* __restrict__ p, int splits, int64_t stride) {
+  floatx4 acc = *reinterpret_cast<const floatx4*>(p);
+  p += stride;
+  int left = splits - 1;
+  for (; left > 7; left -= 8, p += 8 * stride) add_partials<8>(acc, p, stride);
+  switch (left) {
+    case 7: add_partials<7>(acc, p, stride); break;
+    case 6: add_partials<6>(acc, p, stride); break;
+    case 5: add_partials<5>(acc, p, stride); break;
+    case 4: add_partials<4>(acc, p, stride); break;
+    case 3: add_partials<3>(acc, p, stride); break;
+    case 2: add_partials<2>(acc, p, stride); break;
+    case 1: add_partials<1>(acc, p, stride); break;
+  }
+  return acc;
+}
+
 // sums the per-split partial tiles in a fixed order and applies the epilogue (four columns per thread)
 template <int EPI>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ work, int splits, int64_t split_stride,
@@ -1030,11 +1058,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   const int nq = N / 4;
   if (q >= (int64_t)M * nq) return;
   const int m = (int)(q / nq), n = (int)(q - (int64_t)m * nq) * 4;
-  floatx4 acc = *reinterpret_cast<const floatx4*>(work + (int64_t)m * N + n);
-  for (int sp = 1; sp < splits; ++sp) {
-    const floatx4 p = *reinterpret_cast<const floatx4*>(work + sp * split_stride + (int64_t)m * N + n);
-    acc.x += p.x; acc.y += p.y; acc.z += p.z; acc.w += p.w;
-  }
+  floatx4 acc = sum_partials(work + (int64_t)m * N + n, splits, split_stride);
   if (bias) {
     const floatx4 b = *reinterpret_cast<const floatx4*>(bias + n);
     acc.x += b.x; acc.y += b.y; acc.z += b.z; acc.w += b.w;
@@ -1071,24 +1095,22 @@ __global__ __launch_bounds__(1024) void splitk_reduce_ln_kernel(const float* __r
   __shared__ float red[2][16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int m = blockIdx.x, nq = N / 4, NT = blockDim.x, NW = NT / 64;
-  floatx4 v[RLN_Q];
+  floatx4 v[RLN_Q], sc, of;
   float sum = 0.f;
 #pragma unroll
   for (int i = 0; i < RLN_Q; ++i) {
     const int q = i * NT + tid;
     if (q < nq) {
       const int n = q * 4;
-      floatx4 acc = *reinterpret_cast<const floatx4*>(work + (int64_t)m * N + n);
-      for (int sp = 1; sp < splits; ++sp) {
-        const floatx4 p = *reinterpret_cast<const floatx4*>(work + sp * split_stride + (int64_t)m * N + n);
-        acc.x += p.x; acc.y += p.y; acc.z += p.z; acc.w += p.w;
-      }
-      if (bias) {
-        const floatx4 b = *reinterpret_cast<const floatx4*>(bias + n);
-        acc.x += b.x; acc.y += b.y; acc.z += b.z; acc.w += b.w;
-      }
       float* o = x + (int64_t)m * ldx + n;
       const floatx4 old = *reinterpret_cast<const floatx4*>(o);
+      const floatx4 b = bias ? *reinterpret_cast<const floatx4*>(bias + n) : floatx4{0.f, 0.f, 0.f, 0.f};
+      if (i == 0) {                            // needed last, asked for with everything else
+        sc = *reinterpret_cast<const floatx4*>(ln_scale + n);
+        of = *reinterpret_cast<const floatx4*>(ln_offset + n);
+      }
+      floatx4 acc = sum_partials(work + (int64_t)m * N + n, splits, split_stride);
+      if (bias) { acc.x += b.x; acc.y += b.y; acc.z += b.z; acc.w += b.w; }
       // the same two roundings per element as "o[j] += acc.j" of the plain reduce
       acc.x = old.x + acc.x; acc.y = old.y + acc.y; acc.z = old.z + acc.z; acc.w = old.w + acc.w;
       *reinterpret_cast<floatx4*>(o) = acc;
@@ -1121,8 +1143,10 @@ __global__ __launch_bounds__(1024) void splitk_reduce_ln_kernel(const float* __r
     const int q = i * NT + tid;
     if (q < nq) {
       const int n = q * 4;
-      const floatx4 sc = *reinterpret_cast<const floatx4*>(ln_scale + n);
-      const floatx4 of = *reinterpret_cast<const floatx4*>(ln_offset + n);
+      if (i > 0) {
+        sc = *reinterpret_cast<const floatx4*>(ln_scale + n);
+        of = *reinterpret_cast<const floatx4*>(ln_offset + n);
+      }
       const floatx4 y = (sc * inv) * (v[i] - mean) + of;
       if (h_dtype == MTJ_F32) {
         *reinterpret_cast<floatx4*>(reinterpret_cast<float*>(h) + (int64_t)m * ldh + n) = y;
