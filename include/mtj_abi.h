@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define MTJ_ABI_VERSION 5
+#define MTJ_ABI_VERSION 6
 
 enum { MTJ_F32 = 0, MTJ_BF16 = 1, MTJ_F16 = 2 };
 
@@ -245,6 +245,16 @@ int64_t mtj_attn_decode_work_bytes(int64_t B, int64_t H, int64_t dh, int64_t Tca
 int mtj_attn_decode(const float* q, const void* k_cache, const void* v_cache, const int32_t* pos, int64_t B,
                     int64_t H, int64_t Tcap, int64_t dh, void* out, int64_t ld_out, int out_dtype, int dtype,
                     void* work, void* stream);
+
+/* mtj_attn_decode in one launch, for up to 64 sequences: the key ranges follow the lengths of all sequences, and the
+ * workgroup that finishes the last range of a (sequence, head) merges them.  Same arguments and results, except for
+ * `work`: 128-byte aligned, mtj_attn_decode_joined_work_bytes(B, H, dh, Tcap) bytes (0: this shape is not covered, use
+ * mtj_attn_decode), zeroed by the caller ONCE before its first use; every launch leaves its counters at zero.  Calls
+ * sharing one `work` must have the same B, H and dh and must not overlap. */
+int64_t mtj_attn_decode_joined_work_bytes(int64_t B, int64_t H, int64_t dh, int64_t Tcap);
+int mtj_attn_decode_joined(const float* q, const void* k_cache, const void* v_cache, const int32_t* pos, int64_t B,
+                           int64_t H, int64_t Tcap, int64_t dh, void* out, int64_t ld_out, int out_dtype, int dtype,
+                           void* work, void* stream);
 
 /* The partial results of mtj_attn_decode without the merge: mtj_gemv merges them while it stages its input (the
  * attention output is consumed by the out projection only, layers.py:285), which saves a launch and a round trip

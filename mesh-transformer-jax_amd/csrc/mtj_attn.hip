@@ -1104,26 +1104,101 @@ __global__ __launch_bounds__(256) void attn_prefill_q64_kernel(const T* __restri
 // result goes straight to `out`; otherwise attn_combine_kernel (or the prologue of the out-projection GEMV) merges them.
 constexpr int DEC_NI = 8;            // K (and V) loads per lane and step
 constexpr int DEC_PAD = MTJ_DEC_PAD;  // floats in front of the vector of a partial
+constexpr int DEC_RATE = 150;                    // see attn_decode_kernel
+constexpr int JOIN_NW = 8, JOIN_NI = 4;          // wavefronts, loads per lane and step
+constexpr int DEC_LINE = 32;         // floats of a 128-byte line: what two workgroups write never shares one
+constexpr int joined_stride(int dh) { return (dh + DEC_PAD + DEC_LINE - 1) / DEC_LINE * DEC_LINE; }
+__host__ __device__ constexpr int64_t joined_block(int64_t S, int64_t dh) {
+  return DEC_LINE + S * ((dh + DEC_PAD + DEC_LINE - 1) / DEC_LINE * DEC_LINE);
+}
 
-template <typename T, int DH>
-__global__ __launch_bounds__(256) void attn_decode_kernel(const float* __restrict__ q, const T* __restrict__ kc,
+// op over the values of lanes 0 .. l in lane l, for the first B lanes (op(0, x) == x): row shifts inside 16 lanes, then the
+// last lanes of the rows before
+template <class OP> __device__ __forceinline__ int lane_scan(int v, int B, OP op) {
+  v = op(__builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false), v);
+  v = op(__builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false), v);
+  v = op(__builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false), v);
+  v = op(__builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false), v);
+  const int row = (threadIdx.x & 63) >> 4;
+  for (int r = 1; r * 16 < B; ++r) {
+    const int t = __builtin_amdgcn_readlane(v, r * 16 - 1);
+    if (row == r) v = op(t, v);
+  }
+  return v;
+}
+
+// JOIN: one launch whatever the cut, and a cut that follows the lengths of all sequences.  Workgroups of 8 wavefronts (4
+// loads per lane and step, two of them per CU) take the key ranges of all (sequence, head) pairs in order, so that no
+// workgroup between them is empty - workgroups are dealt round-robin over the XCDs, and with the ranges in a grid
+// dimension of their own the short sequences' empty ones would leave XCDs idle -; the workgroup that finishes a pair's last
+// range merges them (an arrivals counter in front of the partials; no workgroup waits for another).
+// What a cut costs and gives was measured: the chip reads as fast as DEC_RATE workgroups that have it to themselves (40 - 53
+// GB/s each), and a merge takes 2 - 3 us, the time of two steps.  So nothing is cut while the longest sequence ends no
+// more than two steps after the chip could have read all keys; beyond that a range is a workgroup's share of the keys, and
+// not below two steps.  16 heads of 256, us, two equal or more ranges and a separate merge launch before: 3 x 33 .. 100
+// keys 7.3 -> 5.8, 4 x 300 10.0 -> 9.0, 8 x 64 7.5 -> 6.3, 8 x 80 .. 640 18.0 -> 14.1, 8 x 250 .. 2000 37 -> 32, 12 x 40 .. 480
+// 18.5 -> 13.7, 16 x 62 .. 1000 33.6 -> 31.2; 8 x 600 19.5 -> 20.3; one range as before, with the rule in front: 16 x 1000
+// 44.2, 32 x 500 43.6, 22 x 1 .. 36 5.6 -> 5.9.
+template <typename T, int DH, bool JOIN, int NW = 4, int NI = DEC_NI>
+__global__ __launch_bounds__(NW * 64) void attn_decode_kernel(const float* __restrict__ q, const T* __restrict__ kc,
                                                           const T* __restrict__ vc, const int32_t* __restrict__ pos,
-                                                          int H, int Tcap, float* __restrict__ work, void* __restrict__ out,
-                                                          int64_t ld_out, int out_dtype) {
+                                                          int B, int H, int Tcap, int smax, float* __restrict__ work,
+                                                          void* __restrict__ out, int64_t ld_out, int out_dtype) {
   constexpr int EPC = kvrow<T>::EPC;
   constexpr int LPK = DH / EPC;      // lanes per key row
   constexpr int KPL = 64 / LPK;      // keys per wavefront load
-  constexpr int NI = DEC_NI;
-  constexpr int STEP = 4 * NI * KPL; // keys per workgroup step
+  constexpr int STEP = NW * NI * KPL; // keys per workgroup step
   static_assert(LPK <= 64 && 64 % LPK == 0, "head dim does not map onto a wavefront");
-  __shared__ float part[4][DH];
-  __shared__ float stat[4][2];
+  __shared__ float part[NW][DH];
+  __shared__ float stat[NW][2];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z, S = gridDim.x;
+  int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+  int S = gridDim.x, nvalid;                                  // key ranges, keys
+  if constexpr (JOIN) {
+    // lane l looks at sequence l
+    int n = 0;
+    if (lane < B) {
+      const int p = pos[lane];
+      n = (p + 1 < Tcap) ? p + 1 : Tcap;
+      n = n > 0 ? n : 0;
+    }
+    const unsigned all = (unsigned)__builtin_amdgcn_readlane(lane_scan(n, B, [](int x, int y) { return x + y; }), B - 1) * (unsigned)H;
+    const unsigned longest = (unsigned)__builtin_amdgcn_readlane(lane_scan(n, B, [](int x, int y) { return x > y ? x : y; }), B - 1);
+    const unsigned grid = gridDim.x, spare = grid - (unsigned)(B * H), least = 2 * STEP;
+    auto most = [](unsigned x, unsigned y) { return x > y ? x : y; };
+    auto ranges = [&](unsigned want) {                         // of lane's sequence, of `want` keys at most
+      int c = (int)(((unsigned)n + want - 1) / want);
+      c = c < smax ? c : smax;
+      return lane >= B ? 0 : c > 1 ? c : 1;
+    };
+    int cut, end;                                              // end: ranges of sequences 0 .. l, per head
+    if (longest <= most(most(all / DEC_RATE, (all + grid - 1) / grid), least) + least) {
+      cut = lane < B ? 1 : 0;
+      end = lane + 1;
+    } else {
+      // a workgroup's share of the keys; where the rounding up leaves too few workgroups for all ranges, as many keys as
+      // never do: the sum of ceil(n / want) is at most the sum of n / want, plus one per (sequence, head)
+      cut = ranges(most((all + grid - 1) / grid, least));
+      end = lane_scan(cut, B, [](int x, int y) { return x + y; });
+      if ((unsigned)__builtin_amdgcn_readlane(end, B - 1) * (unsigned)H > grid) {
+        cut = ranges(most((all + spare - 1) / spare, least));
+        end = lane_scan(cut, B, [](int x, int y) { return x + y; });
+      }
+    }
+    const int w = blockIdx.x;                                  // the workgroups take the ranges in order
+    b = (int)__popcll(__ballot(lane < B && end * H <= w));     // (`end` grows with the lane)
+    if (b >= B) return;
+    S = __builtin_amdgcn_readlane(cut, b);
+    const int r = w - (__builtin_amdgcn_readlane(end, b) - S) * H;
+    h = (int)((unsigned)r / (unsigned)S);
+    split = r - h * S;
+    nvalid = __builtin_amdgcn_readlane(n, b);
+  } else {
+    const int p = pos[b];
+    nvalid = (p + 1 < Tcap) ? p + 1 : Tcap;
+  }
   const int64_t bh = (int64_t)b * H + h;
-  const int p = pos[b];
-  const int nvalid = (p + 1 < Tcap) ? p + 1 : Tcap;
   const int per = (nvalid + S - 1) / S;                       // keys per range
   const int k0 = split * per;
   const int nk = (k0 + per <= nvalid) ? per : nvalid - k0;     // <= 0: an empty range (fewer keys than ranges)
@@ -1141,7 +1216,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const float* __restric
     auto request = [&](int buf, int base) {
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
-        int kk = base + (i * 4 + wave) * KPL + sub;
+        int kk = base + (i * NW + wave) * KPL + sub;
         kk = kk < nk ? kk : nk - 1;
         // streaming loads: the window is read once per step and never again, and kept in the caches it only displaces
         // itself (32 sequences x 2004 keys: 155.6 us against 177.6 with ordinary loads)
@@ -1166,7 +1241,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const float* __restric
         for (int j = 0; j < EPC; ++j) d = fmaf(kf[j], qv[j], d);
 #pragma unroll
         for (int o = LPK / 2; o > 0; o >>= 1) d += __shfl_xor(d, o);
-        const int kk = base + (i * 4 + wave) * KPL + sub;
+        const int kk = base + (i * NW + wave) * KPL + sub;
         sc[i] = kk < nk ? d * scale : -INFINITY;
         mt = fmaxf(mt, sc[i]);
       }
@@ -1211,19 +1286,61 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const float* __restric
   }
   if (lane == 0) { stat[wave][0] = m_run; stat[wave][1] = l_run; }
   __syncthreads();
-  const float m0 = stat[0][0], m1 = stat[1][0], m2 = stat[2][0], m3 = stat[3][0];
-  const float mm = fmaxf(fmaxf(m0, m1), fmaxf(m2, m3));
-  const bool any = mm != -INFINITY;
-  const float f0 = any ? __expf(m0 - mm) : 0.f, f1 = any ? __expf(m1 - mm) : 0.f;
-  const float f2 = any ? __expf(m2 - mm) : 0.f, f3 = any ? __expf(m3 - mm) : 0.f;
-  const float lt = (f0 * stat[0][1] + f1 * stat[1][1]) + (f2 * stat[2][1] + f3 * stat[3][1]);
-  float* wout = work + (bh * S + split) * (DH + DEC_PAD);
-  for (int e = tid; e < DH; e += 256) {
-    const float v = (f0 * part[0][e] + f1 * part[1][e]) + (f2 * part[2][e] + f3 * part[3][e]);
-    if (S == 1 && out) store_as(out, (int64_t)b * ld_out + h * DH + e, lt > 0.f ? v / lt : 0.f, out_dtype);
-    else wout[DEC_PAD + e] = v;
+  float mm = stat[0][0], f[NW], lt = 0.f;
+#pragma unroll
+  for (int i = 1; i < NW; ++i) mm = fmaxf(mm, stat[i][0]);
+#pragma unroll
+  for (int i = 0; i < NW; ++i) f[i] = mm != -INFINITY ? __expf(stat[i][0] - mm) : 0.f;
+  // the wavefronts two by two
+  auto meet = [&](auto value) {
+    float v = 0.f;
+#pragma unroll
+    for (int i = 0; i < NW; i += 4)
+      v += (f[i] * value(i) + f[i + 1] * value(i + 1)) + (f[i + 2] * value(i + 2) + f[i + 3] * value(i + 3));
+    return v;
+  };
+  lt = meet([&](int i) { return stat[i][1]; });
+  if constexpr (JOIN) {
+    float* block = work + bh * joined_block(smax, DH);    // the arrivals counter, then the partials
+    float* wout = block + DEC_LINE + split * joined_stride(DH);
+    for (int e = tid; e < DH; e += NW * 64) {
+      const float v = meet([&](int i) { return part[i][e]; });
+      if (S == 1) store_as(out, (int64_t)b * ld_out + h * DH + e, lt > 0.f ? v / lt : 0.f, out_dtype);
+      else __hip_atomic_store(wout + DEC_PAD + e, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (S == 1) return;
+    if (tid < 2) __hip_atomic_store(wout + tid, tid ? lt : mm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // every store of this workgroup has reached the level that all XCDs share before its arrival is counted
+    __shared__ int last;
+    __builtin_amdgcn_s_waitcnt(wait_vmcnt(0));
+    __syncthreads();
+    if (tid == 0) {
+      unsigned* arrivals = reinterpret_cast<unsigned*>(block);
+      const unsigned before = __hip_atomic_fetch_add(arrivals, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      last = before == (unsigned)S - 1;
+      if (last) __hip_atomic_store(arrivals, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!last) return;
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc(block + DEC_LINE, 0, (int)(S * joined_stride(DH) * sizeof(float)), 0x00020000);
+    if (tid < DH / 4) {
+      const floatx4 r = mtj_merge_partials_coherent(rs, 0, S, joined_stride(DH), 4 * tid);
+      const int64_t o = (int64_t)b * ld_out + h * DH + 4 * tid;
+      store_as(out, o, r.x, out_dtype);
+      store_as(out, o + 1, r.y, out_dtype);
+      store_as(out, o + 2, r.z, out_dtype);
+      store_as(out, o + 3, r.w, out_dtype);
+    }
+  } else {
+    float* wout = work + (bh * S + split) * (DH + DEC_PAD);
+    for (int e = tid; e < DH; e += NW * 64) {
+      const float v = meet([&](int i) { return part[i][e]; });
+      if (S == 1 && out) store_as(out, (int64_t)b * ld_out + h * DH + e, lt > 0.f ? v / lt : 0.f, out_dtype);
+      else wout[DEC_PAD + e] = v;
+    }
+    if (!(S == 1 && out) && tid == 0) { wout[0] = mm; wout[1] = lt; }
   }
-  if (!(S == 1 && out) && tid == 0) { wout[0] = mm; wout[1] = lt; }
 }
 
 // Merge of the S partials of one (sequence, head), four elements per thread (the out-projection GEMV does the same
@@ -1246,6 +1363,14 @@ __global__ __launch_bounds__(DH / 4) void attn_combine_kernel(const float* __res
 // length (8 x 16 heads of 256 x 80 .. 640 keys 17.9 -> 16.3 us, 250 .. 2000 40.8 -> 35.5), leave long equal ones as they are
 // (2000 keys 51.7 -> 49.6) and cost every short window of up to one workgroup step per range: 64 keys 7.8 -> 8.8 us, d_head
 // 64 up to 300 keys 8.1 -> 9.0.
+// key ranges a pair may be cut into (room for their partials), and workgroups: two per CU, or two per pair
+int joined_splits(int64_t B, int64_t H) { return B * H > 64 ? 8 : 16; }
+int64_t joined_grid(int64_t B, int64_t H) { return B * H > 256 ? 2 * B * H : 512; }
+// a lane per sequence, 32-bit sums of keys
+bool joined_ok(int64_t B, int64_t H, int64_t Tcap) {
+  return B > 0 && B <= 64 && H > 0 && H < 65536 && Tcap > 0 && Tcap < (1ll << 30) && (Tcap + 2) * B * H < (1ll << 31);
+}
+
 int decode_splits(int64_t B, int64_t H, int64_t Tcap) {
   int64_t S = 256 / (B * H);
   if (S > (Tcap + 15) / 16) S = (Tcap + 15) / 16;
@@ -1358,7 +1483,7 @@ namespace {
 // merge = false: only the partials are produced (the caller merges them, see mtj_attn_merge), out may be NULL
 int attn_decode_impl(const char* who, const float* q, const void* k_cache, const void* v_cache, const int32_t* pos,
                      int64_t B, int64_t H, int64_t Tcap, int64_t dh, void* out, int64_t ld_out, int out_dtype, int dtype,
-                     void* work, bool merge, void* stream) {
+                     void* work, bool merge, bool join, void* stream) {
   MTJ_REQUIRE(q && k_cache && v_cache && pos && work && (out || !merge), MTJ_EINVAL, "%s: null pointer", who);
   MTJ_REQUIRE(B > 0 && H > 0 && Tcap > 0 && B < 65536 && H < 65536 && Tcap < (1ll << 30), MTJ_EINVAL, "%s: bad shape", who);
   MTJ_REQUIRE(mtj_aligned16(q) && mtj_aligned16(k_cache) && mtj_aligned16(v_cache) && mtj_aligned16(work), MTJ_EALIGN,
@@ -1367,14 +1492,19 @@ int attn_decode_impl(const char* who, const float* q, const void* k_cache, const
     MTJ_REQUIRE(ld_out >= H * dh, MTJ_EINVAL, "%s: ld_out < H * dh", who);
     MTJ_REQUIRE(mtj_is_dtype(out_dtype), MTJ_EDTYPE, "%s: out_dtype %d", who, out_dtype);
   }
-  const int S = decode_splits(B, H, Tcap);
+  const int S = join ? joined_splits(B, H) : decode_splits(B, H, Tcap);
   float* partials = reinterpret_cast<float*>(work);
   dim3 grid((unsigned)S, (unsigned)H, (unsigned)B);
   hipStream_t s = (hipStream_t)stream;
 #define MTJ_DECODE(T, DH)                                                                                         \
   do {                                                                                                            \
-    attn_decode_kernel<T, DH><<<grid, 256, 0, s>>>(q, (const T*)k_cache, (const T*)v_cache, pos, (int)H, (int)Tcap, \
-                                                   partials, out, ld_out, out_dtype);                             \
+    if (join) {                                                                                                   \
+      attn_decode_kernel<T, DH, true, JOIN_NW, JOIN_NI><<<(unsigned)joined_grid(B, H), JOIN_NW * 64, 0, s>>>(       \
+          q, (const T*)k_cache, (const T*)v_cache, pos, (int)B, (int)H, (int)Tcap, S, partials, out, ld_out, out_dtype); \
+      break;                                                                                                      \
+    }                                                                                                             \
+    attn_decode_kernel<T, DH, false><<<grid, 256, 0, s>>>(q, (const T*)k_cache, (const T*)v_cache, pos, (int)B, (int)H, \
+                                                          (int)Tcap, S, partials, out, ld_out, out_dtype);        \
     if (merge && S > 1)                                                                                           \
       attn_combine_kernel<DH><<<dim3((unsigned)H, (unsigned)B), DH / 4, 0, s>>>(partials, S, (int)H, out, ld_out,  \
                                                                                  out_dtype);                      \
@@ -1396,7 +1526,22 @@ extern "C" int mtj_attn_decode(const float* q, const void* k_cache, const void* 
                                int64_t H, int64_t Tcap, int64_t dh, void* out, int64_t ld_out, int out_dtype, int dtype,
                                void* work, void* stream) {
   return attn_decode_impl("mtj_attn_decode", q, k_cache, v_cache, pos, B, H, Tcap, dh, out, ld_out, out_dtype, dtype, work,
-                          true, stream);
+                          true, false, stream);
+}
+
+extern "C" int64_t mtj_attn_decode_joined_work_bytes(int64_t B, int64_t H, int64_t dh, int64_t Tcap) {
+  if (dh <= 0 || !joined_ok(B, H, Tcap)) return 0;
+  return B * H * joined_block(joined_splits(B, H), dh) * (int64_t)sizeof(float);
+}
+
+extern "C" int mtj_attn_decode_joined(const float* q, const void* k_cache, const void* v_cache, const int32_t* pos,
+                                      int64_t B, int64_t H, int64_t Tcap, int64_t dh, void* out, int64_t ld_out,
+                                      int out_dtype, int dtype, void* work, void* stream) {
+  MTJ_REQUIRE((reinterpret_cast<uintptr_t>(work) & 127u) == 0, MTJ_EALIGN, "mtj_attn_decode_joined: work must be 128-byte aligned");
+  MTJ_REQUIRE(B <= 64 && (joined_ok(B, H, Tcap) || B <= 0 || H <= 0 || Tcap <= 0), MTJ_ELIMIT,
+              "mtj_attn_decode_joined: at most 64 sequences, B * H * Tcap below 2^31; use mtj_attn_decode");
+  return attn_decode_impl("mtj_attn_decode_joined", q, k_cache, v_cache, pos, B, H, Tcap, dh, out, ld_out, out_dtype, dtype,
+                          work, true, true, stream);
 }
 
 extern "C" int mtj_attn_decode_partials(const float* q, const void* k_cache, const void* v_cache, const int32_t* pos,
@@ -1404,7 +1549,7 @@ extern "C" int mtj_attn_decode_partials(const float* q, const void* k_cache, con
                                         mtj_attn_merge* merge, void* stream) {
   MTJ_REQUIRE(merge, MTJ_EINVAL, "mtj_attn_decode_partials: null pointer");
   const int rc = attn_decode_impl("mtj_attn_decode_partials", q, k_cache, v_cache, pos, B, H, Tcap, dh, nullptr, 0, MTJ_F32,
-                                  dtype, work, false, stream);
+                                  dtype, work, false, false, stream);
   if (rc) return rc;
   const int S = decode_splits(B, H, Tcap);
   merge->partials = reinterpret_cast<const float*>(work);
@@ -1466,5 +1611,5 @@ extern "C" int mtj_attn_decode_static(const float* q, const void* k_cache, const
   void* work = nullptr;
   if (int rc = scratch_address(&work)) return rc;
   return attn_decode_impl("mtj_attn_decode_static", q, k_cache, v_cache, pos, B, H, Tcap, dh, out, ld_out, out_dtype,
-                          dtype, work, true, stream);
+                          dtype, work, true, false, stream);
 }

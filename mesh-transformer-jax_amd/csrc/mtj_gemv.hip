@@ -390,48 +390,6 @@ struct outatt_args {
 
 __device__ __forceinline__ int oa_pstride(int dh) { return (dh + MTJ_DEC_PAD + 31) / 32 * 32; }
 
-// mtj_merge_partials for partials that other workgroups of the SAME launch have written: every load carries sc1, the
-// cache policy of an agent-scope atomic load, so it is served from the level all XCDs share and never from a line this
-// XCD's L2 (or this CU's vector cache) may still hold from an earlier launch - the partials live at the same addresses in
-// every launch.  rs covers the partials (everything behind the counter block), hoff is the byte offset of the head's
-// first partial in it.  Same arithmetic, same order as mtj_merge_partials.
-constexpr int OA_SC1 = 16;            // cache-policy operand of a buffer load: bit 4 = sc1
-__device__ __forceinline__ floatx4 oa_merge_coherent(__amdgpu_buffer_rsrc_t rs, int hoff, int S, int stride, int e) {
-  float mm = -INFINITY, lt = 0.f;
-  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int s0 = 0; s0 < S; s0 += 4) {
-    float m[4], l[4];
-    floatx4 v[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int off = hoff + (s0 + i < S ? s0 + i : S - 1) * stride * 4;
-      const uint32x2 st = __builtin_bit_cast(uint32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, OA_SC1));
-      m[i] = __uint_as_float(st.x);
-      l[i] = __uint_as_float(st.y);
-      v[i] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs, off + (MTJ_DEC_PAD + e) * 4, 0, OA_SC1));
-    }
-    float mb = mm;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (s0 + i >= S) m[i] = -INFINITY;
-      mb = fmaxf(mb, m[i]);
-    }
-    if (mb == -INFINITY) continue;
-    const float r = (mm == -INFINITY) ? 0.f : __expf(mm - mb);
-    lt *= r;
-    acc *= r;
-    mm = mb;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float f = (m[i] == -INFINITY) ? 0.f : __expf(m[i] - mm);
-      lt = fmaf(f, l[i], lt);
-      acc += f * v[i];
-    }
-  }
-  const float inv = lt > 0.f ? 1.0f / lt : 0.f;
-  return acc * inv;
-}
-
 template <typename T, typename TKV, int DH>
 __global__ __launch_bounds__(1024) void gemv_outatt_kernel(const outatt_args oa) {
   const gemv_args& a = oa.g;
@@ -679,7 +637,7 @@ __global__ __launch_bounds__(1024) void gemv_outatt_kernel(const outatt_args oa)
         __builtin_amdgcn_make_buffer_rsrc(oa.work + OA_HEAD, 0, oa.H * S * ps * 4, 0x00020000);
     for (int k = tid * 4; k < dm; k += 4096) {
       const int hh = k / DH, e = k - hh * DH;
-      *reinterpret_cast<floatx4*>(xs + k) = oa_merge_coherent(prs, hh * S * ps * 4, S, ps, e);
+      *reinterpret_cast<floatx4*>(xs + k) = mtj_merge_partials_coherent(prs, hh * S * ps * 4, S, ps, e);
     }
   }
   __syncthreads();

@@ -199,7 +199,10 @@ class Session:
         nb = 0 if self.gemv_path else L.mtj_gemm_splitk_work_bytes(B, d, d + F, w.mm_dtype)
         nb = max(nb, splitk_work_bound(M, d, d + F, w.mm_dtype))
         self.gemm_work = torch.empty(max(nb, 256), dtype=torch.uint8, device=dev)
-        self.attn_work = torch.zeros(max(L.mtj_attn_decode_work_bytes(B, H, dh, Tcap), 256), dtype=torch.uint8, device=dev)
+        # batched decode attends in one launch where that covers the shape (its counters are zeroed here, once)
+        nb = 0 if self.gemv_path else L.mtj_attn_decode_joined_work_bytes(B, H, dh, Tcap)
+        self.joined_attn = nb > 0
+        self.attn_work = torch.zeros(max(nb or L.mtj_attn_decode_work_bytes(B, H, dh, Tcap), 256), dtype=torch.uint8, device=dev)
         # batch 1: the out projection computes the attention itself when the shape allows it (its counter block is
         # zeroed here, once, and then only the kernel touches it)
         self.fused_attn = bool(self.gemv_path and cfg.get("fused_decode_attention", True) and
@@ -389,8 +392,9 @@ class Engine:
             ip = self._inproj(ses, i, 1, ses.pos, ses.q, F32, ses.act, A, None)
             check(L.mtj_gemm(ptr(ses.h), d, ptr(w.w_in_mm[i]), ptr(w.b1[i]), B, 3 * d + F, d, w.mm_dtype, EPI_INPROJ,
                              None, 0, 0, C.byref(ip), w.alpha_in[i], s))
-            check(L.mtj_attn_decode(ptr(ses.q), ptr(ses.kc[i]), ptr(ses.vc[i]), ptr(ses.pos), B, self.H, ses.Tcap,
-                                    self.dh, ptr(ses.act), d + F, A, A, ptr(ses.attn_work), s))
+            attend = L.mtj_attn_decode_joined if ses.joined_attn else L.mtj_attn_decode
+            check(attend(ptr(ses.q), ptr(ses.kc[i]), ptr(ses.vc[i]), ptr(ses.pos), B, self.H, ses.Tcap,
+                         self.dh, ptr(ses.act), d + F, A, A, ptr(ses.attn_work), s))
             if next_ln is not None:
                 check(L.mtj_gemm_splitk_ln(ptr(ses.act), d + F, ptr(w.w_out_mm[i]), ptr(w.b2[i]), B, d, d + F, w.mm_dtype,
                                            ptr(ses.x), d, ptr(ses.gemm_work), ses.gemm_work.numel(), ptr(next_ln[0]),

@@ -64,6 +64,13 @@ def test_argument_validation_needs_no_device():
     assert lib.mtj_attn_decode_splits(1, 16, 2047) == 8 and lib.mtj_attn_decode_splits(32, 16, 2047) == 1
     assert lib.mtj_attn_decode_splits(1, 16, 20) == 2          # never fewer than 16 slots per range at a full window
     assert lib.mtj_attn_decode_work_bytes(1, 16, 256, 2047) == 16 * 8 * 260 * 4
+    # in one launch: a line for the counter and up to 16 (8 from 65 pairs on) partials of whole lines per (sequence, head)
+    assert lib.mtj_attn_decode_joined_work_bytes(3, 16, 256, 2047) == 48 * (128 + 16 * 288 * 4)
+    assert lib.mtj_attn_decode_joined_work_bytes(64, 16, 64, 2047) == 1024 * (128 + 8 * 96 * 4)
+    for B, H, Tcap in ((65, 16, 100), (64, 4096, 10000), (1, 0, 5), (0, 16, 5), (2, 16, 0)):
+        assert lib.mtj_attn_decode_joined_work_bytes(B, H, 256, Tcap) == 0
+    assert lib.mtj_attn_decode_joined(*[None] * 4, 65, 16, 100, 256, None, 4096, 0, 2, None, None) == -5
+    assert lib.mtj_attn_decode_joined(*[None] * 4, 2, 16, 100, 256, None, 4096, 0, 2, None, None) == -1
     assert lib.mtj_sample_work_bytes(32, 50400) == 256         # kept in the ABI; the sampler sorts nothing
 
 

@@ -917,6 +917,74 @@ def test_attn_decode_key_ranges_of_a_batch(L, dt, dh, H, Tcap, positions, ranges
     test_attn_decode_window(L, dt, dh, H, Tcap, positions)
 
 
+# lengths around the step (64 keys of 256 float16, 256 of 64) and the cut; sequences without a key, past the window, alone
+@pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("dh,H", [(64, 8), (256, 16), (256, 1)])
+@pytest.mark.parametrize("Tcap,steps", [
+    (7, [[0, 6, 9], [3, -1, 6]]), (2047, [[700], [2046], [0]]), (2047, [[63, 64, 1999], [128, 255, 256], [5000, 10, 1300]]),
+    (700, [[80 * (i + 1) - 1 for i in range(8)], [699] * 8]), (1300, [[(i * 131) % 1400 for i in range(24)]]),
+    (1100, [[5] * 31 + [1099], [1099] * 32]), (300, [[(i * 37) % 320 for i in range(64)]])])
+def test_attn_decode_in_one_launch(L, dt, dh, H, Tcap, steps):
+    """mtj_attn_decode_joined against the float64 attention and against mtj_attn_decode; calls in a row share the
+    workspace, whose counters every launch leaves at zero."""
+    a = abi()
+    B = len(steps[0])
+    g = torch.Generator(device=DEV).manual_seed(Tcap + dh + B)
+    kc, vc = (torch.randn(B, H, Tcap, dh, generator=g, device=DEV).to(TD[dt]) for _ in range(2))
+    code = a.dtype_code(TD[dt])
+    work = torch.zeros(L.mtj_attn_decode_joined_work_bytes(B, H, dh, Tcap), dtype=torch.uint8, device=DEV)
+    two = torch.zeros(L.mtj_attn_decode_work_bytes(B, H, dh, Tcap), dtype=torch.uint8, device=DEV)
+    ld = H * dh + 8
+    for positions in steps:
+        q = torch.randn(B, H, dh, generator=g, device=DEV)
+        pos = torch.tensor(positions, dtype=torch.int32, device=DEV)
+        out, again, ref2 = (torch.full((B, ld), 7.0, device=DEV) for _ in range(3))
+        for o in (out, again):
+            a.check(L.mtj_attn_decode_joined(a.ptr(q), a.ptr(kc), a.ptr(vc), a.ptr(pos), B, H, Tcap, dh, a.ptr(o), ld, 0,
+                                             code, a.ptr(work), S()))
+        a.check(L.mtj_attn_decode(a.ptr(q), a.ptr(kc), a.ptr(vc), a.ptr(pos), B, H, Tcap, dh, a.ptr(ref2), ld, 0, code,
+                                  a.ptr(two), S()))
+        torch.cuda.synchronize()
+        assert torch.equal(out, again) and bool((out[:, H * dh:] == 7.0).all())
+        block = work.numel() // (B * H)
+        assert int(work.view(B * H, block)[:, :4].max()) == 0
+        for b, p in enumerate(positions):
+            n = min(p + 1, Tcap)
+            if n <= 0:
+                assert bool((out[b, :H * dh] == 0).all())
+                continue
+            s = (kc[b, :, :n].double() @ q[b].double()[:, :, None])[..., 0] / math.sqrt(dh)
+            ref = (torch.softmax(s, -1)[:, None] @ vc[b, :, :n].double()).reshape(-1)
+            assert rel_err(out[b, :H * dh], ref) < 3e-6, (dt, dh, Tcap, p)
+            assert rel_err(out[b, :H * dh], ref2[b, :H * dh]) < 3e-6
+
+
+def test_attn_decode_in_one_launch_replayed_from_a_graph(L):
+    """Positions move between the replays (the cut follows them), with eager work in between."""
+    a = abi()
+    B, H, dh, Tcap = 5, 16, 256, 900
+    g = torch.Generator(device=DEV).manual_seed(1)
+    q = torch.randn(B, H, dh, generator=g, device=DEV)
+    kc, vc = (torch.randn(B, H, Tcap, dh, generator=g, device=DEV).half() for _ in range(2))
+    pos = torch.zeros(B, dtype=torch.int32, device=DEV)
+    work = torch.zeros(L.mtj_attn_decode_joined_work_bytes(B, H, dh, Tcap), dtype=torch.uint8, device=DEV)
+    out, eager = (torch.zeros(B, H * dh, device=DEV) for _ in range(2))
+    call = lambda o: a.check(L.mtj_attn_decode_joined(a.ptr(q), a.ptr(kc), a.ptr(vc), a.ptr(pos), B, H, Tcap, dh, a.ptr(o),
+                                                      H * dh, 0, 2, a.ptr(work), S()))
+    call(eager)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(out)
+    for positions in ([0, 1, 2, 3, 4], [899, 10, 500, 1200, 64], [899] * 5, [127, 128, 129, 600, 3]):
+        pos.copy_(torch.tensor(positions, dtype=torch.int32))
+        graph.replay()
+        torch.cuda.synchronize()
+        call(eager)
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager), positions
+
+
 @pytest.mark.parametrize("dt", ["f32", "f16"])
 @pytest.mark.parametrize("dh,H,F", [(64, 8, 2048), (256, 16, 16384)])
 @pytest.mark.parametrize("Tcap,p", [(2047, 650), (2047, 2046), (130, 3), (9, 40)])
