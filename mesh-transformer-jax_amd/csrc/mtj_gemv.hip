@@ -159,7 +159,10 @@ __device__ __forceinline__ void stage_x(const gemv_args& a, float* __restrict__ 
 // its arrival; the workgroup whose arrival completes the count reads the word, which by then holds every
 // workgroup's contribution, and does what the sampler does (token, position, embedding of the token for the next
 // step), and puts both words back to 0.  Nobody waits for anybody: the order in which workgroups run does not matter.
-template <typename T, int U, bool FULL, bool MERGE, bool ARGMAX = false>
+// RPT > 1 (FULL): K is U / RPT wavefront loads, a tile is RPT whole rows, and the part of x that a lane multiplies stays in
+// its registers.  With one short row per tile most of the U loads of a wavefront would be outside the row, and nothing in
+// flight but that row.
+template <typename T, int U, bool FULL, bool MERGE, bool ARGMAX = false, int RPT = 1>
 __global__ __launch_bounds__(1024) void gemv_kernel(const gemv_args a) {
   extern __shared__ __align__(16) float xs[];
   __shared__ float red[2][16];
@@ -193,7 +196,13 @@ __global__ __launch_bounds__(1024) void gemv_kernel(const gemv_args a) {
   const int tpr = (K + STEP * U - 1) / (STEP * U);          // tiles per row
   uint32x4 w[U], w2[U];
   __builtin_amdgcn_sched_barrier(0);
-  if (FULL) {
+  if constexpr (RPT > 1) {
+    // (dispatch_rows() sees to RPT rows per wavefront at least)
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      w[u] = __builtin_nontemporal_load(
+          reinterpret_cast<const uint32x4*>(W + (row0 + u / (U / RPT)) * a.K + u % (U / RPT) * STEP + lane * EPC));
+  } else if (FULL) {
     const T* rowp = W + (nrows > 0 ? row0 : 0) * a.K;      // a wavefront without rows reads (and drops) row 0
 #pragma unroll
     for (int u = 0; u < U; ++u) w[u] = __builtin_nontemporal_load(reinterpret_cast<const uint32x4*>(rowp + u * STEP + lane * EPC));
@@ -223,7 +232,56 @@ __global__ __launch_bounds__(1024) void gemv_kernel(const gemv_args a) {
 
   // ---- stream my rows; lane r keeps the sum of row r
   float mine = 0.f;
-  if (FULL) {
+  if constexpr (RPT > 1) {
+    constexpr int LPR = U / RPT;                            // loads per row
+    constexpr bool KEEP = LPR * EPC <= 16;                  // (more would spill)
+    float xr[KEEP ? LPR * EPC : 1];
+    if constexpr (KEEP)
+#pragma unroll
+      for (int j = 0; j < LPR; ++j)
+#pragma unroll
+        for (int e = 0; e < EPC; e += 4)
+          *reinterpret_cast<floatx4*>(xr + j * EPC + e) = *reinterpret_cast<const floatx4*>(xs + j * STEP + lane * EPC + e);
+    const T* base = W + row0 * a.K + lane * EPC;
+    auto consume = [&](const uint32x4 (&t)[U], int r0) {
+      float acc[RPT];
+#pragma unroll
+      for (int i = 0; i < RPT; ++i) {
+        acc[i] = 0.f;
+#pragma unroll
+        for (int j = 0; j < LPR; ++j)
+          chunk<T>::fma(t[i * LPR + j], KEEP ? xr + j * EPC : xs + j * STEP + lane * EPC, acc[i]);
+      }
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+        for (int i = 0; i < RPT; ++i) acc[i] += __shfl_xor(acc[i], o);
+#pragma unroll
+      for (int i = 0; i < RPT; ++i)
+        if (lane == r0 + i) mine = acc[i];                  // rows beyond the last: lanes that finish nothing
+    };
+    auto request = [&](uint32x4 (&t)[U], int r0) {          // rows beyond the last read that one again (and are dropped)
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int r = r0 + u / LPR < nrows ? r0 + u / LPR : nrows - 1;
+        t[u] = __builtin_nontemporal_load(reinterpret_cast<const uint32x4*>(base + (int64_t)r * K + u % LPR * STEP));
+      }
+    };
+    int r0 = 0;
+    for (; r0 + 2 * RPT < nrows; r0 += 2 * RPT) {
+      request(w2, r0 + RPT);
+      consume(w, r0);
+      request(w, r0 + 2 * RPT);
+      consume(w2, r0 + RPT);
+    }
+    if (r0 + RPT < nrows) {
+      request(w2, r0 + RPT);
+      consume(w, r0);
+      consume(w2, r0 + RPT);
+    } else {
+      consume(w, r0);
+    }
+  } else if (FULL) {
     constexpr int TILE = STEP * U;
     const T* base = W + row0 * a.K + lane * EPC;            // tile g of this wavefront starts at base + g * TILE
     const int ntiles = nrows * tpr;
@@ -334,7 +392,7 @@ __global__ __launch_bounds__(1024) void gemv_kernel(const gemv_args a) {
   }
 }
 
-template <typename T, int U, bool FULL, bool MERGE, bool ARGMAX = false>
+template <typename T, int U, bool FULL, bool MERGE, bool ARGMAX = false, int RPT = 1>
 int launch(const gemv_args& a, hipStream_t s) {
   const size_t lds = (size_t)a.K * sizeof(float);
   const int64_t units = a.epi == MTJ_EPI_INPROJ ? a.N / 2 : a.N;
@@ -344,11 +402,11 @@ int launch(const gemv_args& a, hipStream_t s) {
   const int64_t upw = a.epi == MTJ_EPI_INPROJ ? 2 : 1;
   while ((units + grid * 16 - 1) / (grid * 16) * upw > 62) grid *= 2;   // a lane per row: <= 64 rows per wavefront
   static mtj_device_once once;
-  if (int rc = mtj_allow_lds(once, "mtj_gemv", &gemv_kernel<T, U, FULL, MERGE, ARGMAX>, 160 * 1024 - 512)) return rc;
+  if (int rc = mtj_allow_lds(once, "mtj_gemv", &gemv_kernel<T, U, FULL, MERGE, ARGMAX, RPT>, 160 * 1024 - 512)) return rc;
   gemv_args b = a;
   b.upb = (int)(units / grid);
   b.upb_rem = (int)(units % grid);
-  gemv_kernel<T, U, FULL, MERGE, ARGMAX><<<(unsigned)grid, 1024, lds, s>>>(b);
+  gemv_kernel<T, U, FULL, MERGE, ARGMAX, RPT><<<(unsigned)grid, 1024, lds, s>>>(b);
   return mtj_check_launch("mtj_gemv");
 }
 
@@ -649,13 +707,30 @@ __global__ __launch_bounds__(1024) void gemv_outatt_kernel(const outatt_args oa)
   if (lane < nrows) reinterpret_cast<float*>(a.out)[row0 + lane] = mine + pre_add;
 }
 
+template <typename T, bool ARGMAX>
+int dispatch_rows(const gemv_args& a, hipStream_t s) {
+  constexpr int U = 8, STEP = 64 * chunk<T>::EPC;
+  // rows of one, two or four loads, and a tile of them for every wavefront of the grid: 50400 rows of 512 float32 27.6 -> 20.8
+  // us, 1024 41.3 -> 37.2; bfloat16 512 21.6 -> 16.2, 1024 30.8 -> 22.3, 2048 42.5 -> 37.9; 16384 of 512 float32 13.6 -> 11.1.
+  // With less than a tile for a wavefront the rows read twice cost more: 5000 of 512 7.0 against 7.7, 3584 5.8 against 7.0.
+  const int64_t rows = a.N / 4096;
+  if (a.K == STEP && rows >= 8) return launch<T, U, true, false, ARGMAX, 8>(a, s);
+  if (a.K == 2 * STEP && rows >= 4) return launch<T, U, true, false, ARGMAX, 4>(a, s);
+  if (a.K == 4 * STEP && rows >= 2) return launch<T, U, true, false, ARGMAX, 2>(a, s);
+  return a.K % (U * STEP) == 0 ? launch<T, U, true, false, ARGMAX>(a, s) : launch<T, U, false, false, ARGMAX>(a, s);
+}
+
 template <typename T>
 int dispatch(const gemv_args& a, hipStream_t s) {
-  constexpr int U = 8;
-  const bool full = a.K % (U * 64 * chunk<T>::EPC) == 0;
-  if (a.am_work) return full ? launch<T, U, true, false, true>(a, s) : launch<T, U, false, false, true>(a, s);
+  constexpr int U = 8, STEP = 64 * chunk<T>::EPC;
+  const bool full = a.K % (U * STEP) == 0;
+  if (a.am_work) return dispatch_rows<T, true>(a, s);
+  // the out projection of a narrow model, K five times d_model: 512 float32 7.1 -> 5.8 us, 1024 12.5 -> 10.5; bfloat16 512
+  // 4.9 -> 4.6, 1024 8.1 -> 6.5
+  if (!full && a.K % (5 * STEP) == 0 && a.epi == MTJ_EPI_RESID)
+    return a.am.partials ? launch<T, 5, true, true>(a, s) : launch<T, 5, true, false>(a, s);
   if (a.am.partials) return full ? launch<T, U, true, true>(a, s) : launch<T, U, false, true>(a, s);
-  return full ? launch<T, U, true, false>(a, s) : launch<T, U, false, false>(a, s);
+  return dispatch_rows<T, false>(a, s);
 }
 
 }  // namespace

@@ -442,6 +442,15 @@ def test_gemv_store_resid_and_layernorm(L, dt, N, K):
         assert rel_err(out, h @ Wh.double() + bias.double()) < 6e-6
 
 
+@pytest.mark.parametrize("dt,loads", [("f32", 1), ("f32", 2), ("bf16", 4), ("f16", 1), ("bf16", 2), ("f32", 4), ("bf16", 5),
+                                      ("f32", 10)])
+@pytest.mark.parametrize("rows,more", [(0, 5), (8, -1), (8, 0), (8, 4097), (12, 3000)])
+def test_gemv_short_rows(L, dt, loads, rows, more):
+    """Rows of 1, 2 and 4 wavefront loads: tiles of several rows from a tile per wavefront on (`rows` a wavefront and
+    `more`), one row at a time below; 5 and 10 loads: the residual epilogue in tiles of five."""
+    test_gemv_store_resid_and_layernorm(L, dt, 4096 * rows + more, loads * (256 if dt == "f32" else 512))
+
+
 # ------------------------------------------------------------------ fused input projection (GEMM and GEMV)
 def _layer_params(cfg, seed, dt):
     p = O.seeded_params(cfg, seed, TD[dt])
@@ -642,6 +651,29 @@ def test_inproj_gemv_decode_appends_to_ring(dt):
         assert rel_err(ses.kc[0][0, :, pos % Tcap][None], k_ref) < tol
         assert rel_err(ses.vc[0][0, :, pos % Tcap][None], v_ref) < tol
         assert rel_err(ses.act[:, 512:], g_ref) < 3e-6
+
+
+def test_inproj_gemv_of_several_rows_per_tile():
+    """d_model 2048 in bfloat16: 3 or 4 rows (pairs) per wavefront, two per tile; against the float64 layer."""
+    from mesh_transformer.engine import Engine
+    a = abi()
+    d = 2048
+    cfg = dict(layers=1, d_model=d, n_heads=8, n_vocab=64, pe="rotary", pe_rotary_dims=64, cores_per_replica=1)
+    p = _layer_params(cfg, 5, "bf16")
+    eng = Engine(cfg, {k: {n: v.to(DEV) for n, v in m.items()} for k, m in p.items()}, DEV, layer_ids=[0], embed=False, proj=False)
+    ses = eng.session(1, 6, 1, 64)
+    L, w = a.lib(), eng.w
+    x = torch.randn(1, d, generator=torch.Generator().manual_seed(6)).to(DEV)
+    ses.pos.fill_(13)
+    ip = eng._inproj(ses, 0, 1, ses.pos, ses.q, 0, ses.act, 0, None)
+    a.check(L.mtj_gemv(a.ptr(x), a.ptr(w.ln_s[0]), a.ptr(w.ln_o[0]), a.ptr(w.w_in[0]), a.ptr(w.b1[0]), 7 * d, d,
+                       w.dtype, a.EPI_INPROJ, None, 0, C.byref(ip), None, S()))
+    torch.cuda.synchronize()
+    q_ref, k_ref, v_ref, g_ref, _ = _inproj_reference(cfg, p, x.double().cpu(), np.array([13]))
+    assert rel_err(ses.q.reshape(1, eng.H, eng.dh), q_ref) < 3e-6
+    assert rel_err(ses.kc[0][0, :, 1][None], k_ref) < 5e-4       # the K/V window of a bfloat16 model is float16
+    assert rel_err(ses.vc[0][0, :, 1][None], v_ref) < 5e-4
+    assert rel_err(ses.act[:, d:], g_ref) < 3e-6
 
 
 # ------------------------------------------------------------------ attention
@@ -1450,6 +1482,11 @@ def test_logits_launch_that_is_its_own_greedy_sampler(L, dt, N, K, ln):
     with pytest.raises(ValueError):
         a.check(L.mtj_gemv_greedy(a.ptr(x), None, None, a.ptr(W), a.ptr(bias), N, K, code, a.ptr(lg1), a.ptr(tok1), None, 0,
                                   a.ptr(pos1), a.ptr(pos_start), None, None, S()))
+
+
+@pytest.mark.parametrize("dt,N,K", [("f32", 50400, 512), ("bf16", 33000, 512), ("bf16", 8195, 2048), ("f32", 32768, 256)])
+def test_logits_launch_of_short_rows_that_is_its_own_greedy_sampler(L, dt, N, K):
+    test_logits_launch_that_is_its_own_greedy_sampler(L, dt, N, K, True)
 
 
 def test_greedy_lowest_index_on_ties(L):
