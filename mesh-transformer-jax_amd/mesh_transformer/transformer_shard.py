@@ -279,7 +279,7 @@ class CausalTransformer:
             final_state = (toks[:, -1], DecodeStates(eng, ses, P - 1 + G), None)
             out = (toks, None)
             if return_logits:
-                torch.from_numpy(logits_np).view(B, G, eng.w.V).copy_(logits_out)
+                self._to_host(ses, logits_out.view(-1), torch.from_numpy(logits_np).view(-1))
                 out = out + (logits_np,)
             if return_keep_mask:
                 out = out + (masks.permute(1, 0, 2).cpu().numpy().astype(bool),)
@@ -352,6 +352,35 @@ class CausalTransformer:
             all_loss = loss.view(B, T).cpu().numpy()
             return {"loss": all_loss.mean(-1), "last_loss": all_loss[:, -1].copy(), "all_loss": all_loss,
                     "correct": correct.view(B, T).cpu().numpy().astype(bool)}
+
+    HOST_CHUNK = 1 << 20     # floats
+
+    def _to_host(self, ses, src, dst):
+        """dst (host) = src (device), flat float32.  A copy to pageable memory goes at 12 - 17 GB/s; here one half of the session's
+        8 MiB of pinned memory is filled while all threads empty the other (6.4 MB 0.91 -> 0.17 ms, 29 MB 2.8 -> 0.7, 206 MB 12.0 ->
+        5.0; chunks of 2 MiB 0.22, 0.8 and 5.5, of 1 MiB 0.25, 1.0 and 6.8)."""
+        C, n = self.HOST_CHUNK, src.numel()
+        if n <= C // 4:
+            dst.copy_(src)
+            return
+        if getattr(ses, "host_stage", None) is None:
+            ses.host_stage = [(torch.empty(C, dtype=torch.float32, pin_memory=True), torch.cuda.Event()) for _ in range(2)]
+        waiting = []
+
+        def empty_one():
+            (pinned, landed), at = waiting.pop(0)
+            landed.synchronize()
+            dst[at:at + C].copy_(pinned[:min(C, n - at)])
+
+        for i, at in enumerate(range(0, n, C)):
+            if len(waiting) == 2:
+                empty_one()
+            pinned, landed = ses.host_stage[i % 2]
+            pinned[:min(C, n - at)].copy_(src[at:at + C], non_blocking=True)
+            landed.record()
+            waiting.append((ses.host_stage[i % 2], at))
+        while waiting:
+            empty_one()
 
     def _ensure_io(self, ses, G, V):
         if getattr(ses, "G_max", 0) < G:

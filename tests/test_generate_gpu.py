@@ -619,3 +619,19 @@ def test_operands_beyond_the_float16_range_saturate_and_stay_finite():
     assert e_c < 2e-2 < e_f
     _, out = net.generate(O.left_pad(toks, 64), [48], 4, {}, return_logits=True)
     assert np.isfinite(out[2]).all()
+
+
+@pytest.mark.parametrize("n", [1, (1 << 18) - 1, (1 << 18) + 1, (1 << 20) - 1, 1 << 20, (1 << 20) + 1, 1 << 21, (1 << 22) + 17])
+def test_results_reach_the_host_in_chunks(n):
+    """CausalTransformer._to_host around its chunk of 2^20 floats, twice through the same pinned memory, behind work
+    that the stream has not finished yet."""
+    from types import SimpleNamespace
+    from mesh_transformer.transformer_shard import CausalTransformer
+    ses = SimpleNamespace()
+    for k in range(2):
+        src = torch.arange(n, device=DEV, dtype=torch.float32)
+        for _ in range(20):
+            src = src + 1
+        dst = np.full(n + 3, -1.0, np.float32)
+        CausalTransformer._to_host(CausalTransformer, ses, src, torch.from_numpy(dst)[:n])
+        assert np.array_equal(dst[:n], np.arange(n, dtype=np.float32) + 20) and (dst[n:] == -1.0).all()
