@@ -1,11 +1,12 @@
 // MFMA GEMM for prefill and batched decode: C[M, N] = A[M, K] x W[N, K]^T with fused epilogues.
 // Both operands are K-contiguous and accumulation is float32; bf16 uses v_mfma_f32_32x32x16_bf16, float32 uses
-// v_mfma_f32_32x32x2_f32 (true fp32).  Three kernels share the epilogues:
+// v_mfma_f32_32x32x2_f32 (true fp32) up to 64 rows.  Four kernels share the epilogues:
 //   gemm_kernel      any dtype and shape: global -> registers -> LDS (padded rows, so that the 16-byte fragment
 //                    reads of a 32x32 MFMA hit distinct banks), LDS double-buffered;
 //   gemm_dma_kernel  large 16-bit problems: 256x256x64 tiles written straight into LDS by the memory pipeline
 //                    (buffer_load ... lds), rows xor-swizzled instead of padded, no staging registers;
-//   gemm_stream_kernel  16-bit problems of few rows: the same operand path, all rows in one tile, three or four stages.
+//   gemm_stream_kernel  16-bit problems of few rows: the same operand path, all rows in one tile, three or four stages;
+//   gemm_split_kernel  float32 problems of more than 64 rows: every operand as a sum of three bf16 numbers.
 #include "mtj_common.h"
 #include <type_traits>
 
@@ -588,6 +589,190 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_kernel(const gemm_
   epilogue<EPI, WAVES_M, WAVES_N, WM, WN>(a, out, acc, smem, m0, n0);
 }
 
+// float32 operands on the bf16 matrix cores.  A float32 number is the sum of three bf16 numbers without an error (rounded to
+// nearest, each takes 8 of the 24 significant bits of what the ones before it leave), so a product is nine products of parts;
+// the six with the largest weights are taken - the other three together are below 2^-24 of the product - and summed in
+// float32 by the matrix cores, which round once per 16 elements of K instead of once per 2.  Error against float64, 2-norm,
+// normal operands, with v_mfma_f32_32x32x2_f32 and here: K = 512 4.0e-7 and 3.4e-7, 2560 4.6e-7 and 3.9e-7, 4096 1.15e-6 and
+// 1.00e-6, 20480 (four ranges) 1.28e-6 and 1.22e-6.
+// An operand that is infinite, NaN or rounds to infinity gives NaN here, and a product next to the largest number may give
+// infinity; what is not finite is computed again in plain float32.
+//
+// Bound by the matrix cores: six v_mfma_f32_32x32x16_bf16 instead of eight v_mfma_f32_32x32x2_f32 of twice the length; the
+// splitting (11 vector instructions for two elements) runs under them.  N = 28672, K = 4096, 100 / 199 / 511 rows 305 / 517 /
+// 1010 -> 214 / 356 / 692 us (1.0 PFLOP/s of bf16 products); N = 4096, K = 20480 in four ranges, 199 / 511 rows 400 / 700 ->
+// 282 / 477; N = 3584, K = 512, 127 / 1499 rows 47 / 79 -> 35 / 53.
+// A k-tile of 16 goes global -> registers (NS k-tiles in flight) -> three bf16 planes per row in LDS, double-buffered: rows
+// of 3 x 32 bytes, padded to 112 so that the 16-byte fragment reads of 16 consecutive rows hit distinct banks.
+__device__ __attribute__((noinline)) float plain_dot(const float* __restrict__ x, const float* __restrict__ w, int n) {
+  float s = 0.f;
+  for (int k = 0; k < n && s == s; ++k) s = fmaf(x[k], w[k], s);      // a NaN stays one
+  return s;
+}
+__device__ __forceinline__ bool not_finite(float x) { return !(fabsf(x) < INFINITY); }
+
+template <int EPI, int WAVES_M, int WAVES_N, int WM, int WN, int NS>
+__global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_split_kernel(const gemm_args a) {
+  constexpr int NT = WAVES_M * WAVES_N * 64, BK = 16;
+  constexpr int BM = WAVES_M * WM * 32, BN = WAVES_N * WN * 32;
+  constexpr int ROWB = 112, PLANE = 32, STAGEB = (BM + BN) * ROWB;
+  constexpr int ROWS_PER_PASS = NT / 2;                    // a thread takes 8 elements of a row at a time
+  constexpr int A_U = BM / ROWS_PER_PASS, B_U = BN / ROWS_PER_PASS;
+  static_assert(BM % ROWS_PER_PASS == 0 && BN % ROWS_PER_PASS == 0, "tile does not divide over threads");
+  extern __shared__ __align__(16) unsigned char smem[];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+  const int fr = lane & 31, fg = lane >> 5;
+
+  // tile id as in gemm_kernel
+  const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
+  const int nblk = tiles_m * tiles_n;
+  int pid = blockIdx.x;
+  {
+    const int per = nblk / 8;
+    if (pid < per * 8) pid = (pid % 8) * per + pid / 8;
+  }
+  constexpr int GM = 8;
+  const int group = pid / (GM * tiles_n);
+  const int first_m = group * GM;
+  const int gsz = (tiles_m - first_m < GM) ? tiles_m - first_m : GM;
+  // (kept in scalar registers: the buffer descriptors are made of them)
+  const int tm = __builtin_amdgcn_readfirstlane(first_m + (pid % (GM * tiles_n)) % gsz);
+  const int tn = __builtin_amdgcn_readfirstlane((pid % (GM * tiles_n)) / gsz);
+  const int m0 = tm * BM, n0 = tn * BN;
+
+  const int rows_a = (a.M - m0 < BM) ? a.M - m0 : BM, rows_b = (a.N - n0 < BN) ? a.N - n0 : BN;
+  const float* tile_a = reinterpret_cast<const float*>(a.A) + (int64_t)m0 * a.lda;
+  const float* tile_b = reinterpret_cast<const float*>(a.W) + (int64_t)n0 * a.K;
+  const __amdgpu_buffer_rsrc_t ra_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(tile_a), 0, (int)((((int64_t)rows_a - 1) * a.lda + a.K) * 4), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(tile_b), 0, (int)((((int64_t)rows_b - 1) * a.K + a.K) * 4), 0x00020000);
+  const int row0 = tid / 2, half = tid % 2;
+  const int voff_a = (int)(((int64_t)row0 * a.lda + half * 8) * 4), voff_b = (int)(((int64_t)row0 * a.K + half * 8) * 4);
+  const int pass_a = (int)((int64_t)ROWS_PER_PASS * a.lda * 4), pass_b = (int)((int64_t)ROWS_PER_PASS * a.K * 4);
+
+  const int kt0 = __builtin_amdgcn_readfirstlane((int)((int64_t)blockIdx.y * (a.K / BK) / a.splits));
+  const int KT = __builtin_amdgcn_readfirstlane((int)((int64_t)(blockIdx.y + 1) * (a.K / BK) / a.splits)) - kt0;
+  uint32x4 ra[NS][A_U][2], rb[NS][B_U][2];
+  auto load_global = [&](auto ST_, int kt) {
+    constexpr int st = decltype(ST_)::value;
+    const int koff = (kt0 + kt) * BK * 4;
+#pragma unroll
+    for (int i = 0; i < A_U; ++i)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        ra[st][i][c] = __builtin_amdgcn_raw_buffer_load_b128(ra_rsrc, voff_a + 16 * c, koff + i * pass_a, 0);
+#pragma unroll
+    for (int i = 0; i < B_U; ++i)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        rb[st][i][c] = __builtin_amdgcn_raw_buffer_load_b128(rb_rsrc, voff_b + 16 * c, koff + i * pass_b, 0);
+  };
+  // eight float32 numbers -> three times eight bf16
+  auto split_store = [&](unsigned char* dst, const uint32x4 (&r)[2]) {
+    float x[8];
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[4 * c + e] = __uint_as_float(r[c][e]);
+#pragma unroll
+    for (int part = 0; part < 3; ++part) {
+      uint32x4 p;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        p[e] = pack_bf16x2(x[2 * e], x[2 * e + 1]);
+        if (part < 2) { x[2 * e] -= bf16_lo(p[e]); x[2 * e + 1] -= bf16_hi(p[e]); }
+      }
+      *reinterpret_cast<uint32x4*>(dst + part * PLANE) = p;
+    }
+  };
+  auto store_lds = [&](auto ST_, int buf) {
+    constexpr int st = decltype(ST_)::value;
+    unsigned char* d = smem + buf * STAGEB + row0 * ROWB + half * 16;
+#pragma unroll
+    for (int i = 0; i < A_U; ++i) split_store(d + i * ROWS_PER_PASS * ROWB, ra[st][i]);
+#pragma unroll
+    for (int i = 0; i < B_U; ++i) split_store(d + (BM + i * ROWS_PER_PASS) * ROWB, rb[st][i]);
+  };
+
+  floatx16 acc[WM][WN];
+#pragma unroll
+  for (int i = 0; i < WM; ++i)
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+
+  for_stages<0, NS>([&](auto ST_) {
+    if (decltype(ST_)::value < KT) load_global(ST_, decltype(ST_)::value);
+  });
+  store_lds(std::integral_constant<int, 0>{}, 0);
+  if (NS < KT) load_global(std::integral_constant<int, 0>{}, NS);
+  __syncthreads();
+
+  // as in gemm_kernel: PARK = stage of k-tile kt+1, STEADY: k-tiles kt+1 and kt+1+NS both exist
+  auto k_tile = [&](int kt, auto PARK_, auto STEADY_) {
+    constexpr bool steady = decltype(STEADY_)::value;
+    const int buf = kt & 1;
+    const unsigned char* as = smem + buf * STAGEB + (wm * WM * 32 + fr) * ROWB + fg * 16;
+    const unsigned char* bs = smem + buf * STAGEB + (BM + wn * WN * 32 + fr) * ROWB + fg * 16;
+    bf16x8 fa[WM][3], fb[WN][3];
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+#pragma unroll
+      for (int i = 0; i < WM; ++i) fa[i][p] = *reinterpret_cast<const bf16x8*>(as + i * 32 * ROWB + p * PLANE);
+#pragma unroll
+      for (int j = 0; j < WN; ++j) fb[j][p] = *reinterpret_cast<const bf16x8*>(bs + j * 32 * ROWB + p * PLANE);
+    }
+    if (steady || kt + 1 < KT) store_lds(PARK_, buf ^ 1);
+    if (steady || kt + 1 + NS < KT) load_global(PARK_, kt + 1 + NS);
+    // the small products first
+    constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int t = 0; t < 6; ++t)
+#pragma unroll
+      for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][pa[t]], fb[j][pb[t]], acc[i][j], 0, 0, 0);
+    __syncthreads();
+  };
+  int kt = 0;
+  for (; kt + 2 * NS < KT; kt += NS)
+    for_stages<0, NS>([&](auto S_) {
+      constexpr int s = decltype(S_)::value;
+      k_tile(kt + s, std::integral_constant<int, (s + 1) % NS>{}, std::true_type{});
+    });
+  for (; kt < KT; kt += NS)
+    for_stages<0, NS>([&](auto S_) {
+      constexpr int s = decltype(S_)::value;
+      if (kt + s < KT) k_tile(kt + s, std::integral_constant<int, (s + 1) % NS>{}, std::false_type{});
+    });
+
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < WM; ++i)
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) bad |= not_finite(acc[i][j][v]);
+  if (__any(bad))
+    for_tiles<0, 0, WM, WN>([&](auto I_, auto J_) {
+      constexpr int i = decltype(I_)::value, j = decltype(J_)::value;
+      const int c = (wn * WN + j) * 32 + fr;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int r = (wm * WM + i) * 32 + 8 * (v / 4) + 4 * fg + (v % 4);
+        if (not_finite(acc[i][j][v]) && r < rows_a && c < rows_b)
+          acc[i][j][v] = plain_dot(tile_a + (int64_t)r * a.lda + kt0 * BK, tile_b + (int64_t)c * a.K + kt0 * BK, KT * BK);
+      }
+    });
+  void* out = a.splits > 1 ? (void*)(reinterpret_cast<float*>(a.out) + blockIdx.y * a.split_stride) : a.out;
+  epilogue<EPI, WAVES_M, WAVES_N, WM, WN>(a, out, acc, smem, m0, n0);
+}
+
 // 16-bit operands, 256x256 workgroup tile, 8 wavefronts of 128x64, K step 64, two LDS stages of 64 KiB,
 // v_mfma_f32_16x16x32 (under the board's power limit it sustains a higher clock than the 32x32x16 form: 1820 against
 // 1570 TFLOP/s in a register-only loop on random float16 data).
@@ -971,6 +1156,19 @@ int launch(const gemm_args& a, hipStream_t s) {
   return mtj_check_launch("mtj_gemm");
 }
 
+template <int EPI, int WAVES_M, int WAVES_N, int WM, int WN, int NS>
+int launch_split(const gemm_args& a, hipStream_t s) {
+  constexpr int BM = WAVES_M * WM * 32, BN = WAVES_N * WN * 32;
+  constexpr size_t lds = 2 * (size_t)(BM + BN) * 112;
+  static_assert(lds <= 160 * 1024, "tile does not fit LDS");
+  static_assert(lds >= 3 * BM * sizeof(int) + WAVES_M * WAVES_N * 32 * 36 * sizeof(float), "epilogue scratch does not fit");
+  static mtj_device_once once;
+  if (int rc = mtj_allow_lds(once, "mtj_gemm", &gemm_split_kernel<EPI, WAVES_M, WAVES_N, WM, WN, NS>, lds)) return rc;
+  const int tiles = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
+  gemm_split_kernel<EPI, WAVES_M, WAVES_N, WM, WN, NS><<<dim3(tiles, a.splits), WAVES_M * WAVES_N * 64, lds, s>>>(a);
+  return mtj_check_launch("mtj_gemm");
+}
+
 // 256 x 256 tiles of gemm_dma_kernel, one workgroup per CU, from this many of them on: N = 4096, K = 20480 in one K range,
 // 144 tiles 486 us (602 with 128 x 128 tiles), 192 tiles 458 (650); 96 tiles 455 against 384 for two ranges of 128 x 128.
 // So are 144 .. 196 tiles with the other epilogues, us against 128 x 128 tiles, at every K from 256 on: STORE 144 tiles 19 (33) at
@@ -1010,7 +1208,9 @@ int dispatch_tile(const gemm_args& a, hipStream_t s) {
     const int64_t line = EPI == MTJ_EPI_INPROJ && a.K < 768 ? DMA_MIN_TILES_SHORT_INPROJ : DMA_MIN_TILES;
     if (dma_tiles(a.M, a.N) * a.splits >= line) return launch_dma<T, EPI>(a, s);        // 256 x 256, 8 wavefronts of 128 x 64
   }
-  return launch<T, EPI, 2, 2, 2, 2, BK, 2>(a, s);                   // 128 x 128
+  // 128 x 128
+  if constexpr (sizeof(T) == 4) return launch_split<EPI, 2, 2, 2, 2, 3>(a, s);
+  else return launch<T, EPI, 2, 2, 2, 2, BK, 2>(a, s);
 }
 
 template <typename T, int BK>

@@ -152,6 +152,53 @@ def test_gemm_store_and_resid(L, dt, M, N, K):
         assert rel_err(ob, A.double() @ Wh.double()) < TOL[odt] / 2
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 1, 32), (128, 127, 64), (129, 130, 96), (200, 300, 160), (65, 4100, 512), (300, 128, 1024)])
+def test_float32_products_on_the_bf16_matrix_cores(L, M, N, K):
+    """More than 64 rows of float32: tile edges, K from two k-tiles on, scales up to 2^40.  Bound: what the three left-out
+    products and the representation leave is below 2^-23 of sum |a||w|; the float32 additions (6 K / 16, each of 2^-24 of the
+    running sum) add less than 2^-24 (6 K / 16) of it, and sums of random signs are ~sqrt(K) smaller than sum |a||w|."""
+    a = abi()
+    g = torch.Generator().manual_seed(M + N + K)
+    A = (torch.randn(M, K + 4, generator=g) * 2.0 ** torch.randint(-20, 21, (M, 1), generator=g).float()).to(DEV)[:, :K]
+    W = (torch.randn(N, K, generator=g) * 2.0 ** torch.randint(-20, 21, (N, 1), generator=g).float()).to(DEV)
+    out = torch.full((M, N + 4), 7.0, device=DEV)
+    a.check(L.mtj_gemm(a.ptr(A), K + 4, a.ptr(W), None, M, N, K, 0, a.EPI_STORE, a.ptr(out), N + 4, 0, None, 1.0, S()))
+    torch.cuda.synchronize()
+    ref = A.double() @ W.double().t()
+    mag = A.double().abs() @ W.double().abs().t()
+    assert bool(((out[:, :N].double() - ref).abs() <= (2.0 ** -23 + 2.0 ** -24 * 6 * K / 16) * mag).all())
+    scaled = (out[:, :N].double() - ref) / (A.double().norm(dim=1)[:, None] * W.double().norm(dim=1)[None])
+    assert float(scaled.pow(2).mean().sqrt()) < 5e-7                       # (a dot product of these norms is about one)
+    assert bool((out[:, N:] == 7.0).all())
+
+
+def test_float32_products_of_numbers_that_are_not_finite(L):
+    """Infinities, NaN and the largest numbers give what plain float32 gives, in their rows and columns only."""
+    a = abi()
+    M, N, K = 130, 140, 64
+    g = torch.Generator().manual_seed(3)
+    A, W = torch.randn(M, K, generator=g).to(DEV), torch.randn(N, K, generator=g).to(DEV)
+    big = float(torch.finfo(torch.float32).max)
+    W[:, 5] = W[:, 5].to(torch.bfloat16).float()              # exact in one part: the others are zero
+    W[7, 5] = 0.0
+    A[3, 5], A[4, 5], A[129, 0], W[9, 2] = float("inf"), -float("inf"), float("nan"), float("inf")
+    A[20], W[20] = 0.0, 0.0
+    A[20, 1], W[20, 1] = big, 1.0                              # rounds to infinity in bfloat16; the product is the number
+    A[21], W[21] = 0.0, 0.0
+    A[21, 1], W[21, 1] = 1.8446743e19, 1.8446743e19            # a product next to the largest number
+    out = torch.empty(M, N, device=DEV)
+    a.check(L.mtj_gemm(a.ptr(A), K, a.ptr(W), None, M, N, K, 0, a.EPI_STORE, a.ptr(out), N, 0, None, 1.0, S()))
+    torch.cuda.synchronize()
+    ref = A.double() @ W.double().t()
+    plain = ref.abs() < 3e38
+    assert torch.equal(out.isnan(), ref.isnan())
+    inf = ref.isinf()
+    assert torch.equal(out[inf].double(), ref[inf])
+    mag = A.double().abs() @ W.double().abs().t()                          # the bound of the test above
+    assert bool(((out[plain].double() - ref[plain]).abs() <= (2.0 ** -23 + 2.0 ** -24 * 6 * K / 16) * mag[plain]).all())
+    assert float(out[20, 20]) == big and float(out[21, 21]) == float(torch.tensor(1.8446743e19) * torch.tensor(1.8446743e19))
+
+
 def test_pack_cvt_holds_bf16_weights_exactly_in_float16_and_alpha_undoes_the_scale(L):
     """The matrix-core path of a bfloat16 model: weights go to float16 times a power of two (exact for every weight
     whose scaled magnitude is a normal float16), the GEMM multiplies the accumulator by the inverse."""
