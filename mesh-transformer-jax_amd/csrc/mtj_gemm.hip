@@ -1,12 +1,12 @@
 // MFMA GEMM for prefill and batched decode: C[M, N] = A[M, K] x W[N, K]^T with fused epilogues.
 // Both operands are K-contiguous and accumulation is float32; bf16 uses v_mfma_f32_32x32x16_bf16, float32 uses
-// v_mfma_f32_32x32x2_f32 (true fp32) up to 64 rows.  Four kernels share the epilogues:
+// v_mfma_f32_32x32x2_f32 (true fp32) up to 32 rows.  Four kernels share the epilogues:
 //   gemm_kernel      any dtype and shape: global -> registers -> LDS (padded rows, so that the 16-byte fragment
 //                    reads of a 32x32 MFMA hit distinct banks), LDS double-buffered;
 //   gemm_dma_kernel  large 16-bit problems: 256x256x64 tiles written straight into LDS by the memory pipeline
 //                    (buffer_load ... lds), rows xor-swizzled instead of padded, no staging registers;
 //   gemm_stream_kernel  16-bit problems of few rows: the same operand path, all rows in one tile, three or four stages;
-//   gemm_split_kernel  float32 problems of more than 64 rows: every operand as a sum of three bf16 numbers.
+//   gemm_split_kernel  float32 problems of more than 32 rows: every operand as a sum of three bf16 numbers.
 #include "mtj_common.h"
 #include <type_traits>
 
@@ -617,8 +617,8 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_split_kernel(const
   constexpr int BM = WAVES_M * WM * 32, BN = WAVES_N * WN * 32;
   constexpr int ROWB = 112, PLANE = 32, STAGEB = (BM + BN) * ROWB;
   constexpr int ROWS_PER_PASS = NT / 2;                    // a thread takes 8 elements of a row at a time
-  constexpr int A_U = BM / ROWS_PER_PASS, B_U = BN / ROWS_PER_PASS;
-  static_assert(BM % ROWS_PER_PASS == 0 && BN % ROWS_PER_PASS == 0, "tile does not divide over threads");
+  constexpr int A_U = (BM + ROWS_PER_PASS - 1) / ROWS_PER_PASS, B_U = (BN + ROWS_PER_PASS - 1) / ROWS_PER_PASS;
+  static_assert((A_U == 1 || BM % ROWS_PER_PASS == 0) && (B_U == 1 || BN % ROWS_PER_PASS == 0), "tile does not divide over threads");
   extern __shared__ __align__(16) unsigned char smem[];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -692,9 +692,11 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_split_kernel(const
     constexpr int st = decltype(ST_)::value;
     unsigned char* d = smem + buf * STAGEB + row0 * ROWB + half * 16;
 #pragma unroll
-    for (int i = 0; i < A_U; ++i) split_store(d + i * ROWS_PER_PASS * ROWB, ra[st][i]);
+    for (int i = 0; i < A_U; ++i)
+      if (BM >= ROWS_PER_PASS || row0 < BM) split_store(d + i * ROWS_PER_PASS * ROWB, ra[st][i]);
 #pragma unroll
-    for (int i = 0; i < B_U; ++i) split_store(d + (BM + i * ROWS_PER_PASS) * ROWB, rb[st][i]);
+    for (int i = 0; i < B_U; ++i)
+      if (BN >= ROWS_PER_PASS || row0 < BN) split_store(d + (BM + i * ROWS_PER_PASS) * ROWB, rb[st][i]);
   };
 
   floatx16 acc[WM][WN];
@@ -1159,9 +1161,9 @@ int launch(const gemm_args& a, hipStream_t s) {
 template <int EPI, int WAVES_M, int WAVES_N, int WM, int WN, int NS>
 int launch_split(const gemm_args& a, hipStream_t s) {
   constexpr int BM = WAVES_M * WM * 32, BN = WAVES_N * WN * 32;
-  constexpr size_t lds = 2 * (size_t)(BM + BN) * 112;
+  constexpr size_t stages = 2 * (size_t)(BM + BN) * 112, patches = 3 * BM * sizeof(int) + WAVES_M * WAVES_N * 32 * 36 * sizeof(float);
+  constexpr size_t lds = stages > patches ? stages : patches;
   static_assert(lds <= 160 * 1024, "tile does not fit LDS");
-  static_assert(lds >= 3 * BM * sizeof(int) + WAVES_M * WAVES_N * 32 * 36 * sizeof(float), "epilogue scratch does not fit");
   static mtj_device_once once;
   if (int rc = mtj_allow_lds(once, "mtj_gemm", &gemm_split_kernel<EPI, WAVES_M, WAVES_N, WM, WN, NS>, lds)) return rc;
   const int tiles = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
@@ -1201,16 +1203,24 @@ int dispatch_tile(const gemm_args& a, hipStream_t s) {
     if (a.M <= 256) return launch_stream<T, EPI, 128, 4>(a, s);
   } else {
     if (a.M <= 32) return launch<T, EPI, 1, 4, 1, 1, BK, 2>(a, s);  // 32 x 128: the weights stream once
-    if (a.M <= 64) return launch<T, EPI, 1, 4, 2, 1, BK, 2>(a, s);  // 64 x 128
+    // The largest tile that fills most of the chip, two workgroups per CU.  us with 128 x 128 / 64 x 128 / 64 x 64 tiles:
+    // N = 28672, K = 4096 64 rows 202 / 155 / 180, 100 rows 218 / 240 / 287; N = 3584, K = 512 60 rows 35 / 25 / 20, 127 rows
+    // 35 / 25 / 20, 300 36 / 26 / 25, 500 36 / 27 / 26, 1000 39 / 37 / 38; N = 512, K = 2560 in four ranges 127 rows 42 / 31 / 26, 500
+    // 43 / 33 / 29, 2000 51 / 53 / 55; N = 4096, K = 20480 64 rows in eight ranges 136 / 105 / 125, 100 in four 223 / 186 / 217.
+    // (33 .. 64 rows took 171, 27 and 116 of these on v_mfma_f32_32x32x2_f32.)  The statistics of XENT are per 128 columns.
+    // Tiles of 64 rows take a sixth longer for a row (199 rows 417 against 349) and win where they leave out more than that:
+    // 64 rows above, 150.
+    const int64_t rows64 = (a.M + 63) / 64, rows128 = (a.M + 127) / 128, cols128 = (a.N + 127) / 128;
+    if (rows128 * cols128 * a.splits >= 200 && 6 * 2 * rows128 <= 7 * rows64) return launch_split<EPI, 2, 2, 2, 2, 3>(a, s);
+    if constexpr (EPI == MTJ_EPI_XENT) return launch_split<EPI, 2, 2, 1, 2, 4>(a, s);
+    else return rows64 * cols128 * a.splits >= 200 ? launch_split<EPI, 2, 2, 1, 2, 4>(a, s) : launch_split<EPI, 2, 2, 1, 1, 3>(a, s);
   }
   if constexpr (sizeof(T) == 2) {
     // e.g. M = 16384, N = 28672 or N = 4096 (a whole 6B layer at 8 x 2048 tokens): 7168 / 1024 tiles
     const int64_t line = EPI == MTJ_EPI_INPROJ && a.K < 768 ? DMA_MIN_TILES_SHORT_INPROJ : DMA_MIN_TILES;
     if (dma_tiles(a.M, a.N) * a.splits >= line) return launch_dma<T, EPI>(a, s);        // 256 x 256, 8 wavefronts of 128 x 64
+    return launch<T, EPI, 2, 2, 2, 2, BK, 2>(a, s);                 // 128 x 128
   }
-  // 128 x 128
-  if constexpr (sizeof(T) == 4) return launch_split<EPI, 2, 2, 2, 2, 3>(a, s);
-  else return launch<T, EPI, 2, 2, 2, 2, BK, 2>(a, s);
 }
 
 template <typename T, int BK>

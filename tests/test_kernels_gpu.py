@@ -152,9 +152,10 @@ def test_gemm_store_and_resid(L, dt, M, N, K):
         assert rel_err(ob, A.double() @ Wh.double()) < TOL[odt] / 2
 
 
-@pytest.mark.parametrize("M,N,K", [(65, 1, 32), (128, 127, 64), (129, 130, 96), (200, 300, 160), (65, 4100, 512), (300, 128, 1024)])
+@pytest.mark.parametrize("M,N,K", [(33, 1, 32), (65, 127, 64), (129, 130, 96), (200, 300, 160), (300, 128, 1024),
+                                   (64, 25600, 32), (65, 25601, 64), (150, 12800, 96), (199, 12804, 160), (256, 12868, 512)])
 def test_float32_products_on_the_bf16_matrix_cores(L, M, N, K):
-    """More than 64 rows of float32: tile edges, K from two k-tiles on, scales up to 2^40.  Bound: what the three left-out
+    """More than 32 rows of float32: the edges of the three tiles, K from two k-tiles on, scales up to 2^40.  Bound: what the three left-out
     products and the representation leave is below 2^-23 of sum |a||w|; the float32 additions (6 K / 16, each of 2^-24 of the
     running sum) add less than 2^-24 (6 K / 16) of it, and sums of random signs are ~sqrt(K) smaller than sum |a||w|."""
     a = abi()
@@ -172,10 +173,11 @@ def test_float32_products_on_the_bf16_matrix_cores(L, M, N, K):
     assert bool((out[:, N:] == 7.0).all())
 
 
-def test_float32_products_of_numbers_that_are_not_finite(L):
+@pytest.mark.parametrize("N", [140, 12801])
+def test_float32_products_of_numbers_that_are_not_finite(L, N):
     """Infinities, NaN and the largest numbers give what plain float32 gives, in their rows and columns only."""
     a = abi()
-    M, N, K = 130, 140, 64
+    M, K = 130, 64
     g = torch.Generator().manual_seed(3)
     A, W = torch.randn(M, K, generator=g).to(DEV), torch.randn(N, K, generator=g).to(DEV)
     big = float(torch.finfo(torch.float32).max)
