@@ -74,6 +74,7 @@ struct gemm_args {
   int64_t ldo;
   int out_dtype;
   float alpha;            // multiplies the accumulator first (undoes a power-of-two scale of the packed weights)
+  int m_base;             // INPROJ: what row 0 is the row of (a call may run as two launches)
   int splits;             // > 1: blockIdx.y owns a K range and stores a raw float32 partial at out + y * split_stride
   int64_t split_stride;
   mtj_inproj ip;
@@ -264,7 +265,7 @@ __device__ __forceinline__ void epilogue(const gemm_args& a, void* out, ACC& acc
       const int m = m0 + r;
       int b = 0, pos = -1, t = 0;
       if (m < a.M) {
-        const int rect = a.ip.rows ? a.ip.rows[m] : m;     // row of the [B, Tp] rectangle
+        const int rect = a.ip.rows ? a.ip.rows[m + a.m_base] : m + a.m_base;     // row of the [B, Tp] rectangle
         b = rect / a.ip.Tp;
         t = rect - b * a.ip.Tp;
         pos = a.ip.pos0[b] + t;
@@ -343,7 +344,7 @@ __device__ __forceinline__ void epilogue(const gemm_args& a, void* out, ACC& acc
         if (c.is_fc) {
 #pragma unroll
           for (int k = 0; k < 16; ++k) val[k] = gelu_tanh(val[k] + cur.o[k >> 2][k & 3]);
-          store16(a.ip.act, (int64_t)m * a.ip.ld_act + d + c.c0, val, a.ip.act_dtype);
+          store16(a.ip.act, (int64_t)(m + a.m_base) * a.ip.ld_act + d + c.c0, val, a.ip.act_dtype);
         } else {
           const int pos = row_pos[r];
           if (pos >= 0) {
@@ -1430,6 +1431,22 @@ int64_t dma_cost(int64_t tiles, int64_t kt, int64_t s) {
   return (tiles * s + 255) / 256 * ((kt + s - 1) / s) * 10 + (s > 1 ? tiles * s * 6 / 5 : 0);
 }
 
+// Rows of a fused input projection that run on 256 x 256 tiles when the rest, the rows of its last row of tiles, is better
+// off as a launch of its own: where that row of tiles starts a round of workgroups of which most CUs have nothing (1.6 us a
+// k-tile), and the rest streams the weights once more in less (gemm_stream_kernel: 5.9, 4.8 and 3.6 TB/s for up to 64, 128 and
+// 256 rows, 4 us for the launch).  0: one launch.  d_model 4096, 520 / 580 / 700 rows 182 / 188 / 199 -> 152 / 156 / 183 us, 1030 / 1200 282 /
+// 300 -> 254 / 280, 2874 610 -> 580, 3400 760 -> 709, 5700 (10 rounds) 1179 -> 1140; 7655 (13) 1490 either way, the rounds have
+// drifted apart by then, so beyond 11 it stays one launch; d_model 2048, 1100 rows 111 -> 91;
+// 1024, 2400 rows 76 -> 64; 512, 4800 rows 54.5 -> 48.9.
+int64_t inproj_front(int64_t M, int64_t N, int64_t K) {
+  const int64_t front = (M - 1) / 256 * 256, rest = M - front;
+  if (dma_tiles(front, N) < (K < 768 ? DMA_MIN_TILES_SHORT_INPROJ : DMA_MIN_TILES)) return 0;
+  const int64_t whole = (dma_tiles(front, N) + 255) / 256, rounds = (dma_tiles(M, N) + 255) / 256 - whole;
+  if (whole > 11) return 0;
+  const double rate = rest <= 64 ? 5.9e6 : rest <= 128 ? 4.8e6 : 3.6e6;                  // bytes per us
+  return (double)rounds * (double)(K / 64) * 1.6 > (double)N * (double)K * 2 / rate + 4.0 ? front : 0;
+}
+
 // How a problem is cut so that its output tiles fill the chip evenly: rows [0, front) in one K range with the epilogue of
 // the product itself, the rows behind them in `splits` K ranges with a reduce.
 struct cut_t { int64_t front; int splits; };
@@ -1566,6 +1583,13 @@ extern "C" int mtj_gemm(const void* A, int64_t lda, const void* W, const float* 
     MTJ_REQUIRE(out && ldo >= N, MTJ_EINVAL, "mtj_gemm: RESID needs out with ldo >= N");
   } else {
     return mtj_fail(MTJ_EINVAL, "mtj_gemm: epilogue %d", epi);
+  }
+  if (const int64_t front = epi == MTJ_EPI_INPROJ && dtype != MTJ_F32 ? inproj_front(M, N, K) : 0) {
+    a.M = (int)front;
+    if (int rc = dispatch_dtype(a, dtype, epi, (hipStream_t)stream)) return rc;
+    a.A = rows_from(A, front * lda, dtype);
+    a.M = (int)(M - front);
+    a.m_base = (int)front;
   }
   return dispatch_dtype(a, dtype, epi, (hipStream_t)stream);
 }

@@ -586,6 +586,14 @@ def test_inproj_gemm_where_its_tiles_change(d, heads, Tp):
     _run_inproj_prefill(cfg, _layer_params(cfg, 9, "bf16"), "bf16", B=2, Tp=Tp, Tcap=Tp + 3, pads=[0, 37], seed=10)
 
 
+@pytest.mark.parametrize("Tp,pads", [(1537, [0, 100, 37]), (1600, [1599, 0, 5])])
+def test_inproj_gemm_whose_last_rows_are_a_launch_of_their_own(Tp, pads):
+    """18 rows of 14 tiles fill a round of workgroups, the next row of tiles would start another: rows from 4608 on (3 and 192
+    of them) take the few-row kernel."""
+    cfg = dict(layers=1, d_model=512, n_heads=8, n_vocab=64, pe="rotary", pe_rotary_dims=32, cores_per_replica=1)
+    _run_inproj_prefill(cfg, _layer_params(cfg, 9, "bf16"), "bf16", B=3, Tp=Tp, Tcap=Tp + 3, pads=pads, seed=10)
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 def test_gemm_resid_and_store_on_the_256x256_direct_to_lds_kernel(L, dt):
     """M = N = 4096 is 256 tiles of 256 x 256, so mtj_gemm itself (no K split) runs gemm_dma_kernel with the RESID and
@@ -852,6 +860,10 @@ def test_inproj_gemm_without_the_rows_of_padding(L, dt, B, Tp, pads):
     for x, y in zip(*got):
         assert torch.equal(x == 1000.0, y == 1000.0)               # what is written and what is not
         assert rel_err(x, y) < (1e-6 if dt == "f32" else 1e-3)
+
+
+def test_inproj_gemm_without_the_rows_of_padding_in_two_launches(L):
+    test_inproj_gemm_without_the_rows_of_padding(L, "bf16", 3, 1600, [0, 100, 37])
 
 
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
