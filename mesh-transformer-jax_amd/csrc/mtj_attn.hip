@@ -420,6 +420,10 @@ __global__ __launch_bounds__(NW * 64) void attn_prefill_kernel(const T* __restri
 // 16-byte chunks of a row are xor-swizzled (K: low four bits of the chunk index with the row, V^T: the two bits with
 // (row / 4) % 4) so that the fragment reads of 16 consecutive rows hit 16 distinct bank groups.  Loads beyond the last
 // tile re-read the last tile (into a stage nobody reads again), which keeps the wait count the same in every iteration.
+// KW 2: two pairs share 32 queries (64 per workgroup), one takes the even key tiles and one the odd ones.  An iteration is two
+// tiles of each operand, two iterations fit the stages: K goes into the place of the iteration two before, requested one
+// iteration ahead, V^T into that of the one before, behind the barrier that its readers have reached.  At the end the
+// second pair hands its accumulator and statistics over through LDS.
 constexpr int PP_STAGES = 4, PP_KTILE = 32 * 256 * 2, PP_VTILE = 256 * 32 * 2;
 constexpr int PP_LDS_K = 0, PP_LDS_V = PP_STAGES * PP_KTILE, PP_LDS_S = PP_LDS_V + PP_STAGES * PP_VTILE;
 constexpr int PP_LDS_A = PP_LDS_S + 4 * 4096, PP_LDS_F = PP_LDS_A + 4 * 512, PP_LDS_BYTES = PP_LDS_F + 64;
@@ -442,7 +446,14 @@ template <> struct psum<bf16_t> {
   }
 };
 
-template <typename T>
+template <int N, int K = 0, class F> __device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (K < N) {
+    f(std::integral_constant<int, K>{});
+    static_for<N, K + 1>(f);
+  }
+}
+
+template <typename T, int KW = 1>
 __global__ __launch_bounds__(512) void attn_prefill_pair_kernel(const T* __restrict__ q, const T* __restrict__ kc,
                                                                 const T* __restrict__ vt, const int32_t* __restrict__ pos0,
                                                                 int H, int Tp, int Tcap, int64_t ldvt, T* __restrict__ out,
@@ -450,18 +461,19 @@ __global__ __launch_bounds__(512) void attn_prefill_pair_kernel(const T* __restr
                                                                 const int32_t* __restrict__ key_limit,
                                                                 const int32_t* __restrict__ skipped) {
   static_assert(sizeof(T) == 2, "16-bit types");
-  constexpr int DH = 256, BKV = 32, BQ = 128, KS = DH / 16, NBLK = DH / 32;
+  constexpr int DH = 256, BKV = 32, BQ = 128 / KW, KS = DH / 16, NBLK = DH / 32;
   extern __shared__ __align__(16) unsigned char smem[];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int pw = wave & 3;                      // which 32 queries of the workgroup
+  const int pw = wave & 3;                      // the pair
+  const int qw = KW == 1 ? pw : pw & 1, kw = KW == 1 ? 0 : pw >> 1;   // which 32 queries of the workgroup, which tile of an iteration
   const bool value_role = wave >= 4;
   const int fr = lane & 31, fg = lane >> 5;
   const int hb = blockIdx.x % (H * nseq), qblk = blockIdx.x / (H * nseq);
   const int h = hb % H, b = hb / H;
   const int qt0 = (nqblk - 1 - qblk) * BQ;      // longest workgroups first
-  const int t = qt0 + pw * 32 + fr;             // this lane's query (rectangle index)
+  const int t = qt0 + qw * 32 + fr;             // this lane's query (rectangle index)
   const int64_t bh = (int64_t)b * H + h;
 
   float* sx = reinterpret_cast<float*>(smem + PP_LDS_S + pw * 4096) + lane * 4;   // + v4 * 256 floats
@@ -515,7 +527,11 @@ __global__ __launch_bounds__(512) void attn_prefill_pair_kernel(const T* __restr
   auto issue_k = [&](int st, int tile) { issue_k1(st, tile, J0{}); issue_k1(st, tile, J1{}); issue_k1(st, tile, J2{}); issue_k1(st, tile, J3{}); };
   auto issue_v = [&](int st, int tile) { issue_v1(st, tile, J0{}); issue_v1(st, tile, J1{}); issue_v1(st, tile, J2{}); issue_v1(st, tile, J3{}); };
   if (value_role) {
-    issue_k(0, 0); issue_v(0, 0); issue_k(1, 1); issue_v(1, 1); issue_k(2, 2);
+    if constexpr (KW == 1) {
+      issue_k(0, 0); issue_v(0, 0); issue_k(1, 1); issue_v(1, 1); issue_k(2, 2);
+    } else {
+      issue_k(0, 0); issue_k(1, 1); issue_k(2, 2); issue_k(3, 3); issue_v(0, 0); issue_v(1, 1);
+    }
   } else {
     const int tq = (t < Tp) ? t : Tp - 1;
     const T* qp = q + (bh * Tp + tq) * DH + fg * 8;
@@ -530,10 +546,11 @@ __global__ __launch_bounds__(512) void attn_prefill_pair_kernel(const T* __restr
   const int last_t = (qt0 + BQ - 1 < Tp - 1) ? qt0 + BQ - 1 : Tp - 1;
   const int kmax = last_t + p0;                 // last key any query of this workgroup may see
   const int klast = Tp - 1 + p0;                // last key position that exists for this sequence
-  const int wave_last = qt0 + pw * 32 + 31 + p0;     // last key this pair may see
-  const int wave_first0 = (qt0 + pw * 32 + 31 < Tp) ? qt0 + pw * 32 + p0 : -1;
+  const int wave_last = qt0 + qw * 32 + 31 + p0;     // last key this pair may see
+  const int wave_first0 = (qt0 + qw * 32 + 31 < Tp) ? qt0 + qw * 32 + p0 : -1;
   const int wave_first = wave_first0 < klim ? wave_first0 : klim;
   const int ntiles = (kmax >= 0) ? kmax / BKV + 1 : 0;
+  const int niter = (ntiles + KW - 1) / KW;     // iteration i: tiles i * KW + kw
 
   if (!value_role) {
     // ---------------- score wavefront
@@ -554,15 +571,15 @@ __global__ __launch_bounds__(512) void attn_prefill_pair_kernel(const T* __restr
         if (ks >= ks_lo && ks < ks_hi) kf[ks] = mma<T>::load(reinterpret_cast<const T*>(kp + kxo[ks & 7] + (ks >> 3) * 256));
     };
     __builtin_amdgcn_s_barrier();               // tile 0 has landed (the value wavefronts waited for it)
-    if (ntiles > 0) read_k(0, 0, 8);
-    for (int i = 0; i <= ntiles; ++i) {
-      const int key0 = i * BKV;
-      const bool active = i < ntiles && key0 <= wave_last;
+    if (ntiles > 0) read_k(kw, 0, 8);
+    for (int i = 0; i <= niter; ++i) {
+      const int tile = i * KW + kw, key0 = tile * BKV;
+      const bool active = tile < ntiles && key0 <= wave_last;
       floatx16 s;
       if (active) {
         // one accumulation chain (dependent MFMAs of one shape issue back to back); the fragments of k-steps 0-7 were
         // fetched in the previous phase, those of k-steps 8-15 arrive under the first eight MFMAs
-        read_k(i, 8, 16);
+        read_k(tile, 8, 16);
         __builtin_amdgcn_sched_barrier(0);
         s = mma<T>::first(kf[0], qf[0]);
 #pragma unroll
@@ -598,8 +615,8 @@ __global__ __launch_bounds__(512) void attn_prefill_pair_kernel(const T* __restr
           *reinterpret_cast<floatx4*>(sx + v4 * 256) = floatx4{s[4 * v4], s[4 * v4 + 1], s[4 * v4 + 2], s[4 * v4 + 3]};
         if (lane == 0) *fx = moved ? 1 : 0;
       }
-      // K tile i+1 has landed (the value wavefronts waited for it before the barrier above)
-      if (i + 1 < ntiles && key0 + BKV <= wave_last) read_k(i + 1, 0, 8);
+      // the next K tile has landed (the value wavefronts waited for it before the barrier above)
+      if (tile + KW < ntiles && key0 + KW * BKV <= wave_last) read_k(tile + KW, 0, 8);
       __builtin_amdgcn_s_barrier();
     }
     return;
@@ -612,18 +629,18 @@ __global__ __launch_bounds__(512) void attn_prefill_pair_kernel(const T* __restr
 #pragma unroll
     for (int v = 0; v < 16; ++v) o[i][v] = 0.f;
   float lrun = 0.f, mneg = 0.f;
-  __builtin_amdgcn_s_waitcnt(wait_vmcnt(12));               // tile 0 of K and V^T
+  __builtin_amdgcn_s_waitcnt(wait_vmcnt(KW == 1 ? 12 : 16));   // tile 0 of K and V^T; the first two K tiles
   __builtin_amdgcn_s_barrier();
 
   const int vx = (fr >> 2) & 3;
   const unsigned char* vbase = smem + PP_LDS_V + fr * 64;
   const int vpos0 = ((0 + fg) ^ vx) * 16, vpos1 = ((2 + fg) ^ vx) * 16;
   const int last = ntiles > 0 ? ntiles - 1 : 0;
-  for (int i = 0; i <= ntiles; ++i) {
+  for (int i = 0; i <= niter; ++i) {
     // ---- phase 1: the probabilities of tile i-1 and its V^T fragments
     const int tk3 = i + 3 < last ? i + 3 : last, tv2 = i + 2 < last ? i + 2 : last;   // the tiles requested in phase 2
-    const int tv = i - 1;
-    const bool active = tv >= 0 && tv * BKV <= wave_last;
+    const int tv = (i - 1) * KW + kw;
+    const bool active = i > 0 && tv < ntiles && tv * BKV <= wave_last;
     typename mma<T>::frag pf[2], vf[2][NBLK];
     if (active) {
       const unsigned char* vp = vbase + (tv & (PP_STAGES - 1)) * PP_VTILE;
@@ -665,13 +682,35 @@ __global__ __launch_bounds__(512) void attn_prefill_pair_kernel(const T* __restr
       float lt = psum<T>::run(pf[1], psum<T>::run(pf[0], 0.f));
       lrun += sum_halves(lt);
     }
-    __builtin_amdgcn_s_waitcnt(wait_vmcnt(8));              // K of tile i+1 and V^T of tile i have landed
+    // KW 1: K of tile i+1 and V^T of tile i have landed.  KW 2: K of the next iteration has, and this iteration's V^T has been
+    // read: the requests of phase 2 go into its place
+    __builtin_amdgcn_s_waitcnt(KW == 1 ? wait_vmcnt(8) : wait_vmcnt(8) & wait_lgkmcnt(0));
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     // ---- phase 2: O^T += V^T P^T, and the requests for K tile i+3 and V^T tile i+2 (their stages were last read in
     // iteration i-1), one per two MFMAs.  (Issued by the score wavefronts instead, whose second phase is the longer
     // one, the kernel is 5 % slower.)
+    if constexpr (KW == 2) {
+      // K of iteration i+2 into the place of this one's, V^T of iteration i+1 into that of the last one's
+      const int tk0 = 2 * i + 4 < last ? 2 * i + 4 : last, tk1 = 2 * i + 5 < last ? 2 * i + 5 : last;
+      if (active) {
+        static_for<8>([&](auto N_) {
+          constexpr int n = decltype(N_)::value;
+          mma<T>::run(o[(2 * n) & 7], vf[n >> 2][(2 * n) & 7], pf[n >> 2]);
+          mma<T>::run(o[(2 * n + 1) & 7], vf[n >> 2][(2 * n + 1) & 7], pf[n >> 2]);
+          __builtin_amdgcn_sched_barrier(0);
+          issue_k1(2 * i + (n >> 2), n >> 2 ? tk1 : tk0, std::integral_constant<int, n & 3>{});
+          __builtin_amdgcn_sched_barrier(0);
+        });
+      } else {
+        issue_k(2 * i, tk0);
+        issue_k(2 * i + 1, tk1);
+      }
+      issue_v(2 * i + 2, 2 * i + 2 < last ? 2 * i + 2 : last);
+      issue_v(2 * i + 3, 2 * i + 3 < last ? 2 * i + 3 : last);
+      __builtin_amdgcn_s_waitcnt(wait_vmcnt(16));             // V^T of this iteration has landed
+    } else {
     if (active) {
       mma<T>::run(o[0], vf[0][0], pf[0]); mma<T>::run(o[1], vf[0][1], pf[0]);
       __builtin_amdgcn_sched_barrier(0); issue_k1(i + 3, tk3, J0{}); __builtin_amdgcn_sched_barrier(0);
@@ -693,11 +732,37 @@ __global__ __launch_bounds__(512) void attn_prefill_pair_kernel(const T* __restr
       issue_k(i + 3, tk3);
       issue_v(i + 2, tv2);
     }
+    }
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
   }
   __builtin_amdgcn_s_waitcnt(wait_vmcnt(0));                // the surplus loads land before the LDS is given away
+
+  if constexpr (KW == 2) {
+    // the two halves of the keys: the wavefronts of the odd tiles hand over (one float per lane and register: 32 KiB each)
+    float* mine = reinterpret_cast<float*>(smem) + qw * (NBLK * 16 * 64) + lane;
+    float* stat = reinterpret_cast<float*>(smem + PP_LDS_S) + qw * 128 + lane;
+    __builtin_amdgcn_s_barrier();                           // every wavefront's loads have landed
+    if (kw == 1) {
+#pragma unroll
+      for (int n = 0; n < NBLK; ++n)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) mine[(n * 16 + v) * 64] = o[n][v];
+      stat[0] = mneg;
+      stat[64] = lrun;
+    }
+    __syncthreads();
+    if (kw == 1) return;
+    const float l1 = stat[64], m0 = lrun > 0.f ? -mneg : -INFINITY, m1 = l1 > 0.f ? -stat[0] : -INFINITY;
+    const float m = fmaxf(m0, m1);
+    const float f0 = m0 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m0 - m), f1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - m);
+    lrun = f0 * lrun + f1 * l1;
+#pragma unroll
+    for (int n = 0; n < NBLK; ++n)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) o[n][v] = f0 * o[n][v] + f1 * mine[(n * 16 + v) * 64];   // (0 x NaN stays NaN)
+  }
 
   // ---- write O: register v of block n is head-dim n*32 + 8*(v/4) + 4*fg + v%4 of query t
   const out_rows rows(b, Tp, p0, skipped);
@@ -769,14 +834,6 @@ template <> __device__ __forceinline__ uint32_t pack_prob<f16_t>(float lo, float
   return __builtin_bit_cast(uint32_t, r);
 }
 // f(integral_constant<int, K>) for K = 0 .. N-1, in order
-template <int N, int K = 0, class F> __device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (K < N) {
-    f(std::integral_constant<int, K>{});
-    static_for<N, K + 1>(f);
-  }
-}
-
-
 template <typename T>
 __global__ __launch_bounds__(256) void attn_prefill_q64_kernel(const T* __restrict__ q, const T* __restrict__ kc,
                                                                const T* __restrict__ vt, const int32_t* __restrict__ pos0,
@@ -1409,15 +1466,15 @@ int attn_prefill_impl(const void* q, const void* k_cache, const void* v_t, const
         (const T*)q, (const T*)k_cache, (const T*)v_t, pos0, (int)H, (int)Tp, (int)Tcap, ldvt, (T*)out, ld_out,      \
         (int)B, (int)nqblk, key_limit, skipped);                                                                              \
   } while (0)
-#define MTJ_PREFILL_PAIR(T)                                                                                          \
+#define MTJ_PREFILL_PAIR(T, KW)                                                                                      \
   do {                                                                                                               \
     static_assert(PP_LDS_BYTES <= 160 * 1024, "attention tiles do not fit LDS");                                     \
     static mtj_device_once once;                                                                                     \
-    if (int rc = mtj_allow_lds(once, "mtj_attn_prefill", &attn_prefill_pair_kernel<T>, PP_LDS_BYTES)) return rc;     \
-    const int64_t nqblk = (Tp + 127) / 128;                                                                          \
+    if (int rc = mtj_allow_lds(once, "mtj_attn_prefill", (&attn_prefill_pair_kernel<T, KW>), PP_LDS_BYTES)) return rc; \
+    const int64_t nqblk = (Tp + 128 / KW - 1) / (128 / KW);                                                          \
     MTJ_REQUIRE(nqblk * H * B < (1ll << 31), MTJ_ELIMIT, "mtj_attn_prefill: too many workgroups");                    \
     MTJ_REQUIRE(Tcap * 512 < (1ll << 31) && 512 * ldvt < (1ll << 31), MTJ_ELIMIT, "mtj_attn_prefill: window too long"); \
-    attn_prefill_pair_kernel<T><<<(unsigned)(nqblk * H * B), 512, PP_LDS_BYTES, s>>>(                                 \
+    attn_prefill_pair_kernel<T, KW><<<(unsigned)(nqblk * H * B), 512, PP_LDS_BYTES, s>>>(                                 \
         (const T*)q, (const T*)k_cache, (const T*)v_t, pos0, (int)H, (int)Tp, (int)Tcap, ldvt, (T*)out, ld_out,      \
         (int)B, (int)nqblk, key_limit, skipped);                                                                     \
   } while (0)
@@ -1437,11 +1494,18 @@ int attn_prefill_impl(const void* q, const void* k_cache, const void* v_t, const
   // 472 us against 529 for 8 sequences, 796 against 1069 for 16, but 225 against 208 for 4); shorter problems keep the
   // 128-query workgroups
   const bool q64 = dh == 256 && B * H * ((Tp + 255) / 256) >= 1024;
+  // Few workgroups (one per CU): the longest walks over all keys while most of the chip has ended or had nothing, so the keys
+  // are shared by two pairs of wavefronts.  16 heads, us: 300 tokens 20.9 -> 19.2, 511 24.3 -> 20.2, 1023 39.7 -> 31.5, 1500 (192
+  // workgroups) 54.6 -> 43.8, 2 x 500 27.0 -> 23.6, 3 x 300 22.0 -> 20.9; beyond, 2 x 1023 (256) 42.1 against 43.7, 8 x 300 31
+  // against 40; with two tiles there is nothing to share: 4 x 61 10.2 against 11.8.
+  const bool two = Tp > 64 && B * H * ((Tp + 127) / 128) <= 192;
   if (dtype == MTJ_BF16 && q64) MTJ_PREFILL_Q64(bf16_t);
   else if (dtype == MTJ_F16 && q64) MTJ_PREFILL_Q64(f16_t);
-  else if (dtype == MTJ_BF16 && dh == 256) MTJ_PREFILL_PAIR(bf16_t);
+  else if (dtype == MTJ_BF16 && dh == 256 && two) MTJ_PREFILL_PAIR(bf16_t, 2);
+  else if (dtype == MTJ_BF16 && dh == 256) MTJ_PREFILL_PAIR(bf16_t, 1);
   else if (dtype == MTJ_BF16 && dh == 64) MTJ_PREFILL(bf16_t, 64, 8, 64);
-  else if (dtype == MTJ_F16 && dh == 256) MTJ_PREFILL_PAIR(f16_t);
+  else if (dtype == MTJ_F16 && dh == 256 && two) MTJ_PREFILL_PAIR(f16_t, 2);
+  else if (dtype == MTJ_F16 && dh == 256) MTJ_PREFILL_PAIR(f16_t, 1);
   else if (dtype == MTJ_F16 && dh == 64) MTJ_PREFILL(f16_t, 64, 8, 64);
   else if (dtype == MTJ_F32 && dh == 256) MTJ_PREFILL(float, 256, 4, 32);
   else if (dtype == MTJ_F32 && dh == 64) MTJ_PREFILL(float, 64, 4, 32);

@@ -801,6 +801,34 @@ def test_attn_prefill(L, dt, dh, H, Tp):
             assert rel_err(out[b * Tp:(b + 1) * Tp, :H * dh], ref) < ATT_TOL[dt], (dt, dh, Tp, b)
 
 
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("H,Tp", [(2, 65), (2, 96), (2, 97), (1, 129), (2, 161), (1, 511), (2, 1023), (50, 129), (49, 250)])
+def test_attn_prefill_with_the_keys_shared_by_two_pairs(L, dt, H, Tp):
+    """d_head 256 and up to 192 workgroups of 128 queries (200 and 196 for the last two): odd and even tile counts, queries
+    whose second pair has no tile, a partial last tile in either."""
+    test_attn_prefill(L, dt, 256, H, Tp)
+
+
+def test_attn_prefill_of_infinite_and_nan_values_with_the_keys_shared_by_two_pairs(L):
+    """A NaN or infinite value reaches the queries that may see its key, whichever pair holds it, and no other (bfloat16: a float16
+    result saturates)."""
+    a = abi()
+    B, H, Tp, dh = 1, 1, 200, 256
+    for key, bad in ((10, float("nan")), (40, float("nan")), (70, float("inf"))):
+        g = torch.Generator().manual_seed(key)
+        q, kc = (torch.randn(B, H, Tp, dh, generator=g).bfloat16().to(DEV) for _ in range(2))
+        vt = torch.zeros(B, H, dh, 256, dtype=torch.bfloat16, device=DEV)
+        vt[..., :Tp] = torch.randn(B, H, dh, Tp, generator=g).bfloat16().to(DEV)
+        vt[0, 0, 3, key] = bad
+        pos0 = torch.zeros(1, dtype=torch.int32, device=DEV)
+        out = torch.zeros(Tp, dh, dtype=torch.bfloat16, device=DEV)
+        a.check(L.mtj_attn_prefill(a.ptr(q), a.ptr(kc), a.ptr(vt), a.ptr(pos0), B, H, Tp, Tp, dh, 256, a.ptr(out), dh, 1, None, S()))
+        torch.cuda.synchronize()
+        # key tiles are 32 keys, walked as a whole up to the tile of the query block: 0 x NaN below the diagonal of its own tile
+        assert bool((~out[key:, 3].isfinite()).all()) and bool(out[:key // 32 * 32].isfinite().all())
+        assert bool(out[:, 4:].isfinite().all())
+
+
 @pytest.mark.parametrize("dt,dh,H,pads,Tp", [
     ("f32", 64, 3, [0, 5, 40], 41), ("f32", 256, 2, [7, 0], 33), ("f16", 64, 2, [299, 0, 301], 301), ("bf16", 64, 2, [0, 1], 64),
     ("f16", 256, 2, [0, 129, 199, 13], 200), ("bf16", 256, 1, [1, 0], 2),
