@@ -133,44 +133,60 @@ extern "C" int mtj_embed(const int32_t* tok, int64_t M, const void* W, const flo
   return mtj_check_launch("mtj_embed");
 }
 
-// ---------------------------------------------------------------- LayerNorm: one wavefront per row
+// ---------------------------------------------------------------- LayerNorm
 // Two passes over a row that stays in registers (mean first, then centred variance, as the reference
 // computes jnp.var); all statistics float32.
-#define LN_MAX_PER_LANE 64  // floats per lane: d <= 64 lanes * 64 = 4096
+constexpr int LN_MAX = 4096;         // columns
 
-template <int OUT_DTYPE>
+// WG false: a wavefront per row, four rows per workgroup (up to 1024 columns); WG true: a workgroup of four wavefronts per row.
+// Four float4 per lane either way.  Bound by memory: what matters is that a CU has other rows in flight while one is reduced,
+// and for a few rows that a row is asked for at once.  With a wavefront per row of 4096 columns (64 registers for the row, 16
+// loads one behind the other) 3 rows took 7.4 us, now 4.3; 511 10.3 -> 5.6, 2872 21.2 -> 16.8, 32736 214 -> 156 (5.2 TB/s); 50000
+// rows of 512 columns 54 -> 29, 2000 of 2048 8.2 -> 6.9.
+template <int OUT_DTYPE, bool WG>
 __global__ __launch_bounds__(256) void layernorm_kernel(const float* __restrict__ x, const float* __restrict__ scale,
                                                         const float* __restrict__ offset, int64_t M, int d,
                                                         void* __restrict__ out) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  constexpr int NT = WG ? 256 : 64, V = 4;
+  __shared__ float red[2][4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, at = WG ? threadIdx.x : lane;
+  const int64_t row = WG ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + wave;
   if (row >= M) return;
   const float* xr = x + row * d;
   const int nvec = d >> 2;  // float4 chunks
-  floatx4 v[LN_MAX_PER_LANE / 4];
+  auto row_sum = [&](float s, int which) {
+    s = wave_sum(s);
+    if constexpr (WG) {
+      if (lane == 0) red[which][wave] = s;
+      __syncthreads();
+      s = (red[which][0] + red[which][1]) + (red[which][2] + red[which][3]);
+    }
+    return s;
+  };
+  floatx4 v[V];
   float sum = 0.f;
 #pragma unroll
-  for (int i = 0; i < LN_MAX_PER_LANE / 4; ++i) {
-    const int c = i * 64 + lane;
+  for (int i = 0; i < V; ++i) {
+    const int c = i * NT + at;
     if (c < nvec) {
       v[i] = *reinterpret_cast<const floatx4*>(xr + 4 * c);
       sum += (v[i].x + v[i].y) + (v[i].z + v[i].w);
     }
   }
-  const float mean = wave_sum(sum) / (float)d;
+  const float mean = row_sum(sum, 0) / (float)d;
   float sq = 0.f;
 #pragma unroll
-  for (int i = 0; i < LN_MAX_PER_LANE / 4; ++i) {
-    const int c = i * 64 + lane;
+  for (int i = 0; i < V; ++i) {
+    const int c = i * NT + at;
     if (c < nvec) {
       const floatx4 t = v[i] - mean;
       sq += (t.x * t.x + t.y * t.y) + (t.z * t.z + t.w * t.w);
     }
   }
-  const float inv = rsqrtf(wave_sum(sq) / (float)d + 1e-5f);
+  const float inv = rsqrtf(row_sum(sq, 1) / (float)d + 1e-5f);
 #pragma unroll
-  for (int i = 0; i < LN_MAX_PER_LANE / 4; ++i) {
-    const int c = i * 64 + lane;
+  for (int i = 0; i < V; ++i) {
+    const int c = i * NT + at;
     if (c < nvec) {
       const floatx4 sc = *reinterpret_cast<const floatx4*>(scale + 4 * c);
       const floatx4 of = *reinterpret_cast<const floatx4*>(offset + 4 * c);
@@ -189,21 +205,23 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const float* __restrict_
   }
 }
 
+template <int OUT_DTYPE>
+void launch_layernorm(const float* x, const float* scale, const float* offset, int64_t M, int d, void* out, hipStream_t s) {
+  if (d <= 1024) layernorm_kernel<OUT_DTYPE, false><<<(unsigned)((M + 3) / 4), 256, 0, s>>>(x, scale, offset, M, d, out);
+  else layernorm_kernel<OUT_DTYPE, true><<<(unsigned)M, 256, 0, s>>>(x, scale, offset, M, d, out);
+}
+
 extern "C" int mtj_layernorm(const float* x, const float* scale, const float* offset, int64_t M, int64_t d,
                              void* out, int out_dtype, void* stream) {
   MTJ_REQUIRE(x && scale && offset && out, MTJ_EINVAL, "mtj_layernorm: null pointer");
-  MTJ_REQUIRE(M > 0 && d > 0 && d % 4 == 0 && d <= 64 * LN_MAX_PER_LANE, MTJ_EINVAL,
-              "mtj_layernorm: d=%lld must be a multiple of 4 and <= %d", (long long)d, 64 * LN_MAX_PER_LANE);
+  MTJ_REQUIRE(M > 0 && d > 0 && d % 4 == 0 && d <= LN_MAX, MTJ_EINVAL,
+              "mtj_layernorm: d=%lld must be a multiple of 4 and <= %d", (long long)d, LN_MAX);
   MTJ_REQUIRE(mtj_aligned16(x) && mtj_aligned16(scale) && mtj_aligned16(offset) && mtj_aligned16(out), MTJ_EALIGN,
               "mtj_layernorm: pointers must be 16-byte aligned");
   hipStream_t s = (hipStream_t)stream;
-  const unsigned grid = (unsigned)((M + 3) / 4);
-  if (out_dtype == MTJ_F32)
-    layernorm_kernel<MTJ_F32><<<grid, 256, 0, s>>>(x, scale, offset, M, (int)d, out);
-  else if (out_dtype == MTJ_BF16)
-    layernorm_kernel<MTJ_BF16><<<grid, 256, 0, s>>>(x, scale, offset, M, (int)d, out);
-  else if (out_dtype == MTJ_F16)
-    layernorm_kernel<MTJ_F16><<<grid, 256, 0, s>>>(x, scale, offset, M, (int)d, out);
+  if (out_dtype == MTJ_F32) launch_layernorm<MTJ_F32>(x, scale, offset, M, (int)d, out, s);
+  else if (out_dtype == MTJ_BF16) launch_layernorm<MTJ_BF16>(x, scale, offset, M, (int)d, out, s);
+  else if (out_dtype == MTJ_F16) launch_layernorm<MTJ_F16>(x, scale, offset, M, (int)d, out, s);
   else
     return mtj_fail(MTJ_EDTYPE, "mtj_layernorm: out_dtype %d", out_dtype);
   return mtj_check_launch("mtj_layernorm");

@@ -102,6 +102,23 @@ def test_layernorm(L, d, out_dt):
     assert torch.equal(o2[0], of)
 
 
+@pytest.mark.parametrize("d,M", [(4, 7), (1020, 5), (1024, 1), (1028, 3), (2052, 2), (4092, 9), (4096, 1)])
+def test_layernorm_rows_of_a_wavefront_and_of_a_workgroup(L, d, M):
+    """Up to 1024 columns a wavefront takes a row, beyond that a workgroup; a large mean, and rows in place."""
+    a = abi()
+    g = torch.Generator().manual_seed(d + M)
+    x = (torch.randn(M, d, generator=g) + 50.0).to(DEV)
+    sc, of = (torch.randn(d, generator=g).to(DEV) for _ in range(2))
+    ref = O.replicated_layer_norm(x.double().cpu(), sc.double().cpu(), of.double().cpu())
+    out = torch.full((M + 1, d), 7.0, device=DEV)
+    a.check(L.mtj_layernorm(a.ptr(x), a.ptr(sc), a.ptr(of), M, d, a.ptr(out), 0, S()))
+    a.check(L.mtj_layernorm(a.ptr(x), a.ptr(sc), a.ptr(of), M, d, a.ptr(x), 0, S()))
+    torch.cuda.synchronize()
+    # float32 of a value near 50 with deviation 1: 50 * 2^-24 each, and the mean rounded once more
+    assert rel_err(out[:M], ref) < 2 * 50 * 2.0 ** -24
+    assert torch.equal(x, out[:M]) and bool((out[M] == 7.0).all())
+
+
 def test_layernorm_rejects_bad_shapes(L):
     a = abi()
     x = torch.zeros(2, 6, device=DEV)
