@@ -1502,9 +1502,12 @@ cut_t pick_cut(int64_t M, int64_t N, int64_t K, int dtype) {
       return {0, 1};
     }
   }
-  // 128 x 128 tiles, two workgroups per CU: up to 4 ranges
+  // 128 x 128 tiles, two workgroups per CU: up to 4 ranges, for float32, whose k-tiles take longer than the partials they cost, up
+  // to 16 (N = 4096, K = 20480, 4 / 8 / 16 at most: 65 rows 214 / 165 / 150 us, 128 rows 198 / 163 / 152, 199 274 / 253 / 250; N =
+  // 1024, K = 5120, 100 rows 44 / 27 / 27)
+  const int most = dtype == MTJ_F32 ? 16 : 4;
   const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
-  while (splits < 4 && tiles * splits * 2 <= 512 && kt % (splits * 2) == 0 && kt / (splits * 2) >= 16) splits *= 2;
+  while (splits < most && tiles * splits * 2 <= 512 && kt % (splits * 2) == 0 && kt / (splits * 2) >= 16) splits *= 2;
   return {0, splits};
 }
 
