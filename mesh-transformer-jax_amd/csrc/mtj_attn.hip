@@ -404,6 +404,175 @@ __global__ __launch_bounds__(NW * 64) void attn_prefill_kernel(const T* __restri
 }
 
 // ------------------------------------------------------------------------------------------------
+// float32 prefill: the mathematics and lane layout of attn_prefill_kernel, but the four wavefronts of a
+// workgroup share 32 queries and take every fourth key tile, and meet through LDS at the end.  A tile is 16384 cycles of
+// v_mfma_f32_32x32x2_f32 at d_head 256, so what bounds a short prompt is the wavefront with the most tiles, on a chip most of
+// which is idle.  No tile is used by two wavefronts: the fragments come straight from memory, a step ahead of their use.
+// 16 heads of 256, us, against attn_prefill_kernel with 128 queries per workgroup and its tiles in LDS: 100 tokens 47 -> 17, 199 73
+// -> 26, 511 157 -> 44, 1000 309 -> 96, 4 x 511 164 -> 115, 8 x 1024 771 -> 748; 8 heads of 64: 127 tokens 14.6 -> 6.6, 1499 124 -> 47.
+// The error is a little smaller too (four shorter sums): 511 tokens 4.4e-7 -> 4.1e-7.
+template <int DH>
+__global__ __launch_bounds__(256) void attn_prefill_f32_kernel(const float* __restrict__ q, const float* __restrict__ kc,
+                                                               const float* __restrict__ vt, const int32_t* __restrict__ pos0,
+                                                               int H, int Tp, int Tcap, int64_t ldvt, float* __restrict__ out,
+                                                               int64_t ld_out, int nseq, int nqblk,
+                                                               const int32_t* __restrict__ key_limit,
+                                                               const int32_t* __restrict__ skipped) {
+  using M = mma<float>;
+  constexpr int BQ = 32, BKV = 32, NW = 4, KS = DH / 16, NBLK = DH / 32, HB = NBLK > 4 ? 4 : NBLK;
+  extern __shared__ __align__(16) unsigned char smem[];      // [NW][NBLK * 16][64] accumulators, [NW][2][64] statistics
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int fr = lane & 31, fg = lane >> 5;
+  const int hb = blockIdx.x % (H * nseq), qblk = blockIdx.x / (H * nseq);
+  const int h = hb % H, b = hb / H;
+  const int qt0 = (nqblk - 1 - qblk) * BQ;      // longest workgroups first
+  const int p0 = pos0[b];                       // <= 0: minus the number of padding rows
+  const int t = qt0 + fr;                       // this lane's query (rectangle index)
+  const int qpos = (t < Tp) ? t + p0 : -1;      // its position; < 0 = padding / out of range
+  const int klim = key_limit ? key_limit[b] : 0x7fffffff;
+  const int qsee = qpos < klim ? qpos : klim;   // last key this query may see
+  const int kmax = ((qt0 + BQ - 1 < Tp - 1) ? qt0 + BQ - 1 : Tp - 1) + p0;
+  const int klast = Tp - 1 + p0;                // last key position that exists for this sequence
+  const int64_t bh = (int64_t)b * H + h;
+
+  M::frag qf[KS];
+  {
+    const float* qp = q + (bh * Tp + (t < Tp ? t : Tp - 1)) * DH + fg * 8;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = M::load(qp + ks * 16);
+  }
+  const int krow = 16 * (fr >> 4) + 8 * ((fr >> 2) & 1) + 4 * ((fr >> 3) & 1) + (fr & 3);
+  floatx16 o[NBLK];
+#pragma unroll
+  for (int i = 0; i < NBLK; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) o[i][v] = 0.f;
+  float mrun = -INFINITY, lrun = 0.f;           // running max (log2 units) and sum
+  const float sc2 = rsqrtf((float)DH) * 1.4426950408889634f;   // 1/sqrt(dh) * log2(e)
+
+  const int ntiles = (kmax >= 0) ? kmax / BKV + 1 : 0;
+  for (int kt = wave; kt < ntiles; kt += NW) {
+    const int key0 = kt * BKV;
+    // K rows beyond the last key are clamped to it (the mask removes them)
+    const float* kp = kc + (bh * Tcap + (key0 + krow <= klast ? key0 + krow : klast)) * DH + fg * 8;
+    const float* vp = vt + (bh * DH + fr) * ldvt + key0 + fg * 8;
+    floatx16 s;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) s[v] = 0.f;
+    M::frag vf[2][HB];
+    {
+      constexpr int G = 2;
+      M::frag kf[2][G];
+#pragma unroll
+      for (int g = 0; g < G; ++g) kf[0][g] = M::load(kp + g * 16);
+#pragma unroll
+      for (int k0 = 0; k0 < KS; k0 += G) {
+        const int cur = (k0 / G) & 1, nxt = cur ^ 1;
+        if (k0 + G < KS) {
+#pragma unroll
+          for (int g = 0; g < G; ++g) kf[nxt][g] = M::load(kp + (k0 + G + g) * 16);
+        } else {                                 // the first V^T fragments travel under the last scores and the softmax
+#pragma unroll
+          for (int i = 0; i < HB; ++i) vf[0][i] = M::load(vp + (int64_t)i * 32 * ldvt);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int g = 0; g < G; ++g) M::run(s, kf[cur][g], qf[k0 + g]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    // register v is key key0 + 16*(v/8) + 8*fg + v%8
+    float mt = -INFINITY;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int key = key0 + 16 * (v / 8) + 8 * fg + (v % 8);
+      s[v] = (key <= qsee) ? s[v] * sc2 : -INFINITY;
+      mt = fmaxf(mt, s[v]);
+    }
+    mt = fmaxf(mt, __shfl_xor(mt, 32));
+    if (__any(mt > mrun + 6.0f)) {               // see attn_prefill_kernel
+      const float mnew = fmaxf(mrun, mt);
+      const float alpha = (mnew == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(mrun - mnew);   // mrun = -inf -> 0
+      lrun *= alpha;
+#pragma unroll
+      for (int i = 0; i < NBLK; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[i][v] *= alpha;
+      mrun = mnew;
+    }
+    const float msafe = (mrun == -INFINITY) ? 0.f : mrun;
+    float lt = 0.f, p[16];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      p[v] = __builtin_amdgcn_exp2f(s[v] - msafe);          // masked -> exp2(-inf) = 0
+      lt += p[v];
+    }
+    lt += __shfl_xor(lt, 32);
+    lrun += lt;
+    const M::frag pf[2] = {M::from_floats(p), M::from_floats(p + 8)};
+    const bool partial = key0 + BKV - 1 > klast; // what V^T holds beyond the last key must not reach the product
+    // step n: blocks HB * (n / 2) .. of the head dim, keys 16 * (n % 2) .. of the tile
+    constexpr int STEPS = 2 * (NBLK / HB);
+#pragma unroll
+    for (int n = 0; n < STEPS; ++n) {
+      const int cur = n & 1, nxt = cur ^ 1;
+      if (n + 1 < STEPS) {
+#pragma unroll
+        for (int i = 0; i < HB; ++i) vf[nxt][i] = M::load(vp + (int64_t)(HB * ((n + 1) / 2) + i) * 32 * ldvt + 16 * ((n + 1) % 2));
+      }
+      if (partial) {
+#pragma unroll
+        for (int i = 0; i < HB; ++i)
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            if (key0 + 16 * (n % 2) + 8 * fg + j > klast) vf[cur][i].v[j] = 0.f;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < HB; ++i) M::run(o[HB * (n / 2) + i], vf[cur][i], pf[n % 2]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+
+  // ---- the four wavefronts meet; wavefront w finishes blocks w, w + 4, ..
+  float* acc = reinterpret_cast<float*>(smem);
+  float* stat = acc + NW * NBLK * 16 * 64;
+#pragma unroll
+  for (int i = 0; i < NBLK; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[((wave * NBLK + i) * 16 + v) * 64 + lane] = o[i][v];
+  stat[wave * 128 + lane] = mrun;
+  stat[wave * 128 + 64 + lane] = lrun;
+  __syncthreads();
+  float m[NW], f[NW], mm = -INFINITY, l = 0.f;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    m[w] = stat[w * 128 + lane];
+    mm = fmaxf(mm, m[w]);
+  }
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    f[w] = m[w] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[w] - mm);
+    l = fmaf(f[w], stat[w * 128 + 64 + lane], l);
+  }
+  const out_rows rows(b, Tp, p0, skipped);
+  if (t < rows.first || t >= Tp) return;
+  const float inv = (qpos >= 0 && l > 0.f) ? 1.0f / l : 0.f;
+  float* op = out + (rows.base + t) * ld_out + (int64_t)h * DH;
+  for (int i = wave; i < NBLK; i += NW)
+#pragma unroll
+    for (int v4 = 0; v4 < 4; ++v4) {
+      floatx4 r = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < NW; ++w)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[e] = fmaf(f[w], acc[((w * NBLK + i) * 16 + v4 * 4 + e) * 64 + lane], r[e]);   // (0 x NaN stays NaN)
+      *reinterpret_cast<floatx4*>(op + i * 32 + 8 * v4 + 4 * fg) = r * inv;
+    }
+}
+
+// ------------------------------------------------------------------------------------------------
 // Prefill for 16-bit types at d_head 256: the same mathematics and the same lane layout as attn_prefill_kernel (one
 // lane owns one query, S^T = K Q^T, O^T = V^T P^T, K rows permuted so that the scores land in the operand layout of the
 // second product), but each block of 32 queries is worked on by a PAIR of wavefronts that share a SIMD (wave w and
@@ -1490,6 +1659,17 @@ int attn_prefill_impl(const void* q, const void* k_cache, const void* v_t, const
         (const T*)q, (const T*)k_cache, (const T*)v_t, pos0, (int)H, (int)Tp, (int)Tcap, ldvt, (T*)out, ld_out,      \
         (int)B, (int)nqblk, key_limit, skipped);                                                                     \
   } while (0)
+#define MTJ_PREFILL_F32(DH)                                                                                          \
+  do {                                                                                                               \
+    constexpr size_t lds = (4 * (DH / 32) * 16 * 64 + 4 * 128) * sizeof(float);                                      \
+    static mtj_device_once once;                                                                                     \
+    if (int rc = mtj_allow_lds(once, "mtj_attn_prefill", &attn_prefill_f32_kernel<DH>, lds)) return rc;              \
+    const int64_t nqblk = (Tp + 31) / 32;                                                                            \
+    MTJ_REQUIRE(nqblk * H * B < (1ll << 31), MTJ_ELIMIT, "mtj_attn_prefill: too many workgroups");                    \
+    attn_prefill_f32_kernel<DH><<<(unsigned)(nqblk * H * B), 256, lds, s>>>(                                          \
+        (const float*)q, (const float*)k_cache, (const float*)v_t, pos0, (int)H, (int)Tp, (int)Tcap, ldvt, (float*)out, ld_out, \
+        (int)B, (int)nqblk, key_limit, skipped);                                                                     \
+  } while (0)
   // 256-query blocks, two per workgroup, when that still makes two workgroups per CU (measured on 16 heads x 2048 tokens:
   // 472 us against 529 for 8 sequences, 796 against 1069 for 16, but 225 against 208 for 4); shorter problems keep the
   // 128-query workgroups
@@ -1498,6 +1678,10 @@ int attn_prefill_impl(const void* q, const void* k_cache, const void* v_t, const
   // are shared by two pairs of wavefronts.  16 heads, us: 300 tokens 20.9 -> 19.2, 511 24.3 -> 20.2, 1023 39.7 -> 31.5, 1500 (192
   // workgroups) 54.6 -> 43.8, 2 x 500 27.0 -> 23.6, 3 x 300 22.0 -> 20.9; beyond, 2 x 1023 (256) 42.1 against 43.7, 8 x 300 31
   // against 40; with two tiles there is nothing to share: 4 x 61 10.2 against 11.8.
+  // float32: attn_prefill_f32_kernel, except for long prompts that fill the chip at d_head 64, where the tiles in LDS pay: 8 x
+  // 1499 tokens of 8 heads (768 workgroups of 128 queries) 194 us against 185, 16 x 1024 of 16 heads 383 against 334; 4 x 1499 of 8
+  // (384) 106 against 153, 32 x 300 of 16 (1536) 106 against 109.
+  const bool few = dh == 256 || Tp <= 300 || B * H * ((Tp + 127) / 128) <= 512;
   const bool two = Tp > 64 && B * H * ((Tp + 127) / 128) <= 192;
   if (dtype == MTJ_BF16 && q64) MTJ_PREFILL_Q64(bf16_t);
   else if (dtype == MTJ_F16 && q64) MTJ_PREFILL_Q64(f16_t);
@@ -1507,12 +1691,14 @@ int attn_prefill_impl(const void* q, const void* k_cache, const void* v_t, const
   else if (dtype == MTJ_F16 && dh == 256 && two) MTJ_PREFILL_PAIR(f16_t, 2);
   else if (dtype == MTJ_F16 && dh == 256) MTJ_PREFILL_PAIR(f16_t, 1);
   else if (dtype == MTJ_F16 && dh == 64) MTJ_PREFILL(f16_t, 64, 8, 64);
-  else if (dtype == MTJ_F32 && dh == 256) MTJ_PREFILL(float, 256, 4, 32);
+  else if (dtype == MTJ_F32 && dh == 256) MTJ_PREFILL_F32(256);
+  else if (dtype == MTJ_F32 && dh == 64 && few) MTJ_PREFILL_F32(64);
   else if (dtype == MTJ_F32 && dh == 64) MTJ_PREFILL(float, 64, 4, 32);
   else return mtj_fail(MTJ_EINVAL, "mtj_attn_prefill: unsupported dtype %d / d_head %lld (64 or 256)", dtype, (long long)dh);
 #undef MTJ_PREFILL
 #undef MTJ_PREFILL_PAIR
 #undef MTJ_PREFILL_Q64
+#undef MTJ_PREFILL_F32
   return mtj_check_launch("mtj_attn_prefill");
 }
 

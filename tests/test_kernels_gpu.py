@@ -826,6 +826,14 @@ def test_attn_prefill_with_the_keys_shared_by_two_pairs(L, dt, H, Tp):
     test_attn_prefill(L, dt, 256, H, Tp)
 
 
+@pytest.mark.parametrize("dh,H,Tp", [(256, 2, 31), (256, 1, 97), (256, 2, 161), (256, 1, 300), (64, 3, 129), (64, 2, 511),
+                                     (64, 86, 301), (64, 85, 301)])
+def test_attn_prefill_float32_wavefronts_share_the_queries(L, dh, H, Tp):
+    """float32: wavefronts without a key tile (1, 4 and 6 tiles), partial last tiles in each; the last two lie on either
+    side of 512 workgroups of 128 queries, from where long prompts at d_head 64 keep their tiles in LDS."""
+    test_attn_prefill(L, "f32", dh, H, Tp)
+
+
 def test_attn_prefill_of_infinite_and_nan_values_with_the_keys_shared_by_two_pairs(L):
     """A NaN or infinite value reaches the queries that may see its key, whichever pair holds it, and no other (bfloat16: a float16
     result saturates)."""
