@@ -246,8 +246,9 @@ int mtj_attn_decode(const float* q, const void* k_cache, const void* v_cache, co
                     int64_t H, int64_t Tcap, int64_t dh, void* out, int64_t ld_out, int out_dtype, int dtype,
                     void* work, void* stream);
 
-/* mtj_attn_decode in one launch, for up to 64 sequences: the key ranges follow the lengths of all sequences, and the
- * workgroup that finishes the last range of a (sequence, head) merges them.  Same arguments and results, except for
+/* mtj_attn_decode in one launch, for up to 64 sequences: the number of key ranges of a sequence follows its length (and B and
+ * H), and the workgroup that finishes the last range of a (sequence, head) merges them.  Same arguments, and the same results
+ * up to the order of summation, which for a sequence does not depend on the lengths of the others; except for
  * `work`: 128-byte aligned, mtj_attn_decode_joined_work_bytes(B, H, dh, Tcap) bytes (0: this shape is not covered, use
  * mtj_attn_decode), zeroed by the caller ONCE before its first use; every launch leaves its counters at zero.  Calls
  * sharing one `work` must have the same B, H and dh and must not overlap. */

@@ -1330,7 +1330,6 @@ __global__ __launch_bounds__(256) void attn_prefill_q64_kernel(const T* __restri
 // result goes straight to `out`; otherwise attn_combine_kernel (or the prologue of the out-projection GEMV) merges them.
 constexpr int DEC_NI = 8;            // K (and V) loads per lane and step
 constexpr int DEC_PAD = MTJ_DEC_PAD;  // floats in front of the vector of a partial
-constexpr int DEC_RATE = 150;                    // see attn_decode_kernel
 constexpr int JOIN_NW = 8, JOIN_NI = 4;          // wavefronts, loads per lane and step
 constexpr int DEC_LINE = 32;         // floats of a 128-byte line: what two workgroups write never shares one
 constexpr int joined_stride(int dh) { return (dh + DEC_PAD + DEC_LINE - 1) / DEC_LINE * DEC_LINE; }
@@ -1338,38 +1337,20 @@ __host__ __device__ constexpr int64_t joined_block(int64_t S, int64_t dh) {
   return DEC_LINE + S * ((dh + DEC_PAD + DEC_LINE - 1) / DEC_LINE * DEC_LINE);
 }
 
-// op over the values of lanes 0 .. l in lane l, for the first B lanes (op(0, x) == x): row shifts inside 16 lanes, then the
-// last lanes of the rows before
-template <class OP> __device__ __forceinline__ int lane_scan(int v, int B, OP op) {
-  v = op(__builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false), v);
-  v = op(__builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false), v);
-  v = op(__builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false), v);
-  v = op(__builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false), v);
-  const int row = (threadIdx.x & 63) >> 4;
-  for (int r = 1; r * 16 < B; ++r) {
-    const int t = __builtin_amdgcn_readlane(v, r * 16 - 1);
-    if (row == r) v = op(t, v);
-  }
-  return v;
-}
-
-// JOIN: one launch whatever the cut, and a cut that follows the lengths of all sequences.  Workgroups of 8 wavefronts (4
-// loads per lane and step, two of them per CU) take the key ranges of all (sequence, head) pairs in order, so that no
-// workgroup between them is empty - workgroups are dealt round-robin over the XCDs, and with the ranges in a grid
-// dimension of their own the short sequences' empty ones would leave XCDs idle -; the workgroup that finishes a pair's last
-// range merges them (an arrivals counter in front of the partials; no workgroup waits for another).
-// What a cut costs and gives was measured: the chip reads as fast as DEC_RATE workgroups that have it to themselves (40 - 53
-// GB/s each), and a merge takes 2 - 3 us, the time of two steps.  So nothing is cut while the longest sequence ends no
-// more than two steps after the chip could have read all keys; beyond that a range is a workgroup's share of the keys, and
-// not below two steps.  16 heads of 256, us, two equal or more ranges and a separate merge launch before: 3 x 33 .. 100
-// keys 7.3 -> 5.8, 4 x 300 10.0 -> 9.0, 8 x 64 7.5 -> 6.3, 8 x 80 .. 640 18.0 -> 14.1, 8 x 250 .. 2000 37 -> 32, 12 x 40 .. 480
-// 18.5 -> 13.7, 16 x 62 .. 1000 33.6 -> 31.2; 8 x 600 19.5 -> 20.3; one range as before, with the rule in front: 16 x 1000
-// 44.2, 32 x 500 43.6, 22 x 1 .. 36 5.6 -> 5.9.
+// JOIN: one launch whatever the cut.  Grid (H, B, most ranges): workgroups of 8 wavefronts (4 loads per lane and step, two of
+// them per CU) take the first ranges of all (sequence, head) pairs, then the second ones, ..; a workgroup whose sequence has
+// fewer ranges ends at once.  (With the ranges as the fastest dimension the short sequences' empty workgroups leave XCDs
+// idle, workgroups are dealt round-robin over them: 8 x 64 keys 16.6 us instead of 5.9.)  The workgroup that finishes a
+// pair's last range merges them (an arrivals counter in front of the partials; no workgroup waits for another).
+// How a sequence is cut follows its own length alone, so its bits do not depend on what else is in the batch, and no workgroup
+// looks at another sequence's position.  joined_cut says how.
+struct joined_cut_t { int line, most; };       // a sequence of more than `line` steps is cut into ranges of two steps, `most` at most
 template <typename T, int DH, bool JOIN, int NW = 4, int NI = DEC_NI>
 __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(const float* __restrict__ q, const T* __restrict__ kc,
                                                           const T* __restrict__ vc, const int32_t* __restrict__ pos,
-                                                          int B, int H, int Tcap, int smax, float* __restrict__ work,
-                                                          void* __restrict__ out, int64_t ld_out, int out_dtype) {
+                                                          int H, int Tcap, int smax, joined_cut_t cut,
+                                                          float* __restrict__ work, void* __restrict__ out, int64_t ld_out,
+                                                          int out_dtype) {
   constexpr int EPC = kvrow<T>::EPC;
   constexpr int LPK = DH / EPC;      // lanes per key row
   constexpr int KPL = 64 / LPK;      // keys per wavefront load
@@ -1379,50 +1360,17 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(const float* __res
   __shared__ float stat[NW][2];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  int S = gridDim.x, nvalid;                                  // key ranges, keys
+  const int split = JOIN ? blockIdx.z : blockIdx.x, h = JOIN ? blockIdx.x : blockIdx.y, b = JOIN ? blockIdx.y : blockIdx.z;
+  const int p = pos[b];
+  const int nvalid = (p + 1 < Tcap) ? p + 1 : Tcap;          // keys
+  int S = gridDim.x;                                          // key ranges
   if constexpr (JOIN) {
-    // lane l looks at sequence l
-    int n = 0;
-    if (lane < B) {
-      const int p = pos[lane];
-      n = (p + 1 < Tcap) ? p + 1 : Tcap;
-      n = n > 0 ? n : 0;
+    S = 1;
+    if (nvalid > cut.line * STEP) {
+      S = (nvalid + 2 * STEP - 1) / (2 * STEP);
+      S = S < cut.most ? S : cut.most;
     }
-    const unsigned all = (unsigned)__builtin_amdgcn_readlane(lane_scan(n, B, [](int x, int y) { return x + y; }), B - 1) * (unsigned)H;
-    const unsigned longest = (unsigned)__builtin_amdgcn_readlane(lane_scan(n, B, [](int x, int y) { return x > y ? x : y; }), B - 1);
-    const unsigned grid = gridDim.x, spare = grid - (unsigned)(B * H), least = 2 * STEP;
-    auto most = [](unsigned x, unsigned y) { return x > y ? x : y; };
-    auto ranges = [&](unsigned want) {                         // of lane's sequence, of `want` keys at most
-      int c = (int)(((unsigned)n + want - 1) / want);
-      c = c < smax ? c : smax;
-      return lane >= B ? 0 : c > 1 ? c : 1;
-    };
-    int cut, end;                                              // end: ranges of sequences 0 .. l, per head
-    if (longest <= most(most(all / DEC_RATE, (all + grid - 1) / grid), least) + least) {
-      cut = lane < B ? 1 : 0;
-      end = lane + 1;
-    } else {
-      // a workgroup's share of the keys; where the rounding up leaves too few workgroups for all ranges, as many keys as
-      // never do: the sum of ceil(n / want) is at most the sum of n / want, plus one per (sequence, head)
-      cut = ranges(most((all + grid - 1) / grid, least));
-      end = lane_scan(cut, B, [](int x, int y) { return x + y; });
-      if ((unsigned)__builtin_amdgcn_readlane(end, B - 1) * (unsigned)H > grid) {
-        cut = ranges(most((all + spare - 1) / spare, least));
-        end = lane_scan(cut, B, [](int x, int y) { return x + y; });
-      }
-    }
-    const int w = blockIdx.x;                                  // the workgroups take the ranges in order
-    b = (int)__popcll(__ballot(lane < B && end * H <= w));     // (`end` grows with the lane)
-    if (b >= B) return;
-    S = __builtin_amdgcn_readlane(cut, b);
-    const int r = w - (__builtin_amdgcn_readlane(end, b) - S) * H;
-    h = (int)((unsigned)r / (unsigned)S);
-    split = r - h * S;
-    nvalid = __builtin_amdgcn_readlane(n, b);
-  } else {
-    const int p = pos[b];
-    nvalid = (p + 1 < Tcap) ? p + 1 : Tcap;
+    if (split >= S) return;
   }
   const int64_t bh = (int64_t)b * H + h;
   const int per = (nvalid + S - 1) / S;                       // keys per range
@@ -1435,7 +1383,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(const float* __res
 #pragma unroll
   for (int j = 0; j < EPC; ++j) acc[j] = 0.f;
 
-  if (nk > 0) {
+  if (nk > (JOIN ? wave * KPL : 0)) {                          // (a wavefront without a key asks for none)
     const T* kbase = kc + (bh * Tcap + k0) * DH + el;
     const T* vbase = vc + (bh * Tcap + k0) * DH + el;
     uint32x4 kr[2][NI], vr[2][NI];
@@ -1499,7 +1447,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(const float* __res
     }
     if (base < nk) reduce(0, base);
   }
-  // ---- key subgroups of a wavefront, then the four wavefronts
+  // ---- key subgroups of a wavefront, then the wavefronts
 #pragma unroll
   for (int o = 32; o >= LPK; o >>= 1) {
     l_run += __shfl_xor(l_run, o);
@@ -1589,14 +1537,6 @@ __global__ __launch_bounds__(DH / 4) void attn_combine_kernel(const float* __res
 // length (8 x 16 heads of 256 x 80 .. 640 keys 17.9 -> 16.3 us, 250 .. 2000 40.8 -> 35.5), leave long equal ones as they are
 // (2000 keys 51.7 -> 49.6) and cost every short window of up to one workgroup step per range: 64 keys 7.8 -> 8.8 us, d_head
 // 64 up to 300 keys 8.1 -> 9.0.
-// key ranges a pair may be cut into (room for their partials), and workgroups: two per CU, or two per pair
-int joined_splits(int64_t B, int64_t H) { return B * H > 64 ? 8 : 16; }
-int64_t joined_grid(int64_t B, int64_t H) { return B * H > 256 ? 2 * B * H : 512; }
-// a lane per sequence, 32-bit sums of keys
-bool joined_ok(int64_t B, int64_t H, int64_t Tcap) {
-  return B > 0 && B <= 64 && H > 0 && H < 65536 && Tcap > 0 && Tcap < (1ll << 30) && (Tcap + 2) * B * H < (1ll << 31);
-}
-
 int decode_splits(int64_t B, int64_t H, int64_t Tcap) {
   int64_t S = 256 / (B * H);
   if (S > (Tcap + 15) / 16) S = (Tcap + 15) / 16;
@@ -1608,6 +1548,29 @@ int decode_splits(int64_t B, int64_t H, int64_t Tcap) {
 }  // namespace
 
 namespace {
+
+// Key ranges a pair may be cut into: room for their partials.
+int joined_splits(int64_t B, int64_t H) { return B * H > 64 ? 8 : 16; }
+bool joined_ok(int64_t B, int64_t H, int64_t Tcap) {
+  return B > 0 && B <= 64 && H > 0 && H < 65536 && Tcap > 0 && Tcap < (1ll << 30) && (Tcap + 2) * B * H < (1ll << 31);
+}
+// How mtj_attn_decode_joined cuts a sequence, by the number of (sequence, head) pairs.  A merge takes 2 - 3 us, the time of two
+// steps, and two workgroups on a CU are little faster than one, so: up to 85 pairs as many ranges as the CUs hold once; up
+// to 128 two workgroups on every CU, which unequal sequences use better; up to 160 the same, but only what is longer than
+// four steps; beyond, the pairs alone read nearly as fast as the chip does.  16 heads of 256 in float16, us, geometric means over
+// windows of 200, 300, 480, 700, 1000 and 1900 keys, first all sequences of one length, then lengths from a B-th of that up;
+// in front mtj_attn_decode: 2 sequences 10.4 -> 9.2 and 9.9 -> 8.8, 3 12.2 -> 10.8 and 11.4 -> 9.9, 5 15.1 -> 13.3 and
+// 13.5 -> 11.6, 8 19.7 -> 18.0 and 16.7 -> 14.0, 10 22.1 -> 21.2 and 20.3 -> 16.2, 12 23.8 -> 22.1 and 20.8 -> 18.1, 16 27.9 ->
+// 27.3 and 21.4 -> 19.2.  Cut as 10 are, 11 sequences of one length take 23.5 (23.0 with mtj_attn_decode) and 12 24.3.  (Ranges
+// of equal numbers of keys over the whole batch were as good for most of these and better for unequal lengths at 9 .. 14
+// sequences - 12 x 158 .. 1900 keys 39 against 46 -, but then a sequence's bits depend on its neighbours, and the look at
+// all lengths takes 0.3 us of every launch.)
+joined_cut_t joined_cut(int64_t B, int64_t H) {
+  const int64_t pairs = B * H;
+  if (pairs <= 85) return {2, (int)(pairs <= 16 ? 16 : 256 / pairs)};
+  if (pairs <= 160) return {pairs <= 128 ? 2 : 4, 8};
+  return {1 << 20, 1};
+}
 
 int attn_prefill_impl(const void* q, const void* k_cache, const void* v_t, const int32_t* pos0, int64_t B, int64_t H,
                       int64_t Tp, int64_t Tcap, int64_t dh, int64_t ldvt, void* out, int64_t ld_out, int dtype,
@@ -1743,18 +1706,19 @@ int attn_decode_impl(const char* who, const float* q, const void* k_cache, const
     MTJ_REQUIRE(mtj_is_dtype(out_dtype), MTJ_EDTYPE, "%s: out_dtype %d", who, out_dtype);
   }
   const int S = join ? joined_splits(B, H) : decode_splits(B, H, Tcap);
+  const joined_cut_t cut = joined_cut(B, H);
   float* partials = reinterpret_cast<float*>(work);
   dim3 grid((unsigned)S, (unsigned)H, (unsigned)B);
   hipStream_t s = (hipStream_t)stream;
 #define MTJ_DECODE(T, DH)                                                                                         \
   do {                                                                                                            \
     if (join) {                                                                                                   \
-      attn_decode_kernel<T, DH, true, JOIN_NW, JOIN_NI><<<(unsigned)joined_grid(B, H), JOIN_NW * 64, 0, s>>>(       \
-          q, (const T*)k_cache, (const T*)v_cache, pos, (int)B, (int)H, (int)Tcap, S, partials, out, ld_out, out_dtype); \
+      attn_decode_kernel<T, DH, true, JOIN_NW, JOIN_NI><<<dim3((unsigned)H, (unsigned)B, (unsigned)cut.most), JOIN_NW * 64, 0, s>>>( \
+          q, (const T*)k_cache, (const T*)v_cache, pos, (int)H, (int)Tcap, S, cut, partials, out, ld_out, out_dtype); \
       break;                                                                                                      \
     }                                                                                                             \
-    attn_decode_kernel<T, DH, false><<<grid, 256, 0, s>>>(q, (const T*)k_cache, (const T*)v_cache, pos, (int)B, (int)H, \
-                                                          (int)Tcap, S, partials, out, ld_out, out_dtype);        \
+    attn_decode_kernel<T, DH, false><<<grid, 256, 0, s>>>(q, (const T*)k_cache, (const T*)v_cache, pos, (int)H, (int)Tcap, S, \
+                                                          cut, partials, out, ld_out, out_dtype);                 \
     if (merge && S > 1)                                                                                           \
       attn_combine_kernel<DH><<<dim3((unsigned)H, (unsigned)B), DH / 4, 0, s>>>(partials, S, (int)H, out, ld_out,  \
                                                                                  out_dtype);                      \

@@ -1105,6 +1105,32 @@ def test_attn_decode_in_one_launch(L, dt, dh, H, Tcap, steps):
             assert rel_err(out[b, :H * dh], ref2[b, :H * dh]) < 3e-6
 
 
+@pytest.mark.parametrize("dt,H,dh,B", [("f16", 16, 256, 3), ("f16", 16, 256, 5), ("f16", 16, 256, 8), ("f16", 16, 256, 10),
+                                       ("f16", 16, 256, 11), ("f32", 8, 64, 2), ("bf16", 8, 64, 64)])
+def test_attn_decode_in_one_launch_does_not_depend_on_the_neighbours(L, dt, H, dh, B):
+    """The bits of a sequence are the same whatever the lengths of the others, for batches on both sides of every line of the
+    cut (up to 85, 128, 160 and more (sequence, head) pairs), and within rounding of float64."""
+    a = abi()
+    Tcap = 1900
+    g = torch.Generator(device=DEV).manual_seed(B)
+    q = torch.randn(B, H, dh, generator=g, device=DEV)
+    kc, vc = (torch.randn(B, H, Tcap, dh, generator=g, device=DEV).to(TD[dt]) for _ in range(2))
+    work = torch.zeros(L.mtj_attn_decode_joined_work_bytes(B, H, dh, Tcap), dtype=torch.uint8, device=DEV)
+    for own in (90, 127, 128, 256, 300, 1000, 1899):
+        outs = []
+        for others in ([own] * B, [5] * B, [Tcap - 1] * B, [(b * 397) % Tcap for b in range(B)]):
+            pos = torch.tensor(others[:1] + [own] + others[2:], dtype=torch.int32, device=DEV)
+            out = torch.empty(B, H * dh, device=DEV)
+            a.check(L.mtj_attn_decode_joined(a.ptr(q), a.ptr(kc), a.ptr(vc), a.ptr(pos), B, H, Tcap, dh, a.ptr(out), H * dh, 0,
+                                             a.dtype_code(TD[dt]), a.ptr(work), S()))
+            torch.cuda.synchronize()
+            outs.append(out[1].clone())
+        assert all(torch.equal(o, outs[0]) for o in outs), own
+        s = (kc[1, :, :own + 1].double() @ q[1].double()[:, :, None])[..., 0] / math.sqrt(dh)
+        ref = (torch.softmax(s, -1)[:, None] @ vc[1, :, :own + 1].double()).reshape(-1)
+        assert rel_err(outs[0], ref) < 3e-6, own
+
+
 def test_attn_decode_in_one_launch_replayed_from_a_graph(L):
     """Positions move between the replays (the cut follows them), with eager work in between."""
     a = abi()
