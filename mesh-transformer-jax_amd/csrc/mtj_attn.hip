@@ -1638,14 +1638,19 @@ int attn_prefill_impl(const void* q, const void* k_cache, const void* v_t, const
   // 128-query workgroups
   const bool q64 = dh == 256 && B * H * ((Tp + 255) / 256) >= 1024;
   // Few workgroups (one per CU): the longest walks over all keys while most of the chip has ended or had nothing, so the keys
-  // are shared by two pairs of wavefronts.  16 heads, us: 300 tokens 20.9 -> 19.2, 511 24.3 -> 20.2, 1023 39.7 -> 31.5, 1500 (192
-  // workgroups) 54.6 -> 43.8, 2 x 500 27.0 -> 23.6, 3 x 300 22.0 -> 20.9; beyond, 2 x 1023 (256) 42.1 against 43.7, 8 x 300 31
-  // against 40; with two tiles there is nothing to share: 4 x 61 10.2 against 11.8.
+  // are shared by two pairs of wavefronts, with half the queries in a workgroup.  16 heads, us: 256 tokens 16.8 -> 14.6, 511
+  // 24.3 -> 20.2, 1023 39.7 -> 31.5, 4 x 256 (256 workgroups of 64) 17.8 -> 16.7, 2 x 500 27.0 -> 23.6.  Beyond one round of them it
+  // pays for long prompts only: 2 x 576 (288) 25.0 -> 23.7, 2 x 768 (384) 32.3 -> 31.2, 1500 54.6 -> 43.8, but 3 x 384 (288) 21.6
+  // against 23.7, 6 x 192 14.6 against 22.6, 12 x 128 16.1 against 24.5.  Few tiles: 97 .. 160 tokens 13.1 -> 12.2 (4 x 160 13.7 ->
+  // 13.0; 8 x 128, 256 workgroups, 14.7 against 14.9), 192, where every second workgroup is half empty as it is, 13.1 against
+  // 13.2 (5 x 192 14.2 against 15.1), up to 96 tokens 11.1 against 11.0 (6 x 96 11.4 against 11.8).
+  const int64_t halves = B * H * ((Tp + 63) / 64);
+  const bool two = halves <= 256 ? Tp > 192 || (Tp > 96 && Tp <= 160 && halves < 256)
+                                 : Tp > 512 && B * H * ((Tp + 127) / 128) <= 192;
   // float32: attn_prefill_f32_kernel, except for long prompts that fill the chip at d_head 64, where the tiles in LDS pay: 8 x
   // 1499 tokens of 8 heads (768 workgroups of 128 queries) 194 us against 185, 16 x 1024 of 16 heads 383 against 334; 4 x 1499 of 8
   // (384) 106 against 153, 32 x 300 of 16 (1536) 106 against 109.
   const bool few = dh == 256 || Tp <= 300 || B * H * ((Tp + 127) / 128) <= 512;
-  const bool two = Tp > 64 && B * H * ((Tp + 127) / 128) <= 192;
   if (dtype == MTJ_BF16 && q64) MTJ_PREFILL_Q64(bf16_t);
   else if (dtype == MTJ_F16 && q64) MTJ_PREFILL_Q64(f16_t);
   else if (dtype == MTJ_BF16 && dh == 256 && two) MTJ_PREFILL_PAIR(bf16_t, 2);

@@ -826,6 +826,13 @@ def test_attn_prefill_with_the_keys_shared_by_two_pairs(L, dt, H, Tp):
     test_attn_prefill(L, dt, 256, H, Tp)
 
 
+@pytest.mark.parametrize("H,Tp", [(2, 160), (2, 161), (2, 192), (2, 193), (32, 256), (33, 256), (42, 130), (43, 130), (16, 576),
+                                  (20, 577)])
+def test_attn_prefill_on_both_sides_of_the_lines_of_the_two_pairs(L, H, Tp):
+    """Two sequences of H heads of 256: 160 and 192 tokens, 256 workgroups of 64 queries, and beyond them 192 of 128."""
+    test_attn_prefill(L, "f16", 256, H, Tp)
+
+
 @pytest.mark.parametrize("dh,H,Tp", [(256, 2, 31), (256, 1, 97), (256, 2, 161), (256, 1, 300), (64, 3, 129), (64, 2, 511),
                                      (64, 86, 301), (64, 85, 301)])
 def test_attn_prefill_float32_wavefronts_share_the_queries(L, dh, H, Tp):
