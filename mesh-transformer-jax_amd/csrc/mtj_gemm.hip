@@ -1243,20 +1243,15 @@ template <int C> __device__ __forceinline__ void add_partials(floatx4& acc, cons
 #pragma unroll
   for (int i = 0; i < C; ++i) { acc.x += t[i].x; acc.y += t[i].y; acc.z += t[i].z; acc.w += t[i].w; }
 }
-__device__ __forceinline__ floatx4 sum_partials(const float* __restrict__ p, int splits, int64_t stride) {
+// C: loads in flight.
+template <int C = 8> __device__ __forceinline__ floatx4 sum_partials(const float* __restrict__ p, int splits, int64_t stride) {
   floatx4 acc = *reinterpret_cast<const floatx4*>(p);
   p += stride;
   int left = splits - 1;
-  for (; left > 7; left -= 8, p += 8 * stride) add_partials<8>(acc, p, stride);
-  switch (left) {
-    case 7: add_partials<7>(acc, p, stride); break;
-    case 6: add_partials<6>(acc, p, stride); break;
-    case 5: add_partials<5>(acc, p, stride); break;
-    case 4: add_partials<4>(acc, p, stride); break;
-    case 3: add_partials<3>(acc, p, stride); break;
-    case 2: add_partials<2>(acc, p, stride); break;
-    case 1: add_partials<1>(acc, p, stride); break;
-  }
+  for (; left >= C; left -= C, p += C * stride) add_partials<C>(acc, p, stride);
+  for_stages<1, C>([&](auto N_) {
+    if (left == decltype(N_)::value) add_partials<decltype(N_)::value>(acc, p, stride);
+  });
   return acc;
 }
 
@@ -1296,8 +1291,12 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 // One thread per four columns up to 4096 columns: rows of a narrow model do not wait for idle wavefronts (N = 512, two
 // ranges, with the product: 8000 rows 85 us with 1024 threads per row, 53 with 128, 60 with a separate LayerNorm; N = 4096
 // as before).  The sums of idle wavefronts were zeros, so the results are the same bits.
+// Q quads per thread, one up to 4096 columns.  Two workgroups of 1024 threads per CU need 64 registers or less, and while one
+// waits at a barrier the other loads: with 80, N = 4096 in eight ranges, 511 / 700 / 1500 rows took 19.7 / 19.5 / 29.2 us, now
+// 15.3 / 14.7 / 20.9 (17.2 / 17.8 / 23.2 with one partial load at a time and 44 registers).
 constexpr int RLN_Q = 4;
-__global__ __launch_bounds__(1024) void splitk_reduce_ln_kernel(const float* __restrict__ work, int splits,
+template <int Q>
+__global__ __launch_bounds__(1024, 8) void splitk_reduce_ln_kernel(const float* __restrict__ work, int splits,
                                                                 int64_t split_stride, int N, const float* __restrict__ bias,
                                                                 float* __restrict__ x, int64_t ldx,
                                                                 const float* __restrict__ ln_scale,
@@ -1306,21 +1305,21 @@ __global__ __launch_bounds__(1024) void splitk_reduce_ln_kernel(const float* __r
   __shared__ float red[2][16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int m = blockIdx.x, nq = N / 4, NT = blockDim.x, NW = NT / 64;
-  floatx4 v[RLN_Q], sc, of;
+  floatx4 v[Q], sc, of;
   float sum = 0.f;
 #pragma unroll
-  for (int i = 0; i < RLN_Q; ++i) {
+  for (int i = 0; i < Q; ++i) {
     const int q = i * NT + tid;
     if (q < nq) {
       const int n = q * 4;
       float* o = x + (int64_t)m * ldx + n;
       const floatx4 old = *reinterpret_cast<const floatx4*>(o);
       const floatx4 b = bias ? *reinterpret_cast<const floatx4*>(bias + n) : floatx4{0.f, 0.f, 0.f, 0.f};
-      if (i == 0) {                            // needed last, asked for with everything else
+      if (Q == 1) {                            // needed last, asked for with everything else
         sc = *reinterpret_cast<const floatx4*>(ln_scale + n);
         of = *reinterpret_cast<const floatx4*>(ln_offset + n);
       }
-      floatx4 acc = sum_partials(work + (int64_t)m * N + n, splits, split_stride);
+      floatx4 acc = sum_partials<Q == 1 ? 8 : 4>(work + (int64_t)m * N + n, splits, split_stride);
       if (bias) { acc.x += b.x; acc.y += b.y; acc.z += b.z; acc.w += b.w; }
       // the same two roundings per element as "o[j] += acc.j" of the plain reduce
       acc.x = old.x + acc.x; acc.y = old.y + acc.y; acc.z = old.z + acc.z; acc.w = old.w + acc.w;
@@ -1337,7 +1336,7 @@ __global__ __launch_bounds__(1024) void splitk_reduce_ln_kernel(const float* __r
   const float mean = tot / (float)N;
   float sq = 0.f;
 #pragma unroll
-  for (int i = 0; i < RLN_Q; ++i) {
+  for (int i = 0; i < Q; ++i) {
     if (i * NT + tid < nq) {
       const floatx4 t = v[i] - mean;
       sq += (t.x * t.x + t.y * t.y) + (t.z * t.z + t.w * t.w);
@@ -1350,11 +1349,11 @@ __global__ __launch_bounds__(1024) void splitk_reduce_ln_kernel(const float* __r
   for (int i = 0; i < NW; ++i) var += red[1][i];
   const float inv = rsqrtf(var / (float)N + 1e-5f);
 #pragma unroll
-  for (int i = 0; i < RLN_Q; ++i) {
+  for (int i = 0; i < Q; ++i) {
     const int q = i * NT + tid;
     if (q < nq) {
       const int n = q * 4;
-      if (i > 0) {
+      if (Q > 1) {
         sc = *reinterpret_cast<const floatx4*>(ln_scale + n);
         of = *reinterpret_cast<const floatx4*>(ln_offset + n);
       }
@@ -1675,8 +1674,12 @@ extern "C" int mtj_gemm_splitk_ln(const void* A, int64_t lda, const void* W, con
   a.out = work; a.ldo = N; a.out_dtype = MTJ_F32; a.alpha = alpha;
   a.splits = splits; a.split_stride = M * N;
   if (int rc = dispatch_dtype(a, dtype, MTJ_EPI_STORE, s)) return rc;
-  splitk_reduce_ln_kernel<<<(unsigned)M, rln_threads(N), 0, s>>>((const float*)work, splits, M * N, (int)N, bias, x, ldx, ln_scale,
-                                                       ln_offset, h, ldh, h_dtype);
+  if (N <= 4096)
+    splitk_reduce_ln_kernel<1><<<(unsigned)M, rln_threads(N), 0, s>>>((const float*)work, splits, M * N, (int)N, bias, x, ldx, ln_scale,
+                                                                      ln_offset, h, ldh, h_dtype);
+  else
+    splitk_reduce_ln_kernel<RLN_Q><<<(unsigned)M, rln_threads(N), 0, s>>>((const float*)work, splits, M * N, (int)N, bias, x, ldx,
+                                                                          ln_scale, ln_offset, h, ldh, h_dtype);
   return mtj_check_launch("mtj_gemm_splitk_ln");
 }
 
