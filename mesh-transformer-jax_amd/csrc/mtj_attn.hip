@@ -1647,10 +1647,18 @@ int attn_prefill_impl(const void* q, const void* k_cache, const void* v_t, const
   const int64_t halves = B * H * ((Tp + 63) / 64);
   const bool two = halves <= 256 ? Tp > 192 || (Tp > 96 && Tp <= 160 && halves < 256)
                                  : Tp > 512 && B * H * ((Tp + 127) / 128) <= 192;
-  // float32: attn_prefill_f32_kernel, except for long prompts that fill the chip at d_head 64, where the tiles in LDS pay: 8 x
-  // 1499 tokens of 8 heads (768 workgroups of 128 queries) 194 us against 185, 16 x 1024 of 16 heads 383 against 334; 4 x 1499 of 8
-  // (384) 106 against 153, 32 x 300 of 16 (1536) 106 against 109.
-  const bool few = dh == 256 || Tp <= 300 || B * H * ((Tp + 127) / 128) <= 512;
+  // float32: attn_prefill_f32_kernel, which reads K and V^T once per 32 queries, except where the chip is full of heads and the
+  // tiles in LDS (once per 128 queries) pay; whole workgroups of 128 queries waste least there.  us, tiles in LDS in front:
+  // d_head 256, 16 heads, 4 x 2047 (1024 workgroups of 128) 1380 -> 1295, 6 x 1500 (1152) 1208 -> 1116, 12 x 512 (768) 362 -> 350, 32 x
+  // 300 545 -> 494, but 8 x 2047 (2048) 2779 against 2944, 12 x 1024 (1536) 1170 against 1268, 16 x 1024 1617 against 1879, 24 x 512
+  // (1536) 704 against 786; 8 x 512 (512) 223 against 228, 16 x 512 (1024) 477 against 484.
+  // d_head 64, 8 heads, 4 x 2047 (512) 223 -> 181, 6 x 2047 (768) 245 each; up to 256 tokens by workgroups of 32 queries: 16 x 200
+  // (896) 23.4 -> 20.2, 32 x 128 (1024) 16.2 against 17.1, 64 x 128 27.2 against 29.7, 32 x 200 32.3 against 35.1; at 257 .. 300 the third
+  // workgroup of 128 is nearly empty, 32 x 300 65.8 -> 57.3; up to 64 tokens 64 x 64 15.0 -> 13.7.
+  const int64_t blocks = B * H * ((Tp + 127) / 128);
+  const bool few = dh == 256  ? Tp <= 300 || blocks <= 1152
+                   : Tp <= 256 ? Tp <= 64 || B * H * ((Tp + 31) / 32) < 1024
+                               : Tp <= 300 || blocks <= 512;
   if (dtype == MTJ_BF16 && q64) MTJ_PREFILL_Q64(bf16_t);
   else if (dtype == MTJ_F16 && q64) MTJ_PREFILL_Q64(f16_t);
   else if (dtype == MTJ_BF16 && dh == 256 && two) MTJ_PREFILL_PAIR(bf16_t, 2);
@@ -1659,7 +1667,8 @@ int attn_prefill_impl(const void* q, const void* k_cache, const void* v_t, const
   else if (dtype == MTJ_F16 && dh == 256 && two) MTJ_PREFILL_PAIR(f16_t, 2);
   else if (dtype == MTJ_F16 && dh == 256) MTJ_PREFILL_PAIR(f16_t, 1);
   else if (dtype == MTJ_F16 && dh == 64) MTJ_PREFILL(f16_t, 64, 8, 64);
-  else if (dtype == MTJ_F32 && dh == 256) MTJ_PREFILL_F32(256);
+  else if (dtype == MTJ_F32 && dh == 256 && few) MTJ_PREFILL_F32(256);
+  else if (dtype == MTJ_F32 && dh == 256) MTJ_PREFILL(float, 256, 4, 32);
   else if (dtype == MTJ_F32 && dh == 64 && few) MTJ_PREFILL_F32(64);
   else if (dtype == MTJ_F32 && dh == 64) MTJ_PREFILL(float, 64, 4, 32);
   else return mtj_fail(MTJ_EINVAL, "mtj_attn_prefill: unsupported dtype %d / d_head %lld (64 or 256)", dtype, (long long)dh);

@@ -841,6 +841,13 @@ def test_attn_prefill_float32_wavefronts_share_the_queries(L, dh, H, Tp):
     test_attn_prefill(L, "f32", dh, H, Tp)
 
 
+@pytest.mark.parametrize("dh,H,Tp", [(256, 192, 301), (256, 193, 301), (256, 193, 300), (64, 127, 128), (64, 128, 128),
+                                     (64, 128, 129), (64, 256, 64), (64, 256, 257)])
+def test_attn_prefill_float32_on_both_sides_of_the_lines(L, dh, H, Tp):
+    """Two sequences of H heads: 1152 workgroups of 128 queries at d_head 256, 1024 of 32 at d_head 64 up to 256 tokens."""
+    test_attn_prefill(L, "f32", dh, H, Tp)
+
+
 def test_attn_prefill_of_infinite_and_nan_values_with_the_keys_shared_by_two_pairs(L):
     """A NaN or infinite value reaches the queries that may see its key, whichever pair holds it, and no other (bfloat16: a float16
     result saturates)."""
