@@ -1433,15 +1433,20 @@ int64_t dma_cost(int64_t tiles, int64_t kt, int64_t s) {
 // Rows of a fused input projection that run on 256 x 256 tiles when the rest, the rows of its last row of tiles, is better
 // off as a launch of its own: where that row of tiles starts a round of workgroups of which most CUs have nothing (1.6 us a
 // k-tile), and the rest streams the weights once more in less (gemm_stream_kernel: 5.9, 4.8 and 3.6 TB/s for up to 64, 128 and
-// 256 rows, 4 us for the launch).  0: one launch.  d_model 4096, 520 / 580 / 700 rows 182 / 188 / 199 -> 152 / 156 / 183 us, 1030 / 1200 282 /
-// 300 -> 254 / 280, 2874 610 -> 580, 3400 760 -> 709, 5700 (10 rounds) 1179 -> 1140; 7655 (13) 1490 either way, the rounds have
-// drifted apart by then, so beyond 11 it stays one launch; d_model 2048, 1100 rows 111 -> 91;
-// 1024, 2400 rows 76 -> 64; 512, 4800 rows 54.5 -> 48.9.
+// 256 rows, 4 us for the launch).  0: one launch.  d_model 4096, 580 / 700 rows 194 / 195 -> 152 / 171 us, 1030 / 1270 279 /
+// 297 -> 248 / 276, 2935 606 -> 579, 3400 725 -> 678, 5700 (10 rounds) 1147 -> 1100; d_model 2048, 1085 rows 107 -> 82; 1024, 2420
+// rows 73 -> 63; 512, 4730 rows 53 -> 48.
+// The rounds of one launch drift apart, the sooner the shorter K is against the epilogue, and a round more then costs little,
+// while two launches wait for each other.  So there is a limit of whole rounds in front, by K, from six sizes per round and
+// d_model 512, 768, 1024, 1536, 2048, 3072 and 4096: from 4096 on 10 (11: 6590 rows 1236 against 1262), from 1024 on 6 (beyond,
+// it wins and loses: 1024 16500 281 against 290, 18750 323 -> 308; 1536 12400 409 -> 403, 15500 519 against 535; 2048 8350 454
+// against 462, 11600 624 -> 604; 3072 5510 647 against 657, 7000 830 -> 790), from 768 on 3 (4 .. 11: 15440 176 against 180,
+// 34340 358 against 377), below 1 (2: 512 9240 68 against 77, 3: 13930 93 against 103).
 int64_t inproj_front(int64_t M, int64_t N, int64_t K) {
   const int64_t front = (M - 1) / 256 * 256, rest = M - front;
   if (dma_tiles(front, N) < (K < 768 ? DMA_MIN_TILES_SHORT_INPROJ : DMA_MIN_TILES)) return 0;
   const int64_t whole = (dma_tiles(front, N) + 255) / 256, rounds = (dma_tiles(M, N) + 255) / 256 - whole;
-  if (whole > 11) return 0;
+  if (whole > (K >= 4096 ? 10 : K >= 1024 ? 6 : K >= 768 ? 3 : 1)) return 0;
   const double rate = rest <= 64 ? 5.9e6 : rest <= 128 ? 4.8e6 : 3.6e6;                  // bytes per us
   return (double)rounds * (double)(K / 64) * 1.6 > (double)N * (double)K * 2 / rate + 4.0 ? front : 0;
 }

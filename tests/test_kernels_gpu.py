@@ -611,6 +611,13 @@ def test_inproj_gemm_whose_last_rows_are_a_launch_of_their_own(Tp, pads):
     _run_inproj_prefill(cfg, _layer_params(cfg, 9, "bf16"), "bf16", B=3, Tp=Tp, Tcap=Tp + 3, pads=pads, seed=10)
 
 
+@pytest.mark.parametrize("d,heads,Tp", [(512, 8, 3080), (768, 12, 2060), (768, 12, 4115)])
+def test_inproj_gemm_behind_several_rounds_of_tiles(d, heads, Tp):
+    """A few rows behind two (d_model 512), two and four rounds (768) of tiles: one launch, two launches, one launch."""
+    cfg = dict(layers=1, d_model=d, n_heads=heads, n_vocab=64, pe="rotary", pe_rotary_dims=32, cores_per_replica=1)
+    _run_inproj_prefill(cfg, _layer_params(cfg, 9, "bf16"), "bf16", B=3, Tp=Tp, Tcap=Tp + 3, pads=[0, 37, 5], seed=10)
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 def test_gemm_resid_and_store_on_the_256x256_direct_to_lds_kernel(L, dt):
     """M = N = 4096 is 256 tiles of 256 x 256, so mtj_gemm itself (no K split) runs gemm_dma_kernel with the RESID and
