@@ -591,18 +591,25 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_kernel(const gemm_
 }
 
 // float32 operands on the bf16 matrix cores.  A float32 number is the sum of three bf16 numbers without an error (rounded to
-// nearest, each takes 8 of the 24 significant bits of what the ones before it leave), so a product is nine products of parts;
-// the six with the largest weights are taken - the other three together are below 2^-24 of the product - and summed in
-// float32 by the matrix cores, which round once per 16 elements of K instead of once per 2.  Error against float64, 2-norm,
-// normal operands, with v_mfma_f32_32x32x2_f32 and here: K = 512 4.0e-7 and 3.4e-7, 2560 4.6e-7 and 3.9e-7, 4096 1.15e-6 and
-// 1.00e-6, 20480 (four ranges) 1.28e-6 and 1.22e-6.
+// nearest, each takes 8 of the 24 significant bits of what the ones before it leave), so a product is nine products of
+// parts; the six with the largest weights are taken - the other three together are below 2^-24 of the product -.
+// The bf16 matrix instruction drops low bits of what it adds to a large accumulator, and not symmetrically: with one accumulator
+// for all of K the results lay 1e-7 (K = 2560) to 1e-6 (K = 20480) of their root mean square too low, whatever their sign.
+// So a sum is only CH k-tiles long and then added to a float32 total by the vector unit, and every second sum (and K range) is
+// of products with the sign of A turned, so that what is left of the bias cancels.
+// Error against float64, 2-norm / mean, both over the root mean square of the result, with v_mfma_f32_32x32x2_f32 and here:
+//   normal operands    K = 512   4.1e-7 / -1e-9  and 1.4e-7 / -2e-9      4096   1.2e-6 / -4e-9 and 1.9e-7 / -1e-9
+//                      K = 20480 2.6e-6 /  5e-9  and 3.0e-7 / -1e-9      in four ranges 1.3e-6 / -1e-9 and 2.1e-7 / -2e-10
+//   gelu(2 x normal)   K = 4096  1.1e-6 / -3e-10 and 1.9e-7 / -1e-9      20480  2.6e-6 / -8e-10 and 3.0e-7 / -8e-10
+//   positive operands  K = 4096  9.3e-7 / -7e-9  and 9.9e-8 / -2e-10     20480  1.9e-6 / -2e-7 and 2.0e-7 / -2e-10
 // An operand that is infinite, NaN or rounds to infinity gives NaN here, and a product next to the largest number may give
 // infinity; what is not finite is computed again in plain float32.
 //
-// Bound by the matrix cores: six v_mfma_f32_32x32x16_bf16 instead of eight v_mfma_f32_32x32x2_f32 of twice the length; the
-// splitting (11 vector instructions for two elements) runs under them.  N = 28672, K = 4096, 100 / 199 / 511 rows 305 / 517 /
-// 1010 -> 214 / 356 / 692 us (1.0 PFLOP/s of bf16 products); N = 4096, K = 20480 in four ranges, 199 / 511 rows 400 / 700 ->
-// 282 / 477; N = 3584, K = 512, 127 / 1499 rows 47 / 79 -> 35 / 53.
+// Bound by the vector unit, the barriers and the matrix cores in about equal parts: six v_mfma_f32_32x32x16_bf16 instead of
+// eight v_mfma_f32_32x32x2_f32 of twice the length, 12 vector instructions to split two elements, one per accumulator and sum.
+// us before and now: N = 28672, K = 4096, 65 / 199 / 600 / 2048 rows 290 / 544 / 1319 / 3516 -> 209 / 346 / 848 / 2420 (1.2 PFLOP/s of bf16
+// products); N = 4096, K = 20480, 65 / 128 / 400 / 1024 rows (4 ranges before, up to 16 now) 362 / 380 / 688 / 1379 -> 132 / 150 / 449 /
+// 900; N = 3584, K = 512, 127 / 1500 rows 48 / 77 -> 22 / 54.  The sums cost 4 - 6 % of these (a single accumulator: 600 rows 804).
 // A k-tile of 16 goes global -> registers (NS k-tiles in flight) -> three bf16 planes per row in LDS, double-buffered: rows
 // of 3 x 32 bytes, padded to 112 so that the 16-byte fragment reads of 16 consecutive rows hit distinct banks.
 __device__ __attribute__((noinline)) float plain_dot(const float* __restrict__ x, const float* __restrict__ w, int n) {
@@ -611,10 +618,11 @@ __device__ __attribute__((noinline)) float plain_dot(const float* __restrict__ x
   return s;
 }
 __device__ __forceinline__ bool not_finite(float x) { return !(fabsf(x) < INFINITY); }
+constexpr float SPLIT_UP = 1.f, SPLIT_DOWN = 1.f;
 
 template <int EPI, int WAVES_M, int WAVES_N, int WM, int WN, int NS>
-__global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_split_kernel(const gemm_args a) {
-  constexpr int NT = WAVES_M * WAVES_N * 64, BK = 16;
+__global__ __launch_bounds__(WAVES_M* WAVES_N * 64, WM * WN > 2 ? 2 : 3) void gemm_split_kernel(const gemm_args a) {
+  constexpr int NT = WAVES_M * WAVES_N * 64, BK = 16, CH = 2 * NS;
   constexpr int BM = WAVES_M * WM * 32, BN = WAVES_N * WN * 32;
   constexpr int ROWB = 112, PLANE = 32, STAGEB = (BM + BN) * ROWB;
   constexpr int ROWS_PER_PASS = NT / 2;                    // a thread takes 8 elements of a row at a time
@@ -671,13 +679,13 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_split_kernel(const
       for (int c = 0; c < 2; ++c)
         rb[st][i][c] = __builtin_amdgcn_raw_buffer_load_b128(rb_rsrc, voff_b + 16 * c, koff + i * pass_b, 0);
   };
-  // eight float32 numbers -> three times eight bf16
-  auto split_store = [&](unsigned char* dst, const uint32x4 (&r)[2]) {
+  // eight float32 numbers times `scale` -> three times eight bf16
+  auto split_store = [&](unsigned char* dst, const uint32x4 (&r)[2], float scale) {
     float x[8];
 #pragma unroll
     for (int c = 0; c < 2; ++c)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) x[4 * c + e] = __uint_as_float(r[c][e]);
+      for (int e = 0; e < 4; ++e) x[4 * c + e] = __uint_as_float(r[c][e]) * scale;
 #pragma unroll
     for (int part = 0; part < 3; ++part) {
       uint32x4 p;
@@ -689,18 +697,21 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_split_kernel(const
       *reinterpret_cast<uint32x4*>(dst + part * PLANE) = p;
     }
   };
-  auto store_lds = [&](auto ST_, int buf) {
+  const uint32_t range = blockIdx.y;
+  auto turned = [&](int kt) { return ((uint32_t)kt / CH + range) & 1u; };      // is k-tile kt of a sum with turned signs?
+  auto store_lds = [&](auto ST_, int buf, int kt) {
+    const float scale = turned(kt) ? -SPLIT_UP : SPLIT_UP;
     constexpr int st = decltype(ST_)::value;
     unsigned char* d = smem + buf * STAGEB + row0 * ROWB + half * 16;
 #pragma unroll
     for (int i = 0; i < A_U; ++i)
-      if (BM >= ROWS_PER_PASS || row0 < BM) split_store(d + i * ROWS_PER_PASS * ROWB, ra[st][i]);
+      if (BM >= ROWS_PER_PASS || row0 < BM) split_store(d + i * ROWS_PER_PASS * ROWB, ra[st][i], scale);
 #pragma unroll
     for (int i = 0; i < B_U; ++i)
-      if (BN >= ROWS_PER_PASS || row0 < BN) split_store(d + (BM + i * ROWS_PER_PASS) * ROWB, rb[st][i]);
+      if (BN >= ROWS_PER_PASS || row0 < BN) split_store(d + (BM + i * ROWS_PER_PASS) * ROWB, rb[st][i], SPLIT_UP);
   };
 
-  floatx16 acc[WM][WN];
+  floatx16 acc[WM][WN], sum[WM][WN];
 #pragma unroll
   for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -711,12 +722,14 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_split_kernel(const
   for_stages<0, NS>([&](auto ST_) {
     if (decltype(ST_)::value < KT) load_global(ST_, decltype(ST_)::value);
   });
-  store_lds(std::integral_constant<int, 0>{}, 0);
+  store_lds(std::integral_constant<int, 0>{}, 0, 0);
   if (NS < KT) load_global(std::integral_constant<int, 0>{}, NS);
   __syncthreads();
 
-  // as in gemm_kernel: PARK = stage of k-tile kt+1, STEADY: k-tiles kt+1 and kt+1+NS both exist
-  auto k_tile = [&](int kt, auto PARK_, auto STEADY_) {
+  // k-tile kt, the S-th of its sum; as in gemm_kernel: PARK = stage of k-tile kt+1, STEADY: k-tiles kt+1 and kt+1+NS both exist
+  auto k_tile = [&](int kt, auto S_, auto STEADY_) {
+    constexpr int s = decltype(S_)::value;
+    constexpr std::integral_constant<int, (s + 1) % NS> PARK_{};
     constexpr bool steady = decltype(STEADY_)::value;
     const int buf = kt & 1;
     const unsigned char* as = smem + buf * STAGEB + (wm * WM * 32 + fr) * ROWB + fg * 16;
@@ -729,7 +742,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_split_kernel(const
 #pragma unroll
       for (int j = 0; j < WN; ++j) fb[j][p] = *reinterpret_cast<const bf16x8*>(bs + j * 32 * ROWB + p * PLANE);
     }
-    if (steady || kt + 1 < KT) store_lds(PARK_, buf ^ 1);
+    if (steady || kt + 1 < KT) store_lds(PARK_, buf ^ 1, kt + 1);
     if (steady || kt + 1 + NS < KT) load_global(PARK_, kt + 1 + NS);
     // the small products first
     constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
@@ -739,20 +752,29 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_split_kernel(const
       for (int i = 0; i < WM; ++i)
 #pragma unroll
         for (int j = 0; j < WN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][pa[t]], fb[j][pb[t]], acc[i][j], 0, 0, 0);
+          sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][pa[t]], fb[j][pb[t]], s == 0 && t == 0 ? floatx16{} : sum[i][j], 0, 0, 0);
     __syncthreads();
   };
+  auto add_sum = [&](int kt) {
+    const float scale = turned(kt) ? -SPLIT_DOWN : SPLIT_DOWN;
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][j][v] = fmaf(scale, sum[i][j][v], acc[i][j][v]);
+  };
   int kt = 0;
-  for (; kt + 2 * NS < KT; kt += NS)
-    for_stages<0, NS>([&](auto S_) {
-      constexpr int s = decltype(S_)::value;
-      k_tile(kt + s, std::integral_constant<int, (s + 1) % NS>{}, std::true_type{});
+  for (; kt + CH + NS < KT; kt += CH) {
+    for_stages<0, CH>([&](auto S_) { k_tile(kt + decltype(S_)::value, S_, std::true_type{}); });
+    add_sum(kt);
+  }
+  for (; kt < KT; kt += CH) {
+    for_stages<0, CH>([&](auto S_) {
+      if (kt + decltype(S_)::value < KT) k_tile(kt + decltype(S_)::value, S_, std::false_type{});
     });
-  for (; kt < KT; kt += NS)
-    for_stages<0, NS>([&](auto S_) {
-      constexpr int s = decltype(S_)::value;
-      if (kt + s < KT) k_tile(kt + s, std::integral_constant<int, (s + 1) % NS>{}, std::false_type{});
-    });
+    add_sum(kt);
+  }
 
   bool bad = false;
 #pragma unroll
@@ -1205,16 +1227,16 @@ int dispatch_tile(const gemm_args& a, hipStream_t s) {
   } else {
     if (a.M <= 32) return launch<T, EPI, 1, 4, 1, 1, BK, 2>(a, s);  // 32 x 128: the weights stream once
     // The largest tile that fills most of the chip, two workgroups per CU.  us with 128 x 128 / 64 x 128 / 64 x 64 tiles:
-    // N = 28672, K = 4096 64 rows 202 / 155 / 180, 100 rows 218 / 240 / 287; N = 3584, K = 512 60 rows 35 / 25 / 20, 127 rows
-    // 35 / 25 / 20, 300 36 / 26 / 25, 500 36 / 27 / 26, 1000 39 / 37 / 38; N = 512, K = 2560 in four ranges 127 rows 42 / 31 / 26, 500
-    // 43 / 33 / 29, 2000 51 / 53 / 55; N = 4096, K = 20480 64 rows in eight ranges 136 / 105 / 125, 100 in four 223 / 186 / 217.
-    // (33 .. 64 rows took 171, 27 and 116 of these on v_mfma_f32_32x32x2_f32.)  The statistics of XENT are per 128 columns.
-    // Tiles of 64 rows take a sixth longer for a row (199 rows 417 against 349) and win where they leave out more than that:
-    // 64 rows above, 150.
+    // N = 28672, K = 4096 64 rows 215 / 149 / 174, 100 rows 221 / 215 / 309; N = 3584, K = 512 60 rows 38 / 25 / 22, 127 rows
+    // 38 / 25 / 22, 300 38 / 25 / 26, 500 38 / 26 / 27, 1000 40 / 36 / 45; N = 512, K = 2560 127 rows 45 / 31 / 27, 500
+    // 47 / 32 / 29, 2000 53 / 49 / 60; N = 4096, K = 20480 64 rows in eight ranges 155 / 100 / 122, 100 145 / 162 / 215.
+    // (33 .. 64 rows took 157, 25 and 111 of these on v_mfma_f32_32x32x2_f32.)  The statistics of XENT are per 128 columns.
+    // Tiles of 64 rows take a sixth longer for a row (199 rows 409 against 349) and win where they leave out more than that:
+    // 64 rows above, 129 (321 against 288).
     const int64_t rows64 = (a.M + 63) / 64, rows128 = (a.M + 127) / 128, cols128 = (a.N + 127) / 128;
     if (rows128 * cols128 * a.splits >= 200 && 6 * 2 * rows128 <= 7 * rows64) return launch_split<EPI, 2, 2, 2, 2, 3>(a, s);
-    if constexpr (EPI == MTJ_EPI_XENT) return launch_split<EPI, 2, 2, 1, 2, 4>(a, s);
-    else return rows64 * cols128 * a.splits >= 200 ? launch_split<EPI, 2, 2, 1, 2, 4>(a, s) : launch_split<EPI, 2, 2, 1, 1, 3>(a, s);
+    if constexpr (EPI == MTJ_EPI_XENT) return launch_split<EPI, 2, 2, 1, 2, 2>(a, s);
+    else return rows64 * cols128 * a.splits >= 200 ? launch_split<EPI, 2, 2, 1, 2, 2>(a, s) : launch_split<EPI, 2, 2, 1, 1, 3>(a, s);
   }
   if constexpr (sizeof(T) == 2) {
     // e.g. M = 16384, N = 28672 or N = 4096 (a whole 6B layer at 8 x 2048 tokens): 7168 / 1024 tiles
@@ -1507,8 +1529,8 @@ cut_t pick_cut(int64_t M, int64_t N, int64_t K, int dtype) {
     }
   }
   // 128 x 128 tiles, two workgroups per CU: up to 4 ranges, for float32, whose k-tiles take longer than the partials they cost, up
-  // to 16 (N = 4096, K = 20480, 4 / 8 / 16 at most: 65 rows 214 / 165 / 150 us, 128 rows 198 / 163 / 152, 199 274 / 253 / 250; N =
-  // 1024, K = 5120, 100 rows 44 / 27 / 27)
+  // to 16 (N = 4096, K = 20480, 4 / 8 / 16 at most: 65 rows 184 / 147 / 132 us, 128 rows 197 / 166 / 150, 199 296 / 247 / 252; N =
+  // 1024, K = 5120, 100 rows 46 / 29 / 29)
   const int most = dtype == MTJ_F32 ? 16 : 4;
   const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
   while (splits < most && tiles * splits * 2 <= 512 && kt % (splits * 2) == 0 && kt / (splits * 2) >= 16) splits *= 2;

@@ -190,6 +190,36 @@ def test_float32_products_on_the_bf16_matrix_cores(L, M, N, K):
     assert bool((out[:, N:] == 7.0).all())
 
 
+@pytest.mark.parametrize("kind", ["normal", "gelu", "positive"])
+@pytest.mark.parametrize("M,N,K", [(300, 1024, 512), (100, 512, 2560), (64, 28672, 1024), (150, 4096, 4096), (256, 4096, 20480)])
+def test_float32_products_are_as_exact_as_float32_and_lean_to_no_side(L, kind, M, N, K):
+    """Every tile, against float64.  A total takes one float32 addition per 64 to 96 elements of K, each a rounding of 2^-24 of a
+    running sum of random signs or a growing one: 2^-24 sqrt(K / 64) of the root mean square, twice for what happens inside the
+    sums.  Roundings to nearest lean to no side: the mean error is below a quarter of one (2^-26 of the root mean
+    square; the mean of M N such errors strays by less than a tenth of that)."""
+    a = abi()
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    A, W = torch.randn(M, K, generator=g, device=DEV), 0.02 * torch.randn(N, K, generator=g, device=DEV)
+    if kind == "gelu":
+        A = torch.nn.functional.gelu(2 * A)
+    if kind == "positive":
+        A, W = A.abs(), W.abs()
+    ref = A.double() @ W.double().t()
+    rms = float(ref.pow(2).mean().sqrt())
+    out = torch.empty(M, N, device=DEV)
+    nb = L.mtj_gemm_splitk_work_bytes(M, N, K, 0)
+    work = torch.empty(max(nb, 16), dtype=torch.uint8, device=DEV)
+    for ranges in (False, True):
+        if ranges:
+            a.check(L.mtj_gemm_splitk(a.ptr(A), K, a.ptr(W), None, M, N, K, 0, a.EPI_STORE, a.ptr(out), N, 0, a.ptr(work), nb, 1.0, S()))
+        else:
+            a.check(L.mtj_gemm(a.ptr(A), K, a.ptr(W), None, M, N, K, 0, a.EPI_STORE, a.ptr(out), N, 0, None, 1.0, S()))
+        torch.cuda.synchronize()
+        err = out.double() - ref
+        assert float(err.pow(2).mean().sqrt()) / rms < 2.0 ** -23 * math.sqrt(K / 64), (kind, ranges)
+        assert abs(float(err.mean())) / rms < 2.0 ** -26, (kind, ranges)
+
+
 @pytest.mark.parametrize("N", [140, 12801])
 def test_float32_products_of_numbers_that_are_not_finite(L, N):
     """Infinities, NaN and the largest numbers give what plain float32 gives, in their rows and columns only."""
