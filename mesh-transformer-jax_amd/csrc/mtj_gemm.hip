@@ -603,7 +603,9 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_kernel(const gemm_
 //   gelu(2 x normal)   K = 4096  1.1e-6 / -3e-10 and 1.9e-7 / -1e-9      20480  2.6e-6 / -8e-10 and 3.0e-7 / -8e-10
 //   positive operands  K = 4096  9.3e-7 / -7e-9  and 9.9e-8 / -2e-10     20480  1.9e-6 / -2e-7 and 2.0e-7 / -2e-10
 // An operand that is infinite, NaN or rounds to infinity gives NaN here, and a product next to the largest number may give
-// infinity; what is not finite is computed again in plain float32.
+// infinity; what is not finite is computed again with v_mfma_f32_32x32x2_f32, straight from memory,
+// in the tiles of 32 x 32 that hold it (one infinite operand in 200 rows of N = 28672, K = 4096: 734 us instead of 377, 1386 with a
+// serial walk per element).
 //
 // Bound by the vector unit, the barriers and the matrix cores in about equal parts: six v_mfma_f32_32x32x16_bf16 instead of
 // eight v_mfma_f32_32x32x2_f32 of twice the length, 12 vector instructions to split two elements, one per accumulator and sum.
@@ -612,11 +614,6 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_kernel(const gemm_
 // 900; N = 3584, K = 512, 127 / 1500 rows 48 / 77 -> 22 / 54.  The sums cost 4 - 6 % of these (a single accumulator: 600 rows 804).
 // A k-tile of 16 goes global -> registers (NS k-tiles in flight) -> three bf16 planes per row in LDS, double-buffered: rows
 // of 3 x 32 bytes, padded to 112 so that the 16-byte fragment reads of 16 consecutive rows hit distinct banks.
-__device__ __attribute__((noinline)) float plain_dot(const float* __restrict__ x, const float* __restrict__ w, int n) {
-  float s = 0.f;
-  for (int k = 0; k < n && s == s; ++k) s = fmaf(x[k], w[k], s);      // a NaN stays one
-  return s;
-}
 __device__ __forceinline__ bool not_finite(float x) { return !(fabsf(x) < INFINITY); }
 constexpr float SPLIT_UP = 1.f, SPLIT_DOWN = 1.f;
 
@@ -776,24 +773,27 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64, WM * WN > 2 ? 2 : 3) void ge
     add_sum(kt);
   }
 
-  bool bad = false;
+  for_tiles<0, 0, WM, WN>([&](auto I_, auto J_) {
+    constexpr int i = decltype(I_)::value, j = decltype(J_)::value;
+    bool again = false;
 #pragma unroll
-  for (int i = 0; i < WM; ++i)
+    for (int v = 0; v < 16; ++v) again |= not_finite(acc[i][j][v]);
+    if (!__any(again)) return;
+    floatx16 plain = {};
+    const int off_a = (int)((((int64_t)(wm * WM + i) * 32 + fr) * a.lda + fg * 8) * 4);
+    const int off_b = (int)((((int64_t)(wn * WN + j) * 32 + fr) * a.K + fg * 8) * 4);
+    for (int k = kt0; k < kt0 + KT; ++k) {
+      mma<float>::frag fa, fb;
+      fa.lo = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(ra_rsrc, off_a, k * BK * 4, 0));
+      fa.hi = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(ra_rsrc, off_a + 16, k * BK * 4, 0));
+      fb.lo = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rb_rsrc, off_b, k * BK * 4, 0));
+      fb.hi = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rb_rsrc, off_b + 16, k * BK * 4, 0));
+      mma<float>::run(plain, fa, fb);
+    }
 #pragma unroll
-    for (int j = 0; j < WN; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) bad |= not_finite(acc[i][j][v]);
-  if (__any(bad))
-    for_tiles<0, 0, WM, WN>([&](auto I_, auto J_) {
-      constexpr int i = decltype(I_)::value, j = decltype(J_)::value;
-      const int c = (wn * WN + j) * 32 + fr;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int r = (wm * WM + i) * 32 + 8 * (v / 4) + 4 * fg + (v % 4);
-        if (not_finite(acc[i][j][v]) && r < rows_a && c < rows_b)
-          acc[i][j][v] = plain_dot(tile_a + (int64_t)r * a.lda + kt0 * BK, tile_b + (int64_t)c * a.K + kt0 * BK, KT * BK);
-      }
-    });
+    for (int v = 0; v < 16; ++v)
+      if (not_finite(acc[i][j][v])) acc[i][j][v] = plain[v];
+  });
   void* out = a.splits > 1 ? (void*)(reinterpret_cast<float*>(a.out) + blockIdx.y * a.split_stride) : a.out;
   epilogue<EPI, WAVES_M, WAVES_N, WM, WN>(a, out, acc, smem, m0, n0);
 }

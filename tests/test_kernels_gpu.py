@@ -248,6 +248,36 @@ def test_float32_products_of_numbers_that_are_not_finite(L, N):
     assert float(out[20, 20]) == big and float(out[21, 21]) == float(torch.tensor(1.8446743e19) * torch.tensor(1.8446743e19))
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 130, 2560), (300, 12900, 1024), (129, 4096, 4096)])
+def test_float32_products_of_long_rows_that_are_not_finite(L, M, N, K):
+    """Infinities and NaN in single places of long rows, in one K range and in several: the rows and columns without them are
+    those of finite operands, bit for bit; the others are what float64 makes of them."""
+    a = abi()
+    g = torch.Generator().manual_seed(M)
+    A = torch.randn(M, K + 4, generator=g).to(DEV)
+    W = torch.randn(N, K, generator=g).to(DEV)
+    nb = L.mtj_gemm_splitk_work_bytes(M, N, K, 0)
+    work = torch.empty(max(nb, 16), dtype=torch.uint8, device=DEV)
+
+    def product(ranges):
+        out = torch.empty(M, N, device=DEV)
+        if ranges:
+            a.check(L.mtj_gemm_splitk(a.ptr(A), K + 4, a.ptr(W), None, M, N, K, 0, a.EPI_STORE, a.ptr(out), N, 0, a.ptr(work), nb, 1.0, S()))
+        else:
+            a.check(L.mtj_gemm(a.ptr(A), K + 4, a.ptr(W), None, M, N, K, 0, a.EPI_STORE, a.ptr(out), N, 0, None, 1.0, S()))
+        torch.cuda.synchronize()
+        return out
+    finite = [product(r) for r in (False, True)]
+    A[3, 5], A[M - 1, K - 1], A[40, 700], W[N - 1, 2] = float("inf"), -float("inf"), float("nan"), float("inf")
+    ref = A[:, :K].double() @ W.double().t()
+    rows, cols = torch.ones(M, dtype=torch.bool), torch.ones(N, dtype=torch.bool)
+    rows[[3, M - 1, 40]], cols[N - 1] = False, False
+    for r in (False, True):
+        out = product(r)
+        assert torch.equal(out[rows][:, cols], finite[r][rows][:, cols])
+        assert torch.equal(out.isnan(), ref.isnan()) and torch.equal(out[ref.isinf()].double(), ref[ref.isinf()])
+
+
 def test_pack_cvt_holds_bf16_weights_exactly_in_float16_and_alpha_undoes_the_scale(L):
     """The matrix-core path of a bfloat16 model: weights go to float16 times a power of two (exact for every weight
     whose scaled magnitude is a normal float16), the GEMM multiplies the accumulator by the inverse."""
