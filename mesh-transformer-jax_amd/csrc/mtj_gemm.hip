@@ -592,7 +592,9 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_kernel(const gemm_
 
 // float32 operands on the bf16 matrix cores.  A float32 number is the sum of three bf16 numbers without an error (rounded to
 // nearest, each takes 8 of the 24 significant bits of what the ones before it leave), so a product is nine products of
-// parts; the six with the largest weights are taken - the other three together are below 2^-24 of the product -.
+// parts; the six with the largest weights are taken - the other three together are below 2^-24 of the product -.  So that the
+// lowest part of the smallest number is a normal bf16 number too, both operands are multiplied by 2^24 first (every float32 number
+// is then a multiple of 2^-125); the sums are taken back by 2^-48.
 // The bf16 matrix instruction drops low bits of what it adds to a large accumulator, and not symmetrically: with one accumulator
 // for all of K the results lay 1e-7 (K = 2560) to 1e-6 (K = 20480) of their root mean square too low, whatever their sign.
 // So a sum is only CH k-tiles long and then added to a float32 total by the vector unit, and every second sum (and K range) is
@@ -602,20 +604,20 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_kernel(const gemm_
 //                      K = 20480 2.6e-6 /  5e-9  and 3.0e-7 / -1e-9      in four ranges 1.3e-6 / -1e-9 and 2.1e-7 / -2e-10
 //   gelu(2 x normal)   K = 4096  1.1e-6 / -3e-10 and 1.9e-7 / -1e-9      20480  2.6e-6 / -8e-10 and 3.0e-7 / -8e-10
 //   positive operands  K = 4096  9.3e-7 / -7e-9  and 9.9e-8 / -2e-10     20480  1.9e-6 / -2e-7 and 2.0e-7 / -2e-10
-// An operand that is infinite, NaN or rounds to infinity gives NaN here, and a product next to the largest number may give
-// infinity; what is not finite is computed again with v_mfma_f32_32x32x2_f32, straight from memory,
+// What is not finite (an operand from 2^103 on or NaN, products or sums from 2^79 on, which the scale takes beyond the largest
+// number) is computed again with v_mfma_f32_32x32x2_f32, straight from memory,
 // in the tiles of 32 x 32 that hold it (one infinite operand in 200 rows of N = 28672, K = 4096: 734 us instead of 377, 1386 with a
 // serial walk per element).
 //
 // Bound by the vector unit, the barriers and the matrix cores in about equal parts: six v_mfma_f32_32x32x16_bf16 instead of
-// eight v_mfma_f32_32x32x2_f32 of twice the length, 12 vector instructions to split two elements, one per accumulator and sum.
+// eight v_mfma_f32_32x32x2_f32 of twice the length, 13 vector instructions to split two elements, one per accumulator and sum.
 // us before and now: N = 28672, K = 4096, 65 / 199 / 600 / 2048 rows 290 / 544 / 1319 / 3516 -> 209 / 346 / 848 / 2420 (1.2 PFLOP/s of bf16
 // products); N = 4096, K = 20480, 65 / 128 / 400 / 1024 rows (4 ranges before, up to 16 now) 362 / 380 / 688 / 1379 -> 132 / 150 / 449 /
 // 900; N = 3584, K = 512, 127 / 1500 rows 48 / 77 -> 22 / 54.  The sums cost 4 - 6 % of these (a single accumulator: 600 rows 804).
 // A k-tile of 16 goes global -> registers (NS k-tiles in flight) -> three bf16 planes per row in LDS, double-buffered: rows
 // of 3 x 32 bytes, padded to 112 so that the 16-byte fragment reads of 16 consecutive rows hit distinct banks.
 __device__ __forceinline__ bool not_finite(float x) { return !(fabsf(x) < INFINITY); }
-constexpr float SPLIT_UP = 1.f, SPLIT_DOWN = 1.f;
+constexpr float SPLIT_UP = 0x1p24f, SPLIT_DOWN = 0x1p-48f;
 
 template <int EPI, int WAVES_M, int WAVES_N, int WM, int WN, int NS>
 __global__ __launch_bounds__(WAVES_M* WAVES_N * 64, WM * WN > 2 ? 2 : 3) void gemm_split_kernel(const gemm_args a) {

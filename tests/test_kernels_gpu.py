@@ -220,6 +220,28 @@ def test_float32_products_are_as_exact_as_float32_and_lean_to_no_side(L, kind, M
         assert abs(float(err.mean())) / rms < 2.0 ** -26, (kind, ranges)
 
 
+@pytest.mark.parametrize("small", ["A", "W"])
+@pytest.mark.parametrize("N", [100, 12900])
+def test_float32_products_of_small_numbers(L, N, small):
+    """Rows of one operand from 2^-60 down to subnormal numbers, times numbers around 2^50: as exact as any other product (the bound of
+    test_float32_products_on_the_bf16_matrix_cores).  Rows around 2^100 on the same side take the way of what overflows."""
+    a = abi()
+    M, K = 130, 64
+    g = torch.Generator().manual_seed(N)
+    A, W = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g)
+    s, other = (A, W) if small == "A" else (W, A)
+    other *= 2.0 ** 50
+    for r in range(s.shape[0]):
+        s[r] *= 2.0 ** (-60, -100, -109, -112, -120, -126, -132, -140, 70)[r % 9]
+    A, W = A.to(DEV), W.to(DEV)
+    out = torch.empty(M, N, device=DEV)
+    a.check(L.mtj_gemm(a.ptr(A), K, a.ptr(W), None, M, N, K, 0, a.EPI_STORE, a.ptr(out), N, 0, None, 1.0, S()))
+    torch.cuda.synchronize()
+    err = (out.double() - A.double() @ W.double().t()).abs()
+    mag = A.double().abs() @ W.double().abs().t()
+    assert bool((err <= (2.0 ** -23 + 2.0 ** -24 * 6 * K / 16) * mag).all())
+
+
 @pytest.mark.parametrize("N", [140, 12801])
 def test_float32_products_of_numbers_that_are_not_finite(L, N):
     """Infinities, NaN and the largest numbers give what plain float32 gives, in their rows and columns only."""
