@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define MTJ_ABI_VERSION 6
+#define MTJ_ABI_VERSION 7
 
 enum { MTJ_F32 = 0, MTJ_BF16 = 1, MTJ_F16 = 2 };
 
@@ -158,8 +158,13 @@ int mtj_gemm(const void* A, int64_t lda, const void* W, const float* bias, int64
  * float32 -, at least 8 of them, up to 128 tiles of 128 columns up to 64 rows; at least 32, up to 256 tiles of
  * 128 x 128 or 16-bit operands with 100 .. 128 tiles of 256 x 256 beyond); elsewhere a call that does not meet it
  * runs in one K range.
+ * The number of ranges falls as M grows, so the need is not monotonic in M: 792 rows may need more than 4792.
+ * With more than 64 rows of float32 the product is cut into up to four times as many ranges where `work` holds
+ * them: mtj_gemm_splitk_best_work_bytes() is what the fastest cut takes (the same number everywhere else).  The order of
+ * summation follows the number of ranges.
  * Call sites: the out/fc_out projection of decode_once (layers.py:316-344) at batch > 1. */
 int64_t mtj_gemm_splitk_work_bytes(int64_t M, int64_t N, int64_t K, int dtype);
+int64_t mtj_gemm_splitk_best_work_bytes(int64_t M, int64_t N, int64_t K, int dtype);
 int mtj_gemm_splitk(const void* A, int64_t lda, const void* W, const float* bias, int64_t M, int64_t N, int64_t K,
                     int dtype, int epi, void* out, int64_t ldo, int out_dtype, void* work, int64_t work_bytes,
                     float alpha, void* stream);

@@ -1479,7 +1479,8 @@ int64_t inproj_front(int64_t M, int64_t N, int64_t K) {
 // the product itself, the rows behind them in `splits` K ranges with a reduce.
 struct cut_t { int64_t front; int splits; };
 
-cut_t pick_cut(int64_t M, int64_t N, int64_t K, int dtype) {
+// `most`: ranges of more than 64 rows of float32 (see the end)
+cut_t pick_cut(int64_t M, int64_t N, int64_t K, int dtype, int most = 4) {
   if (N % 4) return {0, 1};
   const int bk = dtype == MTJ_F32 ? 32 : 64;
   const int64_t kt = K / bk;
@@ -1530,10 +1531,10 @@ cut_t pick_cut(int64_t M, int64_t N, int64_t K, int dtype) {
       return {0, 1};
     }
   }
-  // 128 x 128 tiles, two workgroups per CU: up to 4 ranges, for float32, whose k-tiles take longer than the partials they cost, up
-  // to 16 (N = 4096, K = 20480, 4 / 8 / 16 at most: 65 rows 184 / 147 / 132 us, 128 rows 197 / 166 / 150, 199 296 / 247 / 252; N =
-  // 1024, K = 5120, 100 rows 46 / 29 / 29)
-  const int most = dtype == MTJ_F32 ? 16 : 4;
+  // 128 x 128 tiles, two workgroups per CU: up to 4 ranges.  The k-tiles of float32 take longer than the partials they cost, so up to
+  // 16 where the workspace holds them (N = 4096, K = 20480, 4 / 8 / 16 at most: 65 rows 184 / 147 / 132 us, 128 rows 197 / 166 /
+  // 150, 199 296 / 247 / 252; N = 1024, K = 5120, 100 rows 46 / 29 / 29)
+  if (dtype != MTJ_F32) most = 4;
   const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
   while (splits < most && tiles * splits * 2 <= 512 && kt % (splits * 2) == 0 && kt / (splits * 2) >= 16) splits *= 2;
   return {0, splits};
@@ -1544,6 +1545,15 @@ int64_t cut_bytes(const cut_t& cut, int64_t M, int64_t N) {
 }
 bool work_holds(const cut_t& cut, int64_t M, int64_t N, const void* work, int64_t work_bytes) {
   return work && mtj_aligned16(work) && work_bytes >= cut_bytes(cut, M, N);
+}
+// The most ranges that the workspace holds, and four where it holds less: a call with the workspace that
+// mtj_gemm_splitk_work_bytes asks for, or with that of another row count, is not refused for the sake of a faster cut.
+cut_t cut_for(int64_t M, int64_t N, int64_t K, int dtype, const void* work, int64_t work_bytes) {
+  for (int most : {16, 8}) {
+    const cut_t cut = pick_cut(M, N, K, dtype, most);
+    if (work_holds(cut, M, N, work, work_bytes)) return cut;
+  }
+  return pick_cut(M, N, K, dtype);
 }
 
 // Problems whose tiles of one K range leave more than half of the chip idle: mtj_gemm_splitk asks for an `out` that the
@@ -1629,13 +1639,17 @@ extern "C" int64_t mtj_gemm_splitk_work_bytes(int64_t M, int64_t N, int64_t K, i
   if (M <= 0 || N <= 0 || K <= 0 || !mtj_is_dtype(dtype)) return 0;
   return cut_bytes(pick_cut(M, N, K, dtype), M, N);
 }
+extern "C" int64_t mtj_gemm_splitk_best_work_bytes(int64_t M, int64_t N, int64_t K, int dtype) {
+  if (M <= 0 || N <= 0 || K <= 0 || !mtj_is_dtype(dtype)) return 0;
+  return cut_bytes(pick_cut(M, N, K, dtype, 16), M, N);
+}
 
 extern "C" int mtj_gemm_splitk(const void* A, int64_t lda, const void* W, const float* bias, int64_t M, int64_t N,
                                int64_t K, int dtype, int epi, void* out, int64_t ldo, int out_dtype, void* work,
                                int64_t work_bytes, float alpha, void* stream) {
   MTJ_REQUIRE(epi == MTJ_EPI_STORE || epi == MTJ_EPI_RESID, MTJ_EINVAL, "mtj_gemm_splitk: epilogue %d", epi);
   if (int rc = check_common(A, lda, W, M, N, K, dtype, "mtj_gemm_splitk")) return rc;
-  const cut_t cut = pick_cut(M, N, K, dtype);
+  const cut_t cut = cut_for(M, N, K, dtype, work, work_bytes);
   const int splits = cut.splits;
   // the reduce moves four columns at a time
   const bool rows_ok = out && ldo >= N && ldo % 4 == 0 && mtj_aligned16(out) && (!bias || mtj_aligned16(bias));
@@ -1678,7 +1692,7 @@ extern "C" int mtj_gemm_splitk_ln(const void* A, int64_t lda, const void* W, con
                   (!bias || mtj_aligned16(bias)),
               MTJ_EINVAL, "mtj_gemm_splitk_ln: N a multiple of 4 and <= %d, rows of x and h 16-byte aligned", 4 * RLN_Q * 1024);
   if (int rc = check_common(A, lda, W, M, N, K, dtype, "mtj_gemm_splitk_ln")) return rc;
-  const cut_t cut = pick_cut(M, N, K, dtype);
+  const cut_t cut = cut_for(M, N, K, dtype, work, work_bytes);
   const int splits = cut.splits;
   // mtj_layernorm takes dense rows; pick_cut leaves none to it where needs_ranges holds (N <= 16384)
   const bool need = needs_ranges(M, N, K, dtype);

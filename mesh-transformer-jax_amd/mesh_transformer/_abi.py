@@ -9,7 +9,7 @@ import os
 
 F32, BF16, F16 = 0, 1, 2
 EPI_STORE, EPI_RESID, EPI_INPROJ = 0, 1, 2
-ABI_VERSION = 6
+ABI_VERSION = 7
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libmtj_hip.so")
 
@@ -51,6 +51,7 @@ SIGNATURES = {
     "mtj_xent": (_i32, [_p, _i64, _p, _i64, _i64, _p, _p, _p]),
     "mtj_gemm": (_i32, [_p, _i64, _p, _p, _i64, _i64, _i64, _i32, _i32, _p, _i64, _i32, C.POINTER(InProj), C.c_float, _p]),
     "mtj_gemm_splitk_work_bytes": (_i64, [_i64, _i64, _i64, _i32]),
+    "mtj_gemm_splitk_best_work_bytes": (_i64, [_i64, _i64, _i64, _i32]),
     "mtj_gemm_splitk": (_i32, [_p, _i64, _p, _p, _i64, _i64, _i64, _i32, _i32, _p, _i64, _i32, _p, _i64, C.c_float, _p]),
     "mtj_gemm_splitk_ln": (_i32, [_p, _i64, _p, _p, _i64, _i64, _i64, _i32, _p, _i64, _p, _i64, _p, _p, _p, _i64, _i32,
                                  C.c_float, _p]),

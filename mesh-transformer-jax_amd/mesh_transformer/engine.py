@@ -37,13 +37,14 @@ def _f32(t):
     return t.to(torch.float32).contiguous()
 
 
-def splitk_work_bound(M_max, N, K, dtype):
-    """Bytes of split-K workspace that cover every row count 1 .. M_max of an [M, K] x [K, N] product.  The cut
-    into K ranges changes with M, so the need is not monotonic in M; between multiples of 128 rows (and below 64 rows) the
-    cut is the same and the need grows with M, so those row counts are the candidates."""
+def splitk_work_bound(M_max, N, K, dtype, best=False):
+    """Bytes of split-K workspace that cover every row count 1 .. M_max of an [M, K] x [K, N] product (`best`: with the
+    fastest cut of each).  The cut into K ranges changes with M, so the need is not monotonic in M; between multiples of 128
+    rows (and below 64 rows) the cut is the same and the need grows with M, so those row counts are the candidates."""
     L = _abi.lib()
+    query = L.mtj_gemm_splitk_best_work_bytes if best else L.mtj_gemm_splitk_work_bytes
     cand = set(range(1, min(M_max, 64) + 1)) | set(range(128, M_max + 1, 128)) | {M_max}
-    return max(L.mtj_gemm_splitk_work_bytes(m, N, K, dtype) for m in cand)
+    return max(query(m, N, K, dtype) for m in cand)
 
 
 class PackedWeights:
@@ -196,8 +197,8 @@ class Session:
         self.logits = torch.empty(B, V, dtype=torch.float32, device=dev)
         # split-K workspace of the out projection: batched decode (B rows) and every prefill this session can see
         # (1 .. B * Tp_max rows; a shorter prompt is cut into MORE K ranges, so the longest one is not the bound)
-        nb = 0 if self.gemv_path else L.mtj_gemm_splitk_work_bytes(B, d, d + F, w.mm_dtype)
-        nb = max(nb, splitk_work_bound(M, d, d + F, w.mm_dtype))
+        nb = 0 if self.gemv_path else L.mtj_gemm_splitk_best_work_bytes(B, d, d + F, w.mm_dtype)
+        nb = max(nb, splitk_work_bound(M, d, d + F, w.mm_dtype, best=True))
         self.gemm_work = torch.empty(max(nb, 256), dtype=torch.uint8, device=dev)
         # batched decode attends in one launch where that covers the shape (its counters are zeroed here, once)
         nb = 0 if self.gemv_path else L.mtj_attn_decode_joined_work_bytes(B, H, dh, Tcap)

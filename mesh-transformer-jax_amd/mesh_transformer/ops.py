@@ -117,7 +117,7 @@ def _gemm_resid_(x, A, W, bias, alpha):
     M, K = A.shape
     N = W.shape[0]
     L = _abi.lib()
-    nb = L.mtj_gemm_splitk_work_bytes(M, N, K, _code(W))
+    nb = L.mtj_gemm_splitk_best_work_bytes(M, N, K, _code(W))
     work = torch.empty(max(nb, 16), dtype=torch.uint8, device=A.device)
     check(L.mtj_gemm_splitk(ptr(A), A.stride(0), ptr(W), ptr(bias), M, N, K, _code(W), EPI_RESID, ptr(x), x.stride(0), F32,
                             ptr(work), work.numel(), alpha, _s()))

@@ -119,6 +119,31 @@ def test_session_workspace_covers_every_prompt_length():
     assert lib.mtj_gemm_splitk_work_bytes(8 * 99, 4096, 20480, _abi.F16) > lib.mtj_gemm_splitk_work_bytes(8 * 599, 4096, 20480, _abi.F16)
 
 
+def test_splitk_takes_the_workspace_of_more_rows():
+    """float32: the faster cuts are taken where the workspace holds them, and nothing is refused for want of them - neither the
+    workspace that the query asks for nor that of 199 rows with fewer rows; a session holds the fastest cut of every prompt."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("the pointers of this test must never reach a GPU")
+    from mesh_transformer import _abi
+    from mesh_transformer.engine import splitk_work_bound
+    lib, P, N, K = _abi.lib(), 1 << 20, 4096, 20480
+    need = lambda m: lib.mtj_gemm_splitk_work_bytes(m, N, K, 0)
+    best = lambda m: lib.mtj_gemm_splitk_best_work_bytes(m, N, K, 0)
+    for m in (65, 100, 128, 150, 199, 256, 300, 511, 700):
+        assert need(m) == (4 if m <= 512 else 2) * m * N * 4 and best(m) in (need(m), 2 * need(m), 4 * need(m)), m
+        for have in (need(m), max(need(m), need(199)), best(m) - 4, best(m)):
+            for rc in (lib.mtj_gemm_splitk(P, K, P, P, m, N, K, 0, _abi.EPI_RESID, P, N, 0, P, have, 1.0, None),
+                       lib.mtj_gemm_splitk_ln(P, K, P, P, m, N, K, 0, P, N, P, have, P, P, P, N, 0, 1.0, None)):
+                assert rc == -4 if have >= need(m) else rc == -1, (m, have, rc)
+    assert best(128) == 16 * 128 * N * 4 and need(199) >= need(128)
+    for M_max in (100, 700, 2047):
+        assert splitk_work_bound(M_max, N, K, 0, best=True) == max(best(m) for m in range(1, M_max + 1))
+    for dtype in (1, 2):
+        for M, n, k in _splitk_sizes():
+            assert lib.mtj_gemm_splitk_best_work_bytes(M, n, k, dtype) == lib.mtj_gemm_splitk_work_bytes(M, n, k, dtype)
+
+
 def _needs_ranges(lib, M, N, K, dtype):
     """The products that mtj_gemm_splitk has always cut into K ranges, and for which it asks for rows that its reduce can
     take: ranges are doubled while they are no more than the CUs (128-column tiles, 256 x 256 tiles) or two per CU

@@ -490,6 +490,32 @@ def test_reduce_with_layernorm_at_every_row_length(L, N):
     assert rel_err(h[:M], want) < 1e-5 and bool((h[M] == 7.0).all())
 
 
+@pytest.mark.parametrize("M,N,K,best", [(65, 4096, 20480, 16), (100, 4096, 20480, 16), (128, 512, 20480, 16), (199, 4096, 20480, 8),
+                                        (100, 1024, 5120, 8), (700, 1024, 20480, 8), (300, 132, 20480, 16)])
+def test_float32_ranges_as_many_as_the_workspace_holds(L, M, N, K, best):
+    """4, 8 and 16 ranges of more than 64 rows, through the plain reduce and the one that normalises, in the workspace asked for, in
+    that of a larger row count and in the best one.  Bounds of the other float32 products."""
+    a = abi()
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    A = torch.randn(M, K, generator=g, device=DEV)
+    W = 0.05 * torch.randn(N, K, generator=g, device=DEV)
+    bias, sc, of = torch.randn(N, generator=g, device=DEV), 1 + 0.1 * torch.randn(N, generator=g, device=DEV), 0.1 * torch.randn(N, generator=g, device=DEV)
+    x0 = torch.randn(M, N, generator=g, device=DEV)
+    ref = x0.double() + A.double() @ W.double().t() + bias.double()
+    need, most = L.mtj_gemm_splitk_work_bytes(M, N, K, a.F32), L.mtj_gemm_splitk_best_work_bytes(M, N, K, a.F32)
+    assert need == 4 * M * N * 4 and most == best * M * N * 4
+    for have in (need, 2 * need - 4, 2 * need, most):
+        work = torch.full((have + 64,), 7, dtype=torch.uint8, device=DEV)
+        x, y, h = x0.clone(), x0.clone(), torch.zeros(M, N, device=DEV)
+        a.check(L.mtj_gemm_splitk(a.ptr(A), K, a.ptr(W), a.ptr(bias), M, N, K, a.F32, a.EPI_RESID, a.ptr(x), N, 0, a.ptr(work), have, 1.0, S()))
+        a.check(L.mtj_gemm_splitk_ln(a.ptr(A), K, a.ptr(W), a.ptr(bias), M, N, K, a.F32, a.ptr(y), N, a.ptr(work), have,
+                                     a.ptr(sc), a.ptr(of), a.ptr(h), N, a.F32, 1.0, S()))
+        torch.cuda.synchronize()
+        assert rel_err(x, ref) < 2e-6 and torch.equal(x, y), have
+        assert rel_err(h, torch.nn.functional.layer_norm(ref, (N,), sc.double(), of.double(), 1e-5)) < 1e-5
+        assert bool((work[have:] == 7).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(1808, 4096, 2432), (3195, 2048, 2560), (100, 512, 2560), (768, 1024, 5120)])
 def test_splitk_layernorm_on_padded_rows(L, M, N, K):
     """x and h with padded rows, at a short K (128 and 104 tiles of 256 x 256 in two ranges) and at few rows: the padding
