@@ -207,8 +207,14 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const float* __restrict_
 
 template <int OUT_DTYPE>
 void launch_layernorm(const float* x, const float* scale, const float* offset, int64_t M, int d, void* out, hipStream_t s) {
-  if (d <= 1024) layernorm_kernel<OUT_DTYPE, false><<<(unsigned)((M + 3) / 4), 256, 0, s>>>(x, scale, offset, M, d, out);
-  else layernorm_kernel<OUT_DTYPE, true><<<(unsigned)M, 256, 0, s>>>(x, scale, offset, M, d, out);
+  // a launch has less than 2^32 threads
+  constexpr int64_t MOST = 1 << 23;
+  const int esz = OUT_DTYPE == MTJ_F32 ? 4 : 2;
+  for (int64_t m = 0; m < M; m += MOST, x += MOST * d, out = (char*)out + MOST * d * esz) {
+    const int64_t rows = M - m < MOST ? M - m : MOST;
+    if (d <= 1024) layernorm_kernel<OUT_DTYPE, false><<<(unsigned)((rows + 3) / 4), 256, 0, s>>>(x, scale, offset, rows, d, out);
+    else layernorm_kernel<OUT_DTYPE, true><<<(unsigned)rows, 256, 0, s>>>(x, scale, offset, rows, d, out);
+  }
 }
 
 extern "C" int mtj_layernorm(const float* x, const float* scale, const float* offset, int64_t M, int64_t d,

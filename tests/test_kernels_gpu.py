@@ -119,6 +119,28 @@ def test_layernorm_rows_of_a_wavefront_and_of_a_workgroup(L, d, M):
     assert torch.equal(x, out[:M]) and bool((out[M] == 7.0).all())
 
 
+def test_layernorm_of_more_rows_than_a_launch_has_threads_for(L):
+    """2^24 + 3 rows of 1028 columns are 2^32 threads and more; rows on both sides of a launch and the last ones."""
+    M, d = (1 << 24) + 3, 1028
+    if torch.cuda.mem_get_info()[0] < 130 << 30:
+        pytest.skip("needs 104 GB")
+    a = abi()
+    x = torch.zeros(M, d, device=DEV)
+    out = torch.empty(M + 1, d, dtype=torch.float16, device=DEV)
+    out[-9:] = 7.0
+    g = torch.Generator(device=DEV).manual_seed(1)
+    sc, of = torch.randn(d, generator=g, device=DEV), torch.randn(d, generator=g, device=DEV)
+    rows = [0, 1, (1 << 22) - 1, 1 << 22, (1 << 23) - 1, 1 << 23, (1 << 24) - 1, 1 << 24, M - 1]
+    x[rows] = torch.randn(len(rows), d, generator=g, device=DEV)
+    a.check(L.mtj_layernorm(a.ptr(x), a.ptr(sc), a.ptr(of), M, d, a.ptr(out), a.F16, S()))
+    torch.cuda.synchronize()
+    want = torch.nn.functional.layer_norm(x[rows].double(), (d,), sc.double(), of.double(), 1e-5)
+    assert rel_err(out[rows], want) < 5e-4
+    assert torch.equal(out[M - 2], of.half()) and torch.equal(out[12345678], of.half()) and bool((out[M] == 7.0).all())
+    del x, out
+    torch.cuda.empty_cache()
+
+
 def test_layernorm_rejects_bad_shapes(L):
     a = abi()
     x = torch.zeros(2, 6, device=DEV)
