@@ -43,7 +43,7 @@ def _run(logits, top_p, temp, top_k, u, want_filtered, want_mask):
         if top_k is not None:
             i32[0, :R] = np.broadcast_to(np.asarray(top_k, np.int32), (R,))
         f64 = torch.from_numpy(f64).to(dev)
-        i32 = f64[3:].view(torch.int32)
+        i32 = f64.view(-1).view(torch.int32)[6 * R:].view(2, 2 * R)       # (also of no rows, which the kernel refuses)
         tp, tm, uu, (pos, pos_start) = f64[0], f64[1], f64[2], (i32[0, R:], i32[1, :R])
         tk = None if top_k is None else i32[0, :R]
         tok = torch.empty(R, dtype=torch.int32, device=dev)

@@ -1464,6 +1464,22 @@ def _sample(L, logits, top_p, temp, top_k, u):
     return tok.cpu().numpy(), mask.cpu().numpy().astype(bool), filt.cpu().numpy()
 
 
+@pytest.mark.parametrize("as_numpy", [False, True])
+def test_samplers_refuse_logits_without_rows(L, as_numpy):
+    """No rows: the kernel's own refusal (a ValueError), whatever the options; one row of the same call draws."""
+    from mesh_transformer import sampling
+    for rows in (0, 1):
+        lg = torch.zeros(rows, 8, device=DEV)
+        lg = lg.cpu().numpy() if as_numpy else lg
+        for opts in ({}, {"top_k": 3}):
+            call = lambda: sampling.nucleaus_sample(np.zeros(rows), lg, None, **opts)[0]
+            if rows:
+                assert int(call()[0]) in range(8)
+            else:
+                with pytest.raises(ValueError):
+                    call()
+
+
 def test_nucleus_reference_demo_vector(L):
     demo = np.array([[-2, -1, 0, 0.8, 0, 0.1, 0.3, 0.4, 0.5, 0.6, 0.7, -3]], np.float32)   # sampling.py:49
     tok, mask, filt = _sample(L, demo, 0.9, 1.0, None, 0.5)
