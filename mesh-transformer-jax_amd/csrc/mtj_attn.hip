@@ -615,6 +615,7 @@ template <> struct psum<bf16_t> {
   }
 };
 
+// f(integral_constant<int, K>) for K = 0 .. N-1, in order
 template <int N, int K = 0, class F> __device__ __forceinline__ void static_for(F&& f) {
   if constexpr (K < N) {
     f(std::integral_constant<int, K>{});
@@ -1002,7 +1003,6 @@ template <> __device__ __forceinline__ uint32_t pack_prob<f16_t>(float lo, float
   const f16x2 r = {(f16_t)lo, (f16_t)hi};
   return __builtin_bit_cast(uint32_t, r);
 }
-// f(integral_constant<int, K>) for K = 0 .. N-1, in order
 template <typename T>
 __global__ __launch_bounds__(256) void attn_prefill_q64_kernel(const T* __restrict__ q, const T* __restrict__ kc,
                                                                const T* __restrict__ vt, const int32_t* __restrict__ pos0,

@@ -6,7 +6,8 @@
 //   gemm_dma_kernel  large 16-bit problems: 256x256x64 tiles written straight into LDS by the memory pipeline
 //                    (buffer_load ... lds), rows xor-swizzled instead of padded, no staging registers;
 //   gemm_stream_kernel  16-bit problems of few rows: the same operand path, all rows in one tile, three or four stages;
-//   gemm_split_kernel  float32 problems of more than 32 rows: every operand as a sum of three bf16 numbers.
+//   gemm_split_kernel  float32 problems of more than 32 rows: every operand as a sum of three bf16 numbers, float32 totals of
+//                    short sums (more exact than v_mfma_f32_32x32x2_f32 over the same K).
 #include "mtj_common.h"
 #include <type_traits>
 
