@@ -36,16 +36,16 @@ def _run(logits, top_p, temp, top_k, u, want_filtered, want_mask):
     with torch.cuda.device(dev):
         # the rows' parameters and their counters at zero travel together: an upload is 10 - 15 us of the host's time, a fill
         # another 5 (8 rows of 50400 logits: 154 -> 121 us)
-        f64 = np.zeros((5, R))
-        for at, v in zip(f64, (top_p, temp, u)):
-            at[:] = np.broadcast_to(np.asarray(v, np.float64), (R,))
-        i32 = f64[3:].view(np.int32)
+        # (one element more, since torch has no view of another type of nothing: no rows are for the kernel to refuse)
+        f64 = np.zeros(5 * R + 1)
+        for i, v in enumerate((top_p, temp, u)):
+            f64[i * R:(i + 1) * R] = np.broadcast_to(np.asarray(v, np.float64), (R,))
         if top_k is not None:
-            i32[0, :R] = np.broadcast_to(np.asarray(top_k, np.int32), (R,))
+            f64.view(np.int32)[6 * R:7 * R] = np.broadcast_to(np.asarray(top_k, np.int32), (R,))
         f64 = torch.from_numpy(f64).to(dev)
-        i32 = f64.view(-1).view(torch.int32)[6 * R:].view(2, 2 * R)       # (also of no rows, which the kernel refuses)
-        tp, tm, uu, (pos, pos_start) = f64[0], f64[1], f64[2], (i32[0, R:], i32[1, :R])
-        tk = None if top_k is None else i32[0, :R]
+        i32 = f64.view(torch.int32)
+        tp, tm, uu, pos, pos_start = f64[:R], f64[R:2 * R], f64[2 * R:3 * R], i32[7 * R:8 * R], i32[8 * R:9 * R]
+        tk = None if top_k is None else i32[6 * R:7 * R]
         tok = torch.empty(R, dtype=torch.int32, device=dev)
         filtered = torch.empty(R, V, dtype=torch.float32, device=dev) if want_filtered else None
         mask = torch.empty(R, V, dtype=torch.uint8, device=dev) if want_mask else None
