@@ -13,7 +13,9 @@
  *   - return value: 0 on success, a negative MTJ_E* code otherwise; mtj_last_error() returns the
  *     message of the calling thread's last failure;
  *   - activations are float32 unless `dtype` says otherwise; `dtype` selects the storage type of
- *     weights / K,V cache / GEMM inputs: MTJ_F32 (exact path), MTJ_BF16 or MTJ_F16.  The reference multiplies
+ *     weights / K,V cache / GEMM inputs: MTJ_F32 (float32 throughout; mtj_gemm and its kin multiply up to 32 rows on the
+ *     float32 matrix instruction and more rows as exact sums of three bf16 numbers with float32 totals, closer to float64
+ *     than that instruction for every finite operand), MTJ_BF16 or MTJ_F16.  The reference multiplies
  *     float32 activations with bf16 weights (jnp.dot(f32, bf16)); the matrix cores want both operands in one
  *     16-bit type, and float16 holds every bf16 weight exactly (after a power-of-two scale, see
  *     mtj_pack_weight_cvt) while rounding an activation to 11 significant bits instead of bf16's 8, so the
